@@ -13,13 +13,13 @@
 // never expanded (the reference callers repeat_interleave them first,
 // tasft/modules/tasft_attention.py:725-729).
 //
-// Mapping onto CDNA4. A workgroup owns one (batch, query head, query block) and has
-// BS/32 waves; wave w owns 32 query rows. Each key block is computed as
+// Mapping onto CDNA4. A wave owns 32 query rows (block 32: the workgroup is one such wave;
+// blocks 64 and 128: two or four waves per 64 rows). Each key tile is computed as
 // S^T = K . Q^T with v_mfma_f32_32x32x16_bf16 (_f16 for fp16 inputs), so a lane owns one query column of S^T:
 // its running max and sum live in that lane (plus the lane 32 away), and the P^T
 // accumulator registers feed the PV product O^T = V^T . P^T directly as the B operand
-// with no shuffle. K (row major) and V^T (transposed while staging) go through LDS
-// rows padded so the MFMA operand reads are bank-conflict free on the 64-bank LDS.
+// with no shuffle. K and V tiles reach LDS by DMA, row major under an XOR swizzle; V^T
+// operands are read transposed from there.
 #include <algorithm>
 #include <type_traits>
 
@@ -42,6 +42,7 @@ struct PrefillParams {
   float scale_log2;  // softmax scale * log2(e)
   int causal;
   int small_spans;   // S * row bytes of K and V below 2^31: 32-bit DMA address math
+  int small_q;       // the same of Q (block 32)
   int* queue;        // per-partition ticket counters of the persistent launch, or null
   int parts;         // work partitions: 8 (one per XCD) or 1
   int wg_per_part;   // persistent workgroups per partition
@@ -116,209 +117,6 @@ __global__ void bsfa_queue_reset_kernel(int* queue) {
   if (threadIdx.x < kQueueSlots) queue[threadIdx.x] = 0;
 }
 
-template <int BS, int D, int DT>
-__global__ void __launch_bounds__(BS / 32 * kWave)
-bsfa_prefill_kernel(const PrefillParams p) {
-  constexpr int WAVES = BS / 32;
-  constexpr int THREADS = WAVES * kWave;
-  constexpr int KSTEPS = D / 16;   // MFMA k-steps over the head dim
-  constexpr int KTILES = BS / 32;  // 32-key tiles per key block
-  constexpr int DTILES = D / 32;   // 32-row head-dim tiles of O^T
-  constexpr int KST = D + 8;       // LDS row stride of K (16-bit elements)
-  constexpr int VST = BS + 4;      // LDS row stride of V^T (16-bit elements)
-
-  __shared__ __attribute__((aligned(16))) uint16_t k_lds[BS * KST];
-  __shared__ __attribute__((aligned(16))) uint16_t vt_lds[D * VST];
-
-  const int tid = threadIdx.x;
-  const int lane = tid & 63;
-  const int wave = tid >> 6;
-  const int col = lane & 31;
-  const int half = lane >> 5;
-
-  const PrefillItem item = prefill_item(p, (int64_t)blockIdx.x);
-  const int qb = item.qb, b = item.b, kvh = item.kvh, h = item.h;
-  // Varlen launch: items past the last query block of a shorter sequence have no work.
-  const SeqSpan span = seq_span<BS>(p, b);
-  if (qb >= span.NB) return;
-  const int S = span.S, NB = span.NB;
-
-
-  const uint16_t* qbase = p.q + b * p.sq[0] + span.tok0 * p.sq[2] + h * p.sq[1];
-  const uint16_t* kbase = p.k + b * p.sk[0] + span.tok0 * p.sk[2] + kvh * p.sk[1];
-  const uint16_t* vbase = p.v + b * p.sv[0] + span.tok0 * p.sv[2] + kvh * p.sv[1];
-  uint16_t* obase = p.o + b * p.so[0] + span.tok0 * p.so[2] + h * p.so[1];
-  const uint8_t* mrow = p.mask + b * p.sm[0] + h * p.sm[1] + (int64_t)(qb >> p.mshift) * p.sm[2];
-
-  // Q^T as the B operand: lane (col, half) holds query row `qrow`, head dims
-  // ks*16 + half*8 .. +7 for every k-step.
-  const int qrow = qb * BS + wave * 32 + col;
-  const bool qvalid = qrow < S;
-  u32x4_t qf[KSTEPS];
-#pragma unroll
-  for (int ks = 0; ks < KSTEPS; ++ks) {
-    u32x4_t val = {0u, 0u, 0u, 0u};
-    if (qvalid) val = *(const u32x4_t*)(qbase + (int64_t)qrow * p.sq[2] + ks * 16 + half * 8);
-    qf[ks] = val;
-  }
-
-  f32x16_t oacc[DTILES];
-#pragma unroll
-  for (int dt = 0; dt < DTILES; ++dt) oacc[dt] = (f32x16_t){};
-  float m_run = -INFINITY;  // running max (log2 domain), identical in lanes l and l^32
-  float l_run = 0.f;        // this lane's share of the running denominator
-
-  const int kb_end = p.causal ? qb + 1 : NB;
-  for (int chunk = 0; chunk < kb_end; chunk += kWave) {
-    // Every wave reads the same 64 mask bytes, so all waves walk the same key blocks.
-    const int kbl = chunk + lane;
-    const bool act = (kbl < kb_end) && (mrow[(int64_t)(kbl >> p.mshift) * p.sm[3]] != 0);
-    uint64_t bits = __ballot(act);
-    while (bits) {
-      const int kb = chunk + __builtin_ctzll(bits);
-      bits &= bits - 1;
-      const int key0 = kb * BS;
-
-      __syncthreads();  // previous block's LDS reads are complete
-      // Stage K rows (16-byte chunks), zero-filling keys >= S.
-#pragma unroll
-      for (int c = tid; c < BS * D / 8; c += THREADS) {
-        const int r = c / (D / 8);
-        const int cc = c % (D / 8);
-        u32x4_t val = {0u, 0u, 0u, 0u};
-        if (key0 + r < S) val = *(const u32x4_t*)(kbase + (int64_t)(key0 + r) * p.sk[2] + cc * 8);
-        *(u32x4_t*)(k_lds + r * KST + cc * 8) = val;
-      }
-      // Stage V transposed: a unit is 4 keys x 8 head dims, written as 8 rows of V^T.
-#pragma unroll
-      for (int u = tid; u < (BS / 4) * (D / 8); u += THREADS) {
-        const int kq = u % (BS / 4);
-        const int dc = u / (BS / 4);
-        u32x4_t rows[4];
-#pragma unroll
-        for (int j = 0; j < 4; ++j) {
-          const int key = key0 + kq * 4 + j;
-          rows[j] = (u32x4_t){0u, 0u, 0u, 0u};
-          if (key < S) rows[j] = *(const u32x4_t*)(vbase + (int64_t)key * p.sv[2] + dc * 8);
-        }
-#pragma unroll
-        for (int i = 0; i < 8; ++i) {
-          uint32_t e[4];
-#pragma unroll
-          for (int j = 0; j < 4; ++j)
-            e[j] = (i & 1) ? (rows[j][i >> 1] >> 16) : (rows[j][i >> 1] & 0xffffu);
-          const u32x2_t w = {e[0] | (e[1] << 16), e[2] | (e[3] << 16)};
-          *(u32x2_t*)(vt_lds + (dc * 8 + i) * VST + kq * 4) = w;
-        }
-      }
-      __syncthreads();
-
-      // S^T tiles: rows = keys t*32 + ..., cols = this wave's 32 queries.
-      f32x16_t s[KTILES];
-#pragma unroll
-      for (int t = 0; t < KTILES; ++t) {
-        s[t] = (f32x16_t){};
-#pragma unroll
-        for (int ks = 0; ks < KSTEPS; ++ks) {
-          const u32x4_t a = *(const u32x4_t*)(k_lds + (t * 32 + col) * KST + ks * 16 + half * 8);
-          s[t] = mfma16<DT>(a, qf[ks], s[t]);
-        }
-      }
-
-      // Register r of tile t holds key t*32 + 8*(r/4) + 4*half + r%4 for query `qrow`.
-      const bool need_mask = (p.causal && kb == qb) || (key0 + BS > S);
-      float mloc = -INFINITY;
-#pragma unroll
-      for (int t = 0; t < KTILES; ++t) {
-#pragma unroll
-        for (int r = 0; r < 16; ++r) {
-          float x = s[t][r] * p.scale_log2;
-          if (need_mask) {
-            const int key = key0 + t * 32 + 8 * (r >> 2) + 4 * half + (r & 3);
-            if (key >= S || (p.causal && key > qrow)) x = -INFINITY;
-          }
-          s[t][r] = x;
-          mloc = fmaxf(mloc, x);
-        }
-      }
-      mloc = fmaxf(mloc, xor32(mloc));
-      const float m_new = fmaxf(m_run, mloc);
-      const float m_use = (m_new == -INFINITY) ? 0.f : m_new;
-      const float alpha = __builtin_amdgcn_exp2f(m_run - m_use);
-      float lsum = 0.f;
-#pragma unroll
-      for (int t = 0; t < KTILES; ++t) {
-#pragma unroll
-        for (int r = 0; r < 16; ++r) {
-          const float e = __builtin_amdgcn_exp2f(s[t][r] - m_use);
-          s[t][r] = e;
-          lsum += e;
-        }
-      }
-      l_run = l_run * alpha + lsum;
-      m_run = m_new;
-#pragma unroll
-      for (int dt = 0; dt < DTILES; ++dt) oacc[dt] *= alpha;
-
-      // P^T as the B operand of O^T = V^T P^T: k-step (t, pp) uses registers 8pp..8pp+7
-      // of tile t, i.e. keys t*32 + 16pp + 8*(j/4) + 4*half + j%4 for slot j.
-      u32x4_t pb[KTILES][2];
-#pragma unroll
-      for (int t = 0; t < KTILES; ++t) {
-#pragma unroll
-        for (int pp = 0; pp < 2; ++pp) {
-          const u32x4_t w = {pack16x2<DT>(s[t][8 * pp + 0], s[t][8 * pp + 1]),
-                             pack16x2<DT>(s[t][8 * pp + 2], s[t][8 * pp + 3]),
-                             pack16x2<DT>(s[t][8 * pp + 4], s[t][8 * pp + 5]),
-                             pack16x2<DT>(s[t][8 * pp + 6], s[t][8 * pp + 7])};
-          pb[t][pp] = w;
-        }
-      }
-      // V^T as the A operand with the same key order: two 4-key runs per slot group.
-#pragma unroll
-      for (int dt = 0; dt < DTILES; ++dt) {
-#pragma unroll
-        for (int t = 0; t < KTILES; ++t) {
-#pragma unroll
-          for (int pp = 0; pp < 2; ++pp) {
-            const uint16_t* vp = vt_lds + (dt * 32 + col) * VST + t * 32 + pp * 16 + half * 4;
-            const u32x2_t lo = *(const u32x2_t*)vp;
-            const u32x2_t hi = *(const u32x2_t*)(vp + 8);
-            const u32x4_t a = {lo[0], lo[1], hi[0], hi[1]};
-            oacc[dt] = mfma16<DT>(a, pb[t][pp], oacc[dt]);
-          }
-        }
-      }
-    }
-  }
-
-  // Epilogue: combine the two half-lane denominators, normalise, store in the input type.
-  const float l_tot = l_run + xor32(l_run);
-  const float inv = 1.f / (l_tot > 0.f ? l_tot : 1.f);  // empty rows: O = 0; NaN rows stay NaN
-  if (qvalid) {
-    uint16_t* orow = obase + (int64_t)qrow * p.so[2];
-#pragma unroll
-    for (int dt = 0; dt < DTILES; ++dt) {
-#pragma unroll
-      for (int gq = 0; gq < 4; ++gq) {
-        const int d0 = dt * 32 + 8 * gq + 4 * half;
-        const u32x2_t w = {pack16x2<DT>(oacc[dt][4 * gq + 0] * inv, oacc[dt][4 * gq + 1] * inv),
-                           pack16x2<DT>(oacc[dt][4 * gq + 2] * inv, oacc[dt][4 * gq + 3] * inv)};
-        *(u32x2_t*)(orow + d0) = w;
-      }
-    }
-  }
-}
-
-template <int BS, int D, int DT>
-static hipError_t launch_prefill(const PrefillParams& p, hipStream_t stream) {
-  const int64_t grid = (int64_t)p.NB * p.B * p.Hq;
-  hipLaunchKernelGGL((bsfa_prefill_kernel<BS, D, DT>), dim3((unsigned)grid), dim3(BS / 32 * kWave), 0,
-                     stream, p);
-  return hipGetLastError();
-}
-
-
 // ---------------------------------------------------------------------------------------
 // Block size 64: the tuned kernel.
 //
@@ -387,6 +185,12 @@ __device__ __forceinline__ void dma_tile(uint8_t* tile, __amdgpu_buffer_rsrc_t r
 __device__ __forceinline__ __amdgpu_buffer_rsrc_t tile_rsrc(const void* base, int64_t bytes) {
   const int n = bytes > 0x7fffffff ? 0x7fffffff : (bytes < 0 ? 0 : (int)bytes);
   return __builtin_amdgcn_make_buffer_rsrc((void*)base, (short)0, n, 0x00020000);
+}
+
+// One DMA instruction: 16 bytes per lane from r[voff] to 1 KB of LDS at `dst`.
+template <int AUX>
+__device__ __forceinline__ void dma16_lds(__amdgpu_buffer_rsrc_t r, uint8_t* dst, int voff) {
+  __builtin_amdgcn_raw_ptr_buffer_load_lds(r, (TASFT_LDS void*)dst, 16, voff, 0, 0, AUX);
 }
 
 template <int D, int DT>
@@ -970,6 +774,317 @@ bsfa_prefill_bs64_2w_kernel(const PrefillParams p) {
   }
 }
 
+// ---------------------------------------------------------------------------------------
+// Block size 32: one wave per (batch, query head, query block of 32 rows).
+//
+// Neighbouring 32-row query blocks and query heads have their own masks, so a tile that
+// several waves share would be mostly masked work; every wave walks its own blocks with its
+// own LDS tiles instead, and needs no barrier at all. A step takes NT active key blocks
+// (any two: the tile is gathered), 8 KB of K and 8 KB of V at the most: head dim 128 one
+// block, head dim 64 two. K and V arrive by buffer_load_dwordx4 ... lds in the layouts of the
+// block-64 kernels; V's DMA runs under the S MFMAs and the softmax, the next K's under the
+// softmax and PV. Unlike in the block-64 kernels the exp2 reference follows every new
+// maximum, tile by tile: the largest probability of a tile is then exactly 1 and carries no
+// rounding error (the lazy rescale measured 9% faster and its fp16 output 8% further from
+// 64 bits).
+//
+// Bound by the latency of a step (DMA, S, softmax and PV of one wave in turn), hidden by the
+// waves beside it: LDS allows ten per CU, three per SIMD at D=64 need 168 registers at most
+// (two, with 185, measured 5% slower). Against staging through registers with a transpose
+// of V by VALU: B=2, 16 heads, S=4000, D=64, a quarter of the blocks, fp16 48 us (106 us);
+// B=2, 32/8 heads, S=4096, D=128, a fifth, bf16 98 us (261 us). One block per step at D=64
+// took 51.7 us in the first case (and 6% less than two with twice the rows).
+// ---------------------------------------------------------------------------------------
+// SMALL: every row of Q, K and V lies within 2 GB of its head's first (32-bit offsets).
+template <int D, int NT, int DT, bool SMALL>
+__global__ void __launch_bounds__(64) __attribute__((amdgpu_waves_per_eu(D == 64 ? 3 : 2)))
+bsfa_prefill_bs32_kernel(const PrefillParams p) {
+  constexpr int BS = 32;
+  constexpr int KSTEPS = D / 16;
+  constexpr int DTILES = D / 32;
+  constexpr int ROWB = D * 2;
+  constexpr int UPB = BS * ROWB / 1024;  // 1 KB DMA units per block
+  constexpr int RPU = 1024 / ROWB;       // rows per unit
+  constexpr int WAITN = NT * UPB;        // DMA units of one K or V tile
+  static_assert(WAITN == 4 || WAITN == 8, "vmcnt of one tile");
+
+  __shared__ __attribute__((aligned(1024))) uint8_t kS[NT * BS * ROWB];
+  __shared__ __attribute__((aligned(1024))) uint8_t vS[NT * BS * ROWB];
+
+  const int lane = threadIdx.x;
+  const int col = lane & 31;
+  const int half = lane >> 5;
+
+  const PrefillItem item = prefill_item(p, (int64_t)blockIdx.x);
+  const int qb = item.qb, b = item.b, kvh = item.kvh, h = item.h;
+  // Varlen launch: items past the last query block of a shorter sequence have no work.
+  const SeqSpan span = seq_span<BS>(p, b);
+  if (qb >= span.NB) return;
+  const int S = span.S, NB = span.NB;
+
+  const uint16_t* qbase = p.q + b * p.sq[0] + span.tok0 * p.sq[2] + h * p.sq[1];
+  const uint16_t* kbase = p.k + b * p.sk[0] + span.tok0 * p.sk[2] + kvh * p.sk[1];
+  const uint16_t* vbase = p.v + b * p.sv[0] + span.tok0 * p.sv[2] + kvh * p.sv[1];
+  uint16_t* obase = p.o + b * p.so[0] + span.tok0 * p.so[2] + h * p.so[1];
+  const uint8_t* mrow = p.mask + b * p.sm[0] + h * p.sm[1] + (int64_t)qb * p.sm[2];
+
+  const int qrow = qb * BS + col;
+  const int kb_end = p.causal ? qb + 1 : NB;
+  // Blocks from here on need element masks (causal diagonal or partial last block).
+  const int mask_from = p.causal ? qb : ((S % BS) != 0 ? NB - 1 : NB);
+  uint8_t mb = 0;
+  if (lane < kb_end) mb = mrow[(int64_t)lane * p.sm[3]];
+
+  // One 32-row block to `tile`, unit by unit: the lane loads the global chunk that the
+  // (self-inverse) swizzle maps to its 16 bytes. The buffer ends with row S-1, so rows past
+  // it (and every row of a block at or past S) arrive as zeros. `voff` is 32-bit: without
+  // SMALL each unit gets its own base, and offsets count from there.
+  auto dma_block = [&](uint8_t* tile, const uint16_t* base, int64_t stride, int row0,
+                       const uint32_t* voff, auto aux) {
+    constexpr int AUX = decltype(aux)::value;
+    const uint32_t rb = (uint32_t)stride * 2u;
+    if constexpr (SMALL) {
+      const int left = S - row0;
+      const __amdgpu_buffer_rsrc_t r = __builtin_amdgcn_make_buffer_rsrc(
+          (void*)((const uint8_t*)base + (uint32_t)row0 * rb), (short)0,
+          left > 0 ? (int)((uint32_t)(left - 1) * rb + ROWB) : 0, 0x00020000);
+#pragma unroll
+      for (int u = 0; u < UPB; ++u) dma16_lds<AUX>(r, tile + u * 1024, (int)voff[u]);
+    } else {
+#pragma unroll
+      for (int u = 0; u < UPB; ++u) {
+        const int64_t left = (int64_t)S - row0 - u * RPU;
+        dma16_lds<AUX>(tile_rsrc((const uint8_t*)base + (int64_t)(row0 + u * RPU) * stride * 2,
+                                 left > 0 ? (left - 1) * stride * 2 + ROWB : 0),
+                       tile + u * 1024, (int)(voff[u] - (uint32_t)(u * RPU) * rb));
+      }
+    }
+  };
+  uint32_t kvoff[UPB], vvoff[UPB];
+#pragma unroll
+  for (int u = 0; u < UPB; ++u) {
+    const int row = u * RPU + lane / (ROWB / 16), pos = lane % (ROWB / 16);
+    kvoff[u] = ((uint32_t)row * (uint32_t)p.sk[2] + swz_k<D>(row, pos) * 8) * 2u;
+    vvoff[u] = ((uint32_t)row * (uint32_t)p.sv[2] + swz_v<D>(row, pos) * 8) * 2u;
+  }
+  using Default = std::integral_constant<int, 0>;
+  using Streamed = std::integral_constant<int, 2>;  // non-temporal: Q is read once
+  {
+    // Q through the V tile, unused until the first V DMA, in K's layout.
+    uint32_t qvoff[UPB];
+#pragma unroll
+    for (int u = 0; u < UPB; ++u) {
+      const int row = u * RPU + lane / (ROWB / 16), pos = lane % (ROWB / 16);
+      qvoff[u] = ((uint32_t)row * (uint32_t)p.sq[2] + swz_k<D>(row, pos) * 8) * 2u;
+    }
+    dma_block(vS, qbase, p.sq[2], qb * BS, qvoff, Streamed{});
+  }
+
+  // The next NT active blocks; -1 where the row has no more (their keys are masked off).
+  int chunk = 0;
+  uint64_t bits = __ballot(mb != 0);
+  auto next_step = [&](int (&kb)[NT]) {
+#pragma unroll
+    for (int t = 0; t < NT; ++t)
+      kb[t] = (t > 0 && kb[t - 1] < 0)
+                  ? -1
+                  : next_active_block(mrow, p.sm[3], kb_end, lane, chunk, bits, 0);
+  };
+  // A missing second block is loaded from row S on, which is all zeros.
+  auto dma_k = [&](const int (&kb)[NT]) {
+#pragma unroll
+    for (int t = 0; t < NT; ++t)
+      dma_block(kS + t * BS * ROWB, kbase, p.sk[2], kb[t] < 0 ? S : kb[t] * BS, kvoff, Default{});
+  };
+  auto dma_v = [&](const int (&kb)[NT]) {
+#pragma unroll
+    for (int t = 0; t < NT; ++t)
+      dma_block(vS + t * BS * ROWB, vbase, p.sv[2], kb[t] < 0 ? S : kb[t] * BS, vvoff, Default{});
+  };
+  // vmcnt of one tile's units: everything older than the last tile has landed.
+  auto wait_all_but_one_tile = [&]() {
+    if constexpr (WAITN == 8)
+      __builtin_amdgcn_s_waitcnt(0x0f78);
+    else
+      __builtin_amdgcn_s_waitcnt(0x0f74);
+    asm volatile("" ::: "memory");
+  };
+
+  int kb[NT];
+  next_step(kb);
+  u32x4_t qf[KSTEPS];
+  if (kb[0] >= 0) {
+    dma_k(kb);
+    wait_all_but_one_tile();  // Q landed, K in flight
+  } else {
+    __builtin_amdgcn_s_waitcnt(0x0f70);
+    asm volatile("" ::: "memory");
+  }
+#pragma unroll
+  for (int ks = 0; ks < KSTEPS; ++ks)
+    qf[ks] = *(const u32x4_t*)(vS + col * ROWB + swz_k<D>(col, ks * 2 + half) * 16);
+
+  f32x16_t oacc[DTILES];
+#pragma unroll
+  for (int dt = 0; dt < DTILES; ++dt) oacc[dt] = (f32x16_t){};
+  float m_ref = -INFINITY;  // exp2 reference of this lane's query row (log2 domain)
+  float l_run = 0.f;
+  const int grp16 = lane >> 4, t16 = lane & 15;  // ds_read_tr group and lane in group
+  const int tr_row = t16 >> 2;                   // source row offset within a 4-row run
+  const int tr_cb = t16 & 3;                     // source 8-byte column block
+
+  while (kb[0] >= 0) {
+    // vmcnt(0) lgkmcnt(0): K landed, and the reads of the V tile (Q, the last PV) returned.
+    __builtin_amdgcn_s_waitcnt(0x0070);
+    asm volatile("" ::: "memory");
+    dma_v(kb);
+    u32x4_t kf[NT][KSTEPS];
+#pragma unroll
+    for (int t = 0; t < NT; ++t)
+#pragma unroll
+      for (int ks = 0; ks < KSTEPS; ++ks) {
+        const int r = t * 32 + col;
+        kf[t][ks] = *(const u32x4_t*)(kS + r * ROWB + swz_k<D>(r, ks * 2 + half) * 16);
+      }
+    f32x16_t s[NT];
+#pragma unroll
+    for (int t = 0; t < NT; ++t) s[t] = (f32x16_t){};
+#pragma unroll
+    for (int ks = 0; ks < KSTEPS; ++ks)
+#pragma unroll
+      for (int t = 0; t < NT; ++t) s[t] = mfma16<DT>(kf[t][ks], qf[ks], s[t]);
+    __builtin_amdgcn_s_waitcnt(0xc07f);  // lgkmcnt(0): the K reads returned, the tile is free
+    asm volatile("" ::: "memory");
+    int kb_next[NT];
+    next_step(kb_next);
+    // Always one K tile after V (a row's last step loads its own again), so that the V wait
+    // below is one fixed count.
+    int kb_load[NT];
+#pragma unroll
+    for (int t = 0; t < NT; ++t) kb_load[t] = kb_next[0] >= 0 ? kb_next[t] : kb[t];
+    dma_k(kb_load);
+    const bool ragged = kb[NT - 1] < 0;
+    if (ragged || kb[NT - 1] >= mask_from) {
+      // Register rr of tile t holds key kb[t]*32 + 4*half + off(rr), off = 8*(rr/4) + rr%4,
+      // admissible iff off <= lim.
+      const int last = p.causal ? min(qrow, S - 1) : S - 1;
+#pragma unroll
+      for (int t = 0; t < NT; ++t) {
+        const int lim = kb[t] < 0 ? -1 : last - kb[t] * BS - 4 * half;
+#pragma unroll
+        for (int rr = 0; rr < 16; ++rr)
+          s[t][rr] = 8 * (rr >> 2) + (rr & 3) > lim ? -INFINITY : s[t][rr];
+      }
+    }
+    // Scores stay unscaled: scale > 0 commutes with max, and exp2 takes one FMA. Each
+    // 32-key tile has its own reference (the running maximum after it).
+    float ref[NT], alpha[NT];
+    bool moved[NT];
+#pragma unroll
+    for (int t = 0; t < NT; ++t) {
+      float m = fmaxf(fmaxf(s[t][0], s[t][1]), s[t][2]);
+#pragma unroll
+      for (int rr = 3; rr < 15; rr += 2) m = fmaxf(fmaxf(m, s[t][rr]), s[t][rr + 1]);
+      const float mloc = pair_max32(fmaxf(m, s[t][15])) * p.scale_log2;
+      const bool move = mloc > m_ref;
+      moved[t] = __ballot(move) != 0;
+      // exp2(-inf) = 0 clears the (empty) accumulators on a row's first finite score.
+      alpha[t] = move ? __builtin_amdgcn_exp2f(m_ref - mloc) : 1.f;
+      m_ref = move ? mloc : m_ref;
+      ref[t] = (m_ref == -INFINITY) ? 0.f : m_ref;
+    }
+#pragma unroll
+    for (int t = 0; t < NT; ++t) {
+      float lsum = 0.f;
+#pragma unroll
+      for (int rr = 0; rr < 16; ++rr) {
+        const float e = __builtin_amdgcn_exp2f(fmaf(s[t][rr], p.scale_log2, -ref[t]));
+        s[t][rr] = e;
+        lsum += e;
+      }
+      l_run = l_run * alpha[t] + lsum;
+    }
+    // P^T as the B operand of 16-key k-steps: keys 16pp + 8*(j>>2) + 4*half + (j&3) of a
+    // tile for element j, the same key order the V^T reads below use.
+    u32x4_t pb[2 * NT];
+#pragma unroll
+    for (int pp = 0; pp < 2 * NT; ++pp) {
+      const f32x16_t& sv = s[pp >> 1];
+      const int o = 8 * (pp & 1);
+      const u32x4_t w = {pack16x2<DT>(sv[o + 0], sv[o + 1]), pack16x2<DT>(sv[o + 2], sv[o + 3]),
+                         pack16x2<DT>(sv[o + 4], sv[o + 5]), pack16x2<DT>(sv[o + 6], sv[o + 7])};
+      pb[pp] = w;
+    }
+    wait_all_but_one_tile();  // V landed, the next K in flight
+    u32x2_t vlo[2 * NT][DTILES], vhi[2 * NT][DTILES];
+#pragma unroll
+    for (int pp = 0; pp < 2 * NT; ++pp) {
+      const int kk = 16 * pp + 4 * (grp16 >> 1);  // first key of run 1
+#pragma unroll
+      for (int dt = 0; dt < DTILES; ++dt) {
+        const int d0 = dt * 32 + 16 * (grp16 & 1) + 4 * tr_cb;  // source column of this lane
+        const int cc = d0 >> 3, sub = (d0 & 7) * 2;
+        const int r1 = kk + tr_row, r2 = r1 + 8;
+        vlo[pp][dt] = ds_read_tr16_b64((const void*)(vS + r1 * ROWB + swz_v<D>(r1, cc) * 16 + sub));
+        vhi[pp][dt] = ds_read_tr16_b64((const void*)(vS + r2 * ROWB + swz_v<D>(r2, cc) * 16 + sub));
+      }
+    }
+#pragma unroll
+    for (int t = 0; t < NT; ++t) {
+      if (moved[t]) {
+#pragma unroll
+        for (int dt = 0; dt < DTILES; ++dt) oacc[dt] *= alpha[t];
+      }
+#pragma unroll
+      for (int pp = 2 * t; pp < 2 * t + 2; ++pp)
+#pragma unroll
+        for (int dt = 0; dt < DTILES; ++dt) {
+          const u32x4_t a = {vlo[pp][dt][0], vlo[pp][dt][1], vhi[pp][dt][0], vhi[pp][dt][1]};
+          oacc[dt] = mfma16<DT>(a, pb[pp], oacc[dt]);
+        }
+    }
+#pragma unroll
+    for (int t = 0; t < NT; ++t) kb[t] = kb_next[t];
+  }
+  // No DMA into this workgroup's LDS outlives it, and the reads of the V tile are done.
+  __builtin_amdgcn_s_waitcnt(0x0070);
+  asm volatile("" ::: "memory");
+
+  const float l_tot = pair_sum32(l_run);
+  const float inv = 1.f / (l_tot > 0.f ? l_tot : 1.f);  // empty rows: O = 0; NaN rows stay NaN
+  // The output through the V tile, so that whole rows leave: 16-byte chunk c of row r at
+  // position c ^ (r mod chunks). One wave's LDS accesses execute in order.
+  constexpr int CPR = ROWB / 16;
+#pragma unroll
+  for (int dt = 0; dt < DTILES; ++dt)
+#pragma unroll
+    for (int gq = 0; gq < 4; ++gq) {
+      const int d0 = dt * 32 + 8 * gq + 4 * half;
+      const u32x2_t w = {pack16x2<DT>(oacc[dt][4 * gq + 0] * inv, oacc[dt][4 * gq + 1] * inv),
+                         pack16x2<DT>(oacc[dt][4 * gq + 2] * inv, oacc[dt][4 * gq + 3] * inv)};
+      *(u32x2_t*)(vS + col * ROWB + (((d0 >> 3) ^ (col & (CPR - 1))) << 4) + (d0 & 7) * 2) = w;
+    }
+  asm volatile("" ::: "memory");
+#pragma unroll
+  for (int j = 0; j < BS * CPR / kWave; ++j) {
+    const int r = j * (kWave / CPR) + lane / CPR, c = lane % CPR;
+    const u32x4_t v = *(const u32x4_t*)(vS + r * ROWB + ((c ^ (r & (CPR - 1))) << 4));
+    // Non-temporal: the output is not read again here, and K/V stay in L2.
+    if (qb * BS + r < S)
+      __builtin_nontemporal_store(v, (u32x4_t*)(obase + (int64_t)(qb * BS + r) * p.so[2] + c * 8));
+  }
+}
+
+template <int D, int NT, int DT>
+static hipError_t launch_prefill_bs32(const PrefillParams& p, hipStream_t stream) {
+  const int64_t grid = (int64_t)p.NB * p.B * p.Hq;
+  if (p.small_spans && p.small_q)
+    hipLaunchKernelGGL((bsfa_prefill_bs32_kernel<D, NT, DT, true>), dim3((unsigned)grid), dim3(kWave), 0, stream, p);
+  else
+    hipLaunchKernelGGL((bsfa_prefill_bs32_kernel<D, NT, DT, false>), dim3((unsigned)grid), dim3(kWave), 0, stream, p);
+  return hipGetLastError();
+}
+
 // Compute units of the current device (cached per device).
 static int device_cus() {
   static int cached[64] = {0};
@@ -1038,8 +1153,8 @@ static hipError_t launch_prefill_any(const PrefillParams& p, int* queue, int64_t
   }
   if (block_size == 64 && head_dim == 128) return launch_prefill_bs64<128, DT>(p, queue, s);
   if (block_size == 64 && head_dim == 64) return launch_prefill_bs64<64, DT>(p, queue, s);
-  if (head_dim == 128) return launch_prefill<32, 128, DT>(p, s);  // block 32
-  return launch_prefill<32, 64, DT>(p, s);
+  if (head_dim == 128) return launch_prefill_bs32<128, 1, DT>(p, s);  // block 32
+  return launch_prefill_bs32<64, 2, DT>(p, s);
 }
 
 }  // namespace tasft
@@ -1139,6 +1254,7 @@ extern "C" int tasft_bsfa_prefill_fwd(const void* q, const void* k, const void* 
   p.causal = causal ? 1 : 0;
   p.small_spans = (seq_len * k_strides[2] * 2 < 0x7fffffffLL &&
                    seq_len * v_strides[2] * 2 < 0x7fffffffLL) ? 1 : 0;
+  p.small_q = seq_len * q_strides[2] * 2 < 0x7fffffffLL ? 1 : 0;
   p.queue = nullptr;
   p.parts = 1;
   p.wg_per_part = 1;
@@ -1272,6 +1388,7 @@ extern "C" int tasft_bsfa_prefill_varlen_fwd(const void* q, const void* k, const
   p.causal = causal ? 1 : 0;
   p.small_spans = (max_seqlen * k_strides[0] * 2 < 0x7fffffffLL &&
                    max_seqlen * v_strides[0] * 2 < 0x7fffffffLL) ? 1 : 0;
+  p.small_q = max_seqlen * q_strides[0] * 2 < 0x7fffffffLL ? 1 : 0;
   p.queue = nullptr;
   p.parts = 1;
   p.wg_per_part = 1;
