@@ -341,6 +341,30 @@ int tasft_gate_bwd(const float* soft_scores, const float* grad_soft, const void*
                    int64_t block_size, int64_t hidden, int flags, void* stream);
 
 /*
+ * Gradients of the gate's parameters, from dL/dsoft to dL/dW_in, dL/db_in and dL/dw_out: the
+ * pairwise sums of tasft_gate_bwd, reduced on the device, with the weight products. Replaces
+ * what the reference gets from autograd through AttnGate.forward
+ * (tasft/modules/attn_gate.py:248-273).
+ *
+ * soft_scores, grad_soft, fwd_workspace: as in tasft_gate_bwd; q_means [B, Hq, NB, D] and
+ * k_means [B, Hkv, NB, D]: the block means of the same tasft_gate_fwd call; w_out [hidden].
+ * Outputs, fp32 contiguous: dw_in [hidden, 2 D], db_in [hidden], dw_out [hidden], and the
+ * gradients of the projected units du [B, Hq, NB, hidden] (u = W_q qbar + b_in) and
+ * dv [B, Hkv, NB, hidden] (v = W_k kbar, summed over the query heads of a KV head), from which
+ * gradients of Q and K follow. Every sum runs in a fixed order. head_dim at most 256.
+ * workspace: >= tasft_gate_grads_workspace_bytes(...) bytes. flags: TASFT_GATE_CAUSAL.
+ */
+size_t tasft_gate_grads_workspace_bytes(int64_t batch, int64_t num_q_heads, int64_t num_kv_heads,
+                                        int64_t seq_len, int64_t head_dim, int64_t block_size,
+                                        int64_t hidden);
+int tasft_gate_grads(const float* soft_scores, const float* grad_soft, const void* fwd_workspace,
+                     size_t fwd_workspace_bytes, const float* q_means, const float* k_means,
+                     const float* w_out, float* du, float* dv, float* dw_in, float* db_in,
+                     float* dw_out, void* workspace, size_t workspace_bytes, int64_t batch,
+                     int64_t num_q_heads, int64_t num_kv_heads, int64_t seq_len, int64_t head_dim,
+                     int64_t block_size, int64_t hidden, int flags, void* stream);
+
+/*
  * Gate target from Q and K, without the [B, H, S, S] score tensor.
  * Replaces the score producer TASFTAttention._training_forward
  * (tasft/modules/tasft_attention.py:426-458) followed by

@@ -36,6 +36,8 @@ EXPORTED_SYMBOLS = (
     "tasft_gate_decode_rows_fwd",
     "tasft_gate_bwd_workspace_bytes",
     "tasft_gate_bwd",
+    "tasft_gate_grads_workspace_bytes",
+    "tasft_gate_grads",
     "tasft_gate_target_fwd",
     "tasft_gate_kl_fwd",
     "tasft_mask_compact_workspace_bytes",
@@ -104,6 +106,12 @@ _SIGNATURES: dict[str, tuple[object, list[object]]] = {
     "tasft_gate_bwd": (
         _I,
         [_P, _P, _P, _SZ, _P, _SZ, _I64, _I64, _I64, _I64, _I64, _I64, _I, _P],
+    ),
+    "tasft_gate_grads_workspace_bytes": (_SZ, [_I64, _I64, _I64, _I64, _I64, _I64, _I64]),
+    "tasft_gate_grads": (
+        _I,
+        [_P, _P, _P, _SZ, _P, _P, _P, _P, _P, _P, _P, _P, _P, _SZ, _I64, _I64, _I64, _I64, _I64,
+         _I64, _I64, _I, _P],
     ),
     "tasft_gate_kl_fwd": (_I, [_P, _P, _I64, _I64, _I64, _I64, _P, _P, _P]),
     "tasft_gate_target_fwd": (

@@ -267,7 +267,7 @@ class AttnGate(nn.Module):
 
     def _forward_hip_train(self, q: torch.Tensor, k: torch.Tensor, tau: float | torch.Tensor,
                            force_diagonal: bool) -> GateOutput:
-        """HIP forward plus HIP backward (``tasft_gate_bwd``) through autograd: the soft
+        """HIP forward plus HIP backward (``tasft_gate_grads``) through autograd: the soft
         scores carry gradients to the gate parameters (and to Q/K if they require them)
         without materialising the ``[B, H, NB, NB, hidden]`` activations."""
         taus = self._thresholds(tau, q.device)
@@ -450,8 +450,8 @@ class _HipGateFunction(torch.autograd.Function):
     """AttnGate forward/backward on the HIP kernels (gate training).
 
     Backward, with g = dL/dsoft * soft * (1 - soft) (0 where the causal zero applied) and
-    pre_ijc = u_ic + v_jc (u = W_q qbar + b_in, v = W_k kbar): ``tasft_gate_bwd`` reduces
-    the pairwise terms; the rest are plain GEMMs on [B, H, NB, .] tensors:
+    pre_ijc = u_ic + v_jc (u = W_q qbar + b_in, v = W_k kbar), ``tasft_gate_grads`` gives the
+    parameter gradients and dL/du, dL/dv:
       dL/dw_out = sum g relu(pre);  dL/du = w_out * sum_j g [pre > 0];
       dL/dv = w_out * sum_i g [pre > 0] (summed over the query heads of each KV head);
       dL/db_in = sum du;  dL/dW_in = [du^T qbar, dv^T kbar];
@@ -478,22 +478,19 @@ class _HipGateFunction(torch.autograd.Function):
         lib = _native.load_library()
         dev = soft.device
         gs = grad_soft.to(torch.float32).contiguous()
-        pbytes = lib.tasft_gate_bwd_workspace_bytes(B, H, S, bs, hidden)
-        partials = torch.empty(pbytes // 4, dtype=torch.float32, device=dev)
-        status = lib.tasft_gate_bwd(soft.data_ptr(), gs.data_ptr(), workspace.data_ptr(),
-                                    workspace.numel(), partials.data_ptr(), pbytes, B, H, Hkv, S,
-                                    bs, hidden, 1 if causal else 0, _native.stream_handle(dev))
-        _native.check(status, "tasft_gate_bwd", {"shape": [B, H, S, D]})
-        tiles = (nb + 31) // 32
-        plane = B * H * nb * hidden
-        du = partials[: tiles * plane].view(tiles, B, H, nb, hidden).sum(0) * w_out
-        dv = (partials[tiles * plane: 2 * tiles * plane].view(tiles, B, Hkv, H // Hkv, nb, hidden)
-              .sum((0, 3)) * w_out)
-        dw_out = partials[2 * tiles * plane:].view(-1, hidden).sum(0)
-        db_in = du.sum((0, 1, 2))
-        dw_q = _weight_grad(du.reshape(-1, hidden), qm.reshape(-1, D))
-        dw_k = _weight_grad(dv.reshape(-1, hidden), km.reshape(-1, D))
-        dw_in = torch.cat([dw_q, dw_k], dim=1)
+        du = torch.empty((B, H, nb, hidden), dtype=torch.float32, device=dev)
+        dv = torch.empty((B, Hkv, nb, hidden), dtype=torch.float32, device=dev)
+        dw_in = torch.empty((hidden, 2 * D), dtype=torch.float32, device=dev)
+        db_in = torch.empty((hidden,), dtype=torch.float32, device=dev)
+        dw_out = torch.empty((hidden,), dtype=torch.float32, device=dev)
+        n = lib.tasft_gate_grads_workspace_bytes(B, H, Hkv, S, D, bs, hidden)
+        partials = torch.empty(n, dtype=torch.uint8, device=dev)
+        status = lib.tasft_gate_grads(
+            soft.data_ptr(), gs.data_ptr(), workspace.data_ptr(), workspace.numel(), qm.data_ptr(),
+            km.data_ptr(), w_out.data_ptr(), du.data_ptr(), dv.data_ptr(), dw_in.data_ptr(),
+            db_in.data_ptr(), dw_out.data_ptr(), partials.data_ptr(), n, B, H, Hkv, S, D, bs, hidden,
+            1 if causal else 0, _native.stream_handle(dev))
+        _native.check(status, "tasft_gate_grads", {"shape": [B, H, S, D]})
         gq = gk = None
         if ctx.needs_input_grad[0]:
             dqbar = (du @ w_in[:, :D]) / bs
