@@ -409,6 +409,29 @@ int tasft_gate_kl_fwd(const float* gate_scores, const float* target, int64_t bat
                       float* loss_partials, float* grad_scores, void* stream);
 
 /*
+ * tasft_gate_kl_fwd with the loss itself and the check of the scores: *loss receives the sum
+ * of loss_partials divided by B, and status [3] (device int32, zeroed by the caller before the
+ * call) gets in status[1] bit 0 if gate_scores hold a NaN and bit 1 if an infinity
+ * (objectives.py:67-87 rejects both); status[2] is used as a counter.
+ */
+int tasft_gate_kl_loss(const float* gate_scores, const float* target, int64_t batch,
+                       int64_t num_heads, int64_t num_blocks_q, int64_t num_blocks_k,
+                       float* loss_partials, float* grad_scores, float* loss, int* status,
+                       void* stream);
+
+/*
+ * An additive attention mask in the form tasft_gate_target_fwd reads: dst [batch, num_heads,
+ * dst_rows, dst_keys] fp32 contiguous receives src [batch, num_heads, num_rows, seq_len] (fp32,
+ * element strides src_strides[4]) with zeros past it. batch and num_heads are the mask's own
+ * (1 where it broadcasts). status[0] (device int32, zeroed by the caller) gets bit 0 if src holds
+ * a NaN and bit 1 if +inf, which the reference's compute_gate_target rejects
+ * (tasft/training/objectives.py:150-163).
+ */
+int tasft_gate_mask_pad(const float* src, const int64_t* src_strides, int64_t batch,
+                        int64_t num_heads, int64_t num_rows, int64_t seq_len, float* dst,
+                        int64_t dst_rows, int64_t dst_keys, int* status, void* stream);
+
+/*
  * Block mask -> compressed rows (CSR) of its active blocks.
  * No reference counterpart: the reference hands its Triton kernel the dense mask and
  * scans every byte of a row (tasft/kernels/block_sparse_fa.py:192-203); this gives

@@ -40,6 +40,8 @@ EXPORTED_SYMBOLS = (
     "tasft_gate_grads",
     "tasft_gate_target_fwd",
     "tasft_gate_kl_fwd",
+    "tasft_gate_kl_loss",
+    "tasft_gate_mask_pad",
     "tasft_mask_compact_workspace_bytes",
     "tasft_mask_compact",
     "tasft_mask_from_indices",
@@ -114,6 +116,8 @@ _SIGNATURES: dict[str, tuple[object, list[object]]] = {
          _I64, _I64, _I, _P],
     ),
     "tasft_gate_kl_fwd": (_I, [_P, _P, _I64, _I64, _I64, _I64, _P, _P, _P]),
+    "tasft_gate_kl_loss": (_I, [_P, _P, _I64, _I64, _I64, _I64, _P, _P, _P, _P, _P]),
+    "tasft_gate_mask_pad": (_I, [_P, _I64P, _I64, _I64, _I64, _I64, _P, _I64, _I64, _P, _P]),
     "tasft_gate_target_fwd": (
         _I,
         [_P, _P, _P, _P, _I64, _I64, _I64, _I64, _I64, _I64, _I64P, _I64P, _I64P, _F, _I, _I,

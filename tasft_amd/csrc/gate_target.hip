@@ -599,8 +599,56 @@ static hipError_t dispatch_blockmax(const GateTargetParams& p, int64_t block_siz
 //   L = sum_i t_i (log t_i - log u_i)            (entries with t_i = 0 contribute 0),
 //   dL/dg_k = (-t_k / u_k + (sum_i t_i g_i / u_i) / Z) / Z.
 // loss_part[bh] receives L; grad (optional) receives inv_batch * dL/dg (the reference
-// reduces with "batchmean": the sum over (b, h) divided by B).
+// reduces with "batchmean": the sum over (b, h) divided by B). With `loss`, the workgroup
+// that finishes last adds the parts in order (64-bit sum) into *loss, and status[1] collects
+// bit 0 for a NaN and bit 1 for an infinity among the scores; status[2] counts workgroups and,
+// like status[1], must start at zero. Doing both here saves the separate passes over the
+// scores (four element-wise kernels and a reduction, 33 us at 16.8 MB) and the two launches
+// of the sum.
 constexpr float kKlEps = 1e-8f;
+
+// Bit 0: some lane's value is a NaN, bit 1: an infinity (integer tests: the build assumes no
+// NaN in float arithmetic).
+__device__ __forceinline__ int nonfinite_bits(float v) {
+  const uint32_t u = __float_as_uint(v) & 0x7fffffffu;
+  return u > 0x7f800000u ? 1 : (u == 0x7f800000u ? 2 : 0);
+}
+__device__ __forceinline__ void raise_status(int* word, int bits) {
+  const int all = (__ballot(bits & 1) ? 1 : 0) | (__ballot(bits & 2) ? 2 : 0);
+  if (all && (threadIdx.x & 63) == 0) atomicOr(word, all);
+}
+
+struct KlFinish {
+  float* loss;  // or null: partials only
+  int* status;  // [3] with loss, see above
+};
+
+// Thread 0 has stored this workgroup's part with an agent-scope store and calls this with
+// the whole workgroup; the last workgroup sums the parts.
+template <int THREADS>
+__device__ __forceinline__ void kl_finish(const KlFinish& f, const float* loss_part, float inv_batch) {
+  __shared__ int last;
+  __shared__ double sums[THREADS / 64];
+  if (threadIdx.x == 0) {
+    __builtin_amdgcn_s_waitcnt(0x0070);  // the part is at the device's coherence point
+    last = __hip_atomic_fetch_add(f.status + 2, 1, __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_AGENT) ==
+           (int)gridDim.x - 1;
+  }
+  __syncthreads();
+  if (!last) return;
+  double acc = 0.0;
+  for (int64_t i = threadIdx.x; i < (int64_t)gridDim.x; i += THREADS)
+    acc += (double)__hip_atomic_load(loss_part + i, __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_AGENT);
+#pragma unroll
+  for (int off = 32; off >= 1; off >>= 1) acc += __shfl_xor(acc, off, 64);
+  if ((threadIdx.x & 63) == 0) sums[threadIdx.x >> 6] = acc;
+  __syncthreads();
+  if (threadIdx.x == 0) {
+    double t = 0.0;
+    for (int w = 0; w < THREADS / 64; ++w) t += sums[w];
+    *f.loss = (float)(t * inv_batch);
+  }
+}
 
 __device__ __forceinline__ float block_sum256(float v, float* red) {
   v = wave_sum(v);
@@ -612,14 +660,20 @@ __device__ __forceinline__ float block_sum256(float v, float* red) {
 
 __global__ void __launch_bounds__(256)
 gate_kl_kernel(const float* soft, const float* target, int64_t n, float inv_batch,
-               float* loss_part, float* grad) {
+               float* loss_part, float* grad, const KlFinish fin) {
   __shared__ float red[4];
   const int64_t bh = blockIdx.x;
   const float* g = soft + bh * n;
   const float* t = target + bh * n;
   const int tid = threadIdx.x;
   float z = 0.f;
-  for (int64_t i = tid; i < n; i += 256) z += g[i];
+  int bad = 0;
+  for (int64_t i = tid; i < n; i += 256) {
+    const float v = g[i];
+    z += v;
+    bad |= nonfinite_bits(v);
+  }
+  if (fin.loss) raise_status(fin.status + 1, bad);
   z = block_sum256(z, red) + kKlEps;
   const float inv_z = 1.f / z;
   float l = 0.f, s2 = 0.f;
@@ -634,7 +688,7 @@ gate_kl_kernel(const float* soft, const float* target, int64_t n, float inv_batc
   }
   l = block_sum256(l, red);
   s2 = block_sum256(s2, red);
-  if (tid == 0) loss_part[bh] = l;
+  if (tid == 0) __hip_atomic_store(loss_part + bh, l, __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_AGENT);
   if (grad) {
     float* gr = grad + bh * n;
     const float c = s2 * inv_z;
@@ -644,6 +698,7 @@ gate_kl_kernel(const float* soft, const float* target, int64_t n, float inv_batc
       gr[i] = inv_batch * inv_z * (c - ti / u);
     }
   }
+  if (fin.loss) kl_finish<256>(fin, loss_part, inv_batch);
 }
 
 
@@ -666,7 +721,7 @@ __device__ __forceinline__ float block_sum1024(float v, float* red) {
 
 __global__ void __launch_bounds__(kKlThreads)
 gate_kl_reg_kernel(const float* soft, const float* target, int64_t n, float inv_batch,
-                   float* loss_part, float* grad) {
+                   float* loss_part, float* grad, const KlFinish fin) {
   __shared__ float red[kKlThreads / 64];
   const int64_t bh = blockIdx.x;
   const float* g = soft + bh * n;
@@ -674,13 +729,16 @@ gate_kl_reg_kernel(const float* soft, const float* target, int64_t n, float inv_
   const int tid = threadIdx.x;
   float gv[kKlRegs], tv[kKlRegs];
   float z = 0.f;
+  int bad = 0;
 #pragma unroll
   for (int r = 0; r < kKlRegs; ++r) {
     const int64_t i = tid + (int64_t)r * kKlThreads;
     gv[r] = i < n ? g[i] : 0.f;
     tv[r] = i < n ? t[i] : 0.f;
     z += gv[r];
+    bad |= nonfinite_bits(gv[r]);
   }
+  if (fin.loss) raise_status(fin.status + 1, bad);
   z = block_sum1024(z, red) + kKlEps;
   const float inv_z = 1.f / z;
   float l = 0.f, s2 = 0.f;
@@ -694,7 +752,7 @@ gate_kl_reg_kernel(const float* soft, const float* target, int64_t n, float inv_
   }
   l = block_sum1024(l, red);
   s2 = block_sum1024(s2, red);
-  if (tid == 0) loss_part[bh] = l;
+  if (tid == 0) __hip_atomic_store(loss_part + bh, l, __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_AGENT);
   if (grad) {
     float* gr = grad + bh * n;
     const float c = s2 * inv_z;
@@ -704,6 +762,39 @@ gate_kl_reg_kernel(const float* soft, const float* target, int64_t n, float inv_
       if (i < n) gr[i] = inv_batch * inv_z * (c - tv[r] / (gv[r] * inv_z + kKlEps));
     }
   }
+  if (fin.loss) kl_finish<kKlThreads>(fin, loss_part, inv_batch);
+}
+
+// An additive mask as the target kernels read it: dst [B', H', R', padded] fp32 contiguous
+// (each leading dim 1 or full) gets src's values (element strides ss, S keys, R rows) with
+// zeros past them. status[0] collects bit 0 for a NaN and bit 1 for +inf in src (-inf masks);
+// it must start at zero.
+struct MaskPadParams {
+  const float* src;
+  float* dst;
+  int* status;
+  int64_t ss[4];
+  int64_t n;  // elements of dst
+  int H, R, rows, S, padded;  // rows: rows of dst per (b, h)
+};
+
+__global__ void __launch_bounds__(256)
+gate_mask_pad_kernel(const MaskPadParams p) {
+  int bad = 0;
+  for (int64_t i = (int64_t)blockIdx.x * 256 + threadIdx.x; i < p.n; i += (int64_t)gridDim.x * 256) {
+    const int64_t row = i / p.padded;
+    const int c = (int)(i % p.padded);
+    const int r = (int)(row % p.rows);
+    const int64_t bh = row / p.rows;
+    float v = 0.f;
+    if (c < p.S && r < p.R) {
+      v = p.src[(bh / p.H) * p.ss[0] + (bh % p.H) * p.ss[1] + r * p.ss[2] + c * p.ss[3]];
+      const int b = nonfinite_bits(v);
+      bad |= (b == 2 && __float_as_uint(v) == 0xff800000u) ? 0 : b;
+    }
+    p.dst[i] = v;
+  }
+  raise_status(p.status, bad);
 }
 
 }  // namespace tasft
@@ -817,9 +908,10 @@ extern "C" int tasft_gate_target_fwd(const void* q, const void* k, const float* 
   return kOk;
 }
 
-extern "C" int tasft_gate_kl_fwd(const float* gate_scores, const float* target, int64_t batch,
-                                 int64_t num_heads, int64_t num_blocks_q, int64_t num_blocks_k,
-                                 float* loss_partials, float* grad_scores, void* stream) {
+static int gate_kl_launch(const float* gate_scores, const float* target, int64_t batch,
+                          int64_t num_heads, int64_t num_blocks_q, int64_t num_blocks_k,
+                          float* loss_partials, float* grad_scores, const KlFinish& fin,
+                          void* stream) {
   if (!gate_scores || !target || !loss_partials)
     return set_error(kErrInvalidArgument, "gate_kl: null pointer argument");
   if (batch <= 0 || num_heads <= 0 || num_blocks_q <= 0 || num_blocks_k <= 0)
@@ -830,13 +922,60 @@ extern "C" int tasft_gate_kl_fwd(const float* gate_scores, const float* target, 
   if (n <= (int64_t)kKlThreads * kKlRegs)
     hipLaunchKernelGGL(gate_kl_reg_kernel, dim3((unsigned)(batch * num_heads)), dim3(kKlThreads), 0,
                        (hipStream_t)stream, gate_scores, target, n, 1.f / (float)batch,
-                       loss_partials, grad_scores);
+                       loss_partials, grad_scores, fin);
   else
     hipLaunchKernelGGL(gate_kl_kernel, dim3((unsigned)(batch * num_heads)), dim3(256), 0,
                        (hipStream_t)stream, gate_scores, target, n, 1.f / (float)batch,
-                       loss_partials, grad_scores);
+                       loss_partials, grad_scores, fin);
   const hipError_t err = hipGetLastError();
   if (err != hipSuccess)
     return set_error(kErrLaunch, "gate_kl: launch failed: %s", hipGetErrorString(err));
+  return kOk;
+}
+
+extern "C" int tasft_gate_kl_fwd(const float* gate_scores, const float* target, int64_t batch,
+                                 int64_t num_heads, int64_t num_blocks_q, int64_t num_blocks_k,
+                                 float* loss_partials, float* grad_scores, void* stream) {
+  return gate_kl_launch(gate_scores, target, batch, num_heads, num_blocks_q, num_blocks_k,
+                        loss_partials, grad_scores, KlFinish{nullptr, nullptr}, stream);
+}
+
+extern "C" int tasft_gate_kl_loss(const float* gate_scores, const float* target, int64_t batch,
+                                  int64_t num_heads, int64_t num_blocks_q, int64_t num_blocks_k,
+                                  float* loss_partials, float* grad_scores, float* loss,
+                                  int* status, void* stream) {
+  if (!loss || !status) return set_error(kErrInvalidArgument, "gate_kl: null pointer argument");
+  return gate_kl_launch(gate_scores, target, batch, num_heads, num_blocks_q, num_blocks_k,
+                        loss_partials, grad_scores, KlFinish{loss, status}, stream);
+}
+
+extern "C" int tasft_gate_mask_pad(const float* src, const int64_t* src_strides, int64_t batch,
+                                   int64_t num_heads, int64_t num_rows, int64_t seq_len,
+                                   float* dst, int64_t dst_rows, int64_t dst_keys, int* status,
+                                   void* stream) {
+  if (!src || !src_strides || !dst || !status)
+    return set_error(kErrInvalidArgument, "gate_mask_pad: null pointer argument");
+  if (batch <= 0 || num_heads <= 0 || num_rows <= 0 || seq_len <= 0 || dst_rows < num_rows ||
+      dst_keys < seq_len || dst_rows > 0x7fffffffLL || dst_keys > 0x7fffffffLL ||
+      num_heads > 0x7fffffffLL)
+    return set_error(kErrInvalidArgument, "gate_mask_pad: invalid sizes");
+  if (!strides_nonneg(src_strides, 4))
+    return set_error(kErrInvalidArgument, "gate_mask_pad: strides must be non-negative");
+  MaskPadParams p;
+  p.src = src;
+  p.dst = dst;
+  p.status = status;
+  for (int j = 0; j < 4; ++j) p.ss[j] = src_strides[j];
+  p.n = batch * num_heads * dst_rows * dst_keys;
+  p.H = (int)num_heads;
+  p.R = (int)num_rows;
+  p.rows = (int)dst_rows;
+  p.S = (int)seq_len;
+  p.padded = (int)dst_keys;
+  const int64_t blocks = std::min<int64_t>((p.n + 255) / 256, 8192);
+  hipLaunchKernelGGL(gate_mask_pad_kernel, dim3((unsigned)blocks), dim3(256), 0, (hipStream_t)stream, p);
+  const hipError_t err = hipGetLastError();
+  if (err != hipSuccess)
+    return set_error(kErrLaunch, "gate_mask_pad: launch failed: %s", hipGetErrorString(err));
   return kOk;
 }

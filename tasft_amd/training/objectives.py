@@ -124,6 +124,16 @@ def gate_target_from_qk(
         temperature: divide pooled maxima by this before the softmax.
         clamp: if set, clamp finite maxima to ``[-clamp, clamp]`` first.
     """
+    _check_target_inputs(q, k, normalize, temperature)
+    status = _new_status(q.device) if attention_mask is not None else None
+    out = _launch_gate_target(q, k, block_size, causal, scale, normalize, temperature, clamp,
+                              attention_mask, status)
+    if status is not None:
+        _check_mask(int(status[0].item()), attention_mask)
+    return out
+
+
+def _check_target_inputs(q: torch.Tensor, k: torch.Tensor, normalize: str, temperature: float) -> None:
     if q.ndim != 4 or k.ndim != 4:
         raise KernelError("Expected 4D q and k [B, H, S, D]", context={"q": list(q.shape), "k": list(k.shape)})
     B, H, S, D = q.shape
@@ -133,11 +143,38 @@ def gate_target_from_qk(
         raise KernelError("Tensors must be on CUDA device", context={"device": str(q.device)})
     if k.dtype != q.dtype:
         raise KernelError("q and k must have one dtype", context={"q": str(q.dtype), "k": str(k.dtype)})
-    dtype = _native.dtype_code(q.dtype, "gate target kernel")
+    _native.dtype_code(q.dtype, "gate target kernel")
     if normalize not in _NORMALIZE:
         raise ValueError(f"normalize must be one of {sorted(_NORMALIZE)}, got {normalize!r}")
     if not temperature > 0.0:
         raise ValueError(f"temperature must be > 0, got {temperature}")
+
+
+def _new_status(device: torch.device) -> torch.Tensor:
+    """Device status words of one call: [0] the mask's, [1] the gate scores', [2] a counter."""
+    return torch.zeros(3, dtype=torch.int32, device=device)
+
+
+def _nonfinite_error(name: str, tensor: torch.Tensor, bits: int, label: str) -> NaNDetectedError:
+    """The reference's NaN/Inf error for a tensor whose status bits are ``bits`` (1 NaN, 2 Inf)."""
+    has_nan, has_inf = bool(bits & 1), bool(bits & 2)
+    return NaNDetectedError(
+        f"Non-finite values detected in {name}: NaN={has_nan}, Inf={has_inf}",
+        context={"tensor_name": label, "has_nan": has_nan, "has_inf": has_inf,
+                 "shape": list(tensor.shape), "dtype": str(tensor.dtype)},
+    )
+
+
+def _check_mask(bits: int, attention_mask: torch.Tensor) -> None:
+    if bits:
+        raise _nonfinite_error("attn_scores", attention_mask, bits, "attention_mask")
+
+
+def _launch_gate_target(q, k, block_size, causal, scale, normalize, temperature, clamp,
+                        attention_mask, status) -> torch.Tensor:
+    """``gate_target_from_qk`` after its checks; the mask's go to ``status[0]``, unread."""
+    B, H, S, D = q.shape
+    dtype = _native.dtype_code(q.dtype, "gate target kernel")
     lib = _native.load_library()
     q = q if (q.stride(-1) == 1 and all(s % 8 == 0 for s in q.stride()[:-1])) else q.contiguous()
     k = k if (k.stride(-1) == 1 and all(s % 8 == 0 for s in k.stride()[:-1])) else k.contiguous()
@@ -147,24 +184,24 @@ def gate_target_from_qk(
         # The kernels read a mask up to a multiple of 64 rows and keys as well (block 32 runs
         # over 64-token blocks).
         padded = max(nb * block_size, 64 * math.ceil(S / 64))
-        mask_buf, mask_strides = _padded_attention_mask(attention_mask, B, H, S, padded, q.device)
+        mask_buf, mask_strides = _padded_attention_mask(attention_mask, B, H, S, padded, q.device, status)
     out = torch.empty((B, H, nb, nb), dtype=torch.float32, device=q.device)
     sc = float(scale) if scale is not None else 1.0 / math.sqrt(D)
-    status = lib.tasft_gate_target_fwd(
+    code = lib.tasft_gate_target_fwd(
         q.data_ptr(), k.data_ptr(), _native.ptr(mask_buf), out.data_ptr(), B, H, k.shape[1], S, D,
         block_size, _native.strides(q), _native.strides(k), mask_strides, sc, 1 if causal else 0,
         _NORMALIZE[normalize], float(temperature), float(clamp) if clamp is not None else 0.0,
         dtype, _native.stream_handle(q.device),
     )
-    _native.check(status, "tasft_gate_target_fwd", {"shape": [B, H, S, D]})
+    _native.check(code, "tasft_gate_target_fwd", {"shape": [B, H, S, D]})
     return out
 
 
 def _padded_attention_mask(mask: torch.Tensor, B: int, H: int, S: int, padded: int,
-                           device: torch.device):
+                           device: torch.device, status: torch.Tensor):
     """The kernel's form of an additive mask: fp32 ``[B|1, H|1, padded|1, padded]`` with the
     caller's values in the leading ``S`` rows/columns (broadcast dims keep size 1 and get
-    stride 0), and its (b, h, query) element strides."""
+    stride 0), and its (b, h, query) element strides. NaN and +inf are noted in ``status[0]``."""
     ext = mask[:, None, None, :] if mask.ndim == 2 else mask
     if ext.ndim != 4:
         raise KernelError(f"attention_mask must be 2-D [B, S] or 4-D, got {mask.ndim}-D",
@@ -175,49 +212,50 @@ def _padded_attention_mask(mask: torch.Tensor, B: int, H: int, S: int, padded: i
             f"attention_mask shape {tuple(mask.shape)} does not broadcast to {want}",
             context={"attention_mask": list(mask.shape), "scores": list(want)},
         )
-    ext = ext.to(device=device, dtype=torch.float32)
-    has_nan = bool(torch.isnan(ext).any())
-    has_pos_inf = bool((ext == float("inf")).any())
-    if has_nan or has_pos_inf:
-        raise NaNDetectedError(
-            f"Non-finite values detected in attn_scores: NaN={has_nan}, Inf={has_pos_inf}",
-            context={"tensor_name": "attention_mask", "has_nan": has_nan, "has_inf": has_pos_inf,
-                     "shape": list(mask.shape), "dtype": str(mask.dtype)},
-        )
-    rows = padded if ext.shape[2] > 1 else 1
-    buf = torch.zeros((ext.shape[0], ext.shape[1], rows, padded), dtype=torch.float32, device=device)
-    buf[:, :, : ext.shape[2], :S] = ext
+    ext = ext.detach().to(device=device, dtype=torch.float32)
+    mb, mh, mr, _ = ext.shape
+    rows = padded if mr > 1 else 1
+    buf = torch.empty((mb, mh, rows, padded), dtype=torch.float32, device=device)
+    code = _native.load_library().tasft_gate_mask_pad(
+        ext.data_ptr(), _native.strides(ext), mb, mh, mr, S, buf.data_ptr(), rows, padded,
+        status.data_ptr(), _native.stream_handle(device))
+    _native.check(code, "tasft_gate_mask_pad", {"attention_mask": list(mask.shape)})
     st = buf.stride()
-    strides = [st[0] if buf.shape[0] > 1 else 0, st[1] if buf.shape[1] > 1 else 0,
-               st[2] if rows > 1 else 0]
+    strides = [st[0] if mb > 1 else 0, st[1] if mh > 1 else 0, st[2] if rows > 1 else 0]
     return buf, _native.strides_array(strides)
 
 
 class _GateKL(torch.autograd.Function):
-    """KL gate loss on the GPU (``tasft_gate_kl_fwd``): the loss and d(loss)/d(gate scores)
-    come from one kernel; backward scales the saved gradient."""
+    """KL gate loss on the GPU (``tasft_gate_kl_loss``): the loss and d(loss)/d(gate scores)
+    come from one kernel; backward scales the saved gradient. ``status`` (see
+    ``_new_status``) receives the check of the scores."""
 
     @staticmethod
-    def forward(ctx, gate_soft: torch.Tensor, target: torch.Tensor) -> torch.Tensor:
+    def forward(ctx, gate_soft: torch.Tensor, target: torch.Tensor,
+                status: torch.Tensor | None = None) -> torch.Tensor:
         b, h, nbq, nbk = gate_soft.shape
         g = gate_soft.detach().to(torch.float32).contiguous()
         t = target.detach().to(torch.float32).contiguous()
+        if status is None:
+            status = _new_status(g.device)
         partial = torch.empty(b * h, dtype=torch.float32, device=g.device)
+        loss = torch.empty((), dtype=torch.float32, device=g.device)
         grad = torch.empty_like(g) if ctx.needs_input_grad[0] else None
         lib = _native.load_library()
-        status = lib.tasft_gate_kl_fwd(g.data_ptr(), t.data_ptr(), b, h, nbq, nbk, partial.data_ptr(),
-                                       _native.ptr(grad), _native.stream_handle(g.device))
-        _native.check(status, "tasft_gate_kl_fwd", {"shape": [b, h, nbq, nbk]})
+        code = lib.tasft_gate_kl_loss(g.data_ptr(), t.data_ptr(), b, h, nbq, nbk, partial.data_ptr(),
+                                      _native.ptr(grad), loss.data_ptr(), status.data_ptr(),
+                                      _native.stream_handle(g.device))
+        _native.check(code, "tasft_gate_kl_loss", {"shape": [b, h, nbq, nbk]})
         ctx.save_for_backward(grad)
         ctx.in_dtype = gate_soft.dtype
-        return partial.sum() / b
+        return loss
 
     @staticmethod
     def backward(ctx, grad_out: torch.Tensor):
         (grad,) = ctx.saved_tensors
         if grad is None:
-            return None, None
-        return (grad * grad_out).to(ctx.in_dtype), None
+            return None, None, None
+        return (grad * grad_out).to(ctx.in_dtype), None, None
 
 
 def gate_loss_from_qk(
@@ -246,14 +284,28 @@ def gate_loss_from_qk(
                           context={"shape": list(gate_soft_scores.shape)})
     if not gate_soft_scores.is_cuda:
         raise KernelError("Tensors must be on CUDA device", context={"device": str(gate_soft_scores.device)})
-    target = gate_target_from_qk(q, k, block_size, causal=causal, scale=scale,
-                                 attention_mask=attention_mask)
+    _check_target_inputs(q, k, "flat", 1.0)
+    status = _new_status(q.device)
+    target = _launch_gate_target(q, k, block_size, causal, scale, "flat", 1.0, None, attention_mask,
+                                 status)
     if tuple(target.shape) != tuple(gate_soft_scores.shape):
+        _check_mask(int(status[0].item()), attention_mask)
         raise KernelError(
             f"gate scores {tuple(gate_soft_scores.shape)} do not match the target grid {tuple(target.shape)}",
             context={"gate": list(gate_soft_scores.shape), "target": list(target.shape)})
-    _check_finite(gate_soft_scores, "gate_soft_scores")
-    return _GateKL.apply(gate_soft_scores, target)
+    # The kernel checks the scores as it reads them in fp32; a wider type is checked as it is.
+    in_kernel = gate_soft_scores.dtype in (torch.float32, torch.bfloat16, torch.float16)
+    if not in_kernel:
+        _check_mask(int(status[0].item()), attention_mask)
+        _check_finite(gate_soft_scores, "gate_soft_scores")
+    loss = _GateKL.apply(gate_soft_scores, target, status)
+    if in_kernel:
+        # One read for both checks, after everything is queued.
+        mask_bits, gate_bits, _ = status.tolist()
+        _check_mask(mask_bits, attention_mask)
+        if gate_bits:
+            raise _nonfinite_error("gate_soft_scores", gate_soft_scores, gate_bits, "gate_soft_scores")
+    return loss
 
 
 __all__ = ["TASFTObjective", "gate_loss_from_qk", "gate_target_from_qk"]
