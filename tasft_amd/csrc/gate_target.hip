@@ -14,6 +14,8 @@
 // prefill kernel (v_mfma_f32_32x32x16_bf16, or _f16 for fp16 inputs; fp32 accumulation)
 // and keeps only the maximum of every 64x64 tile, so the work is the QK^T half of a dense
 // causal prefill and nothing of size S^2 touches HBM. Kernel 2 normalises in place.
+#include <algorithm>
+
 #include "common.h"
 
 #include "../../include/tasft_amd.h"
@@ -42,6 +44,11 @@ struct GateTargetParams {
   // by the host). Each 32 x 32 quarter of a 64 x 64 score tile is then a whole block,
   // written as it is computed.
   int fine;
+  // One-wave kernel: take the groups in turn at each query slot (all long rows first) instead
+  // of one after another.
+  int interleave;
+  // One-wave kernel: key blocks per workgroup; blockIdx.y counts a row's runs of them.
+  int run;
 };
 
 // Float max into global memory by integer atomics: a value with the sign bit clear orders
@@ -146,8 +153,8 @@ gate_target_normalize_reg_kernel(float* data, int64_t group_len, float inv_temp,
   }
 }
 
-// Block size 64, scores with an additive mask (unmasked scores run the one-wave-per-head
-// kernel below, 7% faster at config 5). A workgroup owns one query block of HPW query heads
+// Block size 64, scores with an additive mask of its own for every query (scores without one
+// run the one-wave-per-head kernel below, 7% faster at config 5). A workgroup owns one query block of HPW query heads
 // of the same KV head (the target is dense, so these heads read exactly the same K blocks)
 // with WPH waves per head: with WPH = 2 (the launched form) wave (hw, w) takes head hw, query rows 32*w..+31
 // and all 64 keys of every causal key block (16 MFMAs per block); with WPH = 4 it takes
@@ -163,10 +170,10 @@ __device__ __forceinline__ int gt_swz(int r, int cc) {
 }
 
 //
-// MASKED adds the caller's additive mask: each wave loads the mask values of its 32 x 64
+// The caller's additive mask: each wave loads the mask values of its 32 x 64
 // sub-tile (float4 per lane and 4-key group) before it issues the next block's DMA, so the
 // fixed DMA wait also covers them, and adds them to the scaled scores before the max.
-template <int D, int HPW, bool MASKED, int DT, int WPH = 2>
+template <int D, int HPW, int DT, int WPH = 2>
 __global__ void __launch_bounds__(HPW * WPH * 64)
 gate_target_bs64_kernel(const GateTargetParams p) {
   constexpr int BS = 64;
@@ -218,9 +225,7 @@ gate_target_bs64_kernel(const GateTargetParams p) {
 
   const int qrow = qb * BS + rh * 32 + col;
   const bool qvalid = qrow < p.S;
-  const float* mrow = MASKED ? p.amask + b * p.sam[0] + h * p.sam[1] + (int64_t)qrow * p.sam[2]
-                             : nullptr;
-  const float post_scale = MASKED ? 1.f : p.scale;
+  const float* mrow = p.amask + b * p.sam[0] + h * p.sam[1] + (int64_t)qrow * p.sam[2];
   u32x4_t qf[KSTEPS];
   auto load_q = [&]() {
 #pragma unroll
@@ -257,15 +262,13 @@ gate_target_bs64_kernel(const GateTargetParams p) {
   // One block from stage kt: this wave's 32 x 32 (or 32 x 64) sub-tile maximum.
   constexpr int NKT = WPH == 4 ? 1 : 2;  // 32-key tiles per wave
   using f32x4_t = float __attribute__((ext_vector_type(4)));
-  f32x4_t mv[NKT][4];  // mask values of this lane's keys (MASKED)
+  f32x4_t mv[NKT][4];  // mask values of this lane's keys
   auto load_mask = [&](int kb) {
-    if constexpr (MASKED) {
 #pragma unroll
-      for (int t = 0; t < NKT; ++t)
+    for (int t = 0; t < NKT; ++t)
 #pragma unroll
-        for (int g4 = 0; g4 < 4; ++g4)
-          mv[t][g4] = *(const f32x4_t*)(mrow + kb * BS + kh * 32 + 32 * t + 8 * g4 + 4 * half);
-    }
+      for (int g4 = 0; g4 < 4; ++g4)
+        mv[t][g4] = *(const f32x4_t*)(mrow + kb * BS + kh * 32 + 32 * t + 8 * g4 + 4 * half);
   };
   auto block_max = [&](const uint8_t* kt, int kb) {
     f32x16_t s[NKT];
@@ -282,12 +285,10 @@ gate_target_bs64_kernel(const GateTargetParams p) {
       }
     }
     const int key0 = kb * BS;
-    if constexpr (MASKED) {
 #pragma unroll
-      for (int t = 0; t < NKT; ++t)
+    for (int t = 0; t < NKT; ++t)
 #pragma unroll
-        for (int rr = 0; rr < 16; ++rr) s[t][rr] = s[t][rr] * p.scale + mv[t][rr >> 2][rr & 3];
-    }
+      for (int rr = 0; rr < 16; ++rr) s[t][rr] = s[t][rr] * p.scale + mv[t][rr >> 2][rr & 3];
     if ((p.causal && kb == qb) || (key0 + BS > p.S) || qb * BS + BS > p.S) {
 #pragma unroll
       for (int t = 0; t < NKT; ++t)
@@ -314,8 +315,8 @@ gate_target_bs64_kernel(const GateTargetParams p) {
         const int r = 2 * qb + rh;
         if (lane == 0 && r < p.NBO) {
           float* o = p.out + (((int64_t)b * p.Hq + h) * p.NBO + r) * p.NBO + 2 * kb;
-          o[0] = m * post_scale;
-          if (2 * kb + 1 < p.NBO) o[1] = m2 * post_scale;
+          o[0] = m;
+          if (2 * kb + 1 < p.NBO) o[1] = m2;
         }
         return 0.f;
       }
@@ -323,18 +324,17 @@ gate_target_bs64_kernel(const GateTargetParams p) {
     }
     return wave_max_dpp(m);
   };
-  // Combine the four partial maxima of this head's block kb (slot kb & 1), scaled.
+  // Combine the partial maxima of this head's block kb (slot kb & 1).
   auto store = [&](int kb) {
     if ((tid % HT) == 0 && !p.fine) {
       const float* rm = red[kb & 1][hw];
       float m = rm[0];
 #pragma unroll
       for (int i = 1; i < WPH; ++i) m = fmaxf(m, rm[i]);
-      // Scaling by scale > 0 before the max is exact: rounding is monotonic.
       if (p.pool)
-        gt_atomic_fmax(orow + (kb >> 1), m * post_scale);
+        gt_atomic_fmax(orow + (kb >> 1), m);
       else
-        orow[kb] = m * post_scale;
+        orow[kb] = m;
     }
   };
 
@@ -374,37 +374,50 @@ gate_target_bs64_kernel(const GateTargetParams p) {
   store(kb_end - 1);
 }
 
-// Unmasked scores: one wave per (head, query block), its 64 query rows as two 32-row MFMA
-// column tiles. Every K fragment read from LDS feeds both row tiles, halving the LDS reads
-// per MFMA of the two-waves-per-head kernel above, and the block maximum is one wave's:
-// no exchange between waves. HPW heads of one KV group share each K tile (three stages,
-// two blocks in flight, as above).
-template <int D, int HPW, int DT>
-__global__ void __launch_bounds__(HPW * 64) __attribute__((amdgpu_waves_per_eu(2)))
+constexpr int kW1Waves = 4;
+
+// One wave per (head, query block), its 64 query rows as two 32-row MFMA column tiles: scores
+// without a mask, or with a key-padding row. Every K fragment read from LDS feeds both row
+// tiles, halving the LDS reads per MFMA of the two-waves-per-head kernel above, and the block
+// maximum is one wave's: no exchange between waves. Four waves share each K tile (three
+// stages, two blocks in flight, as above): the heads of a KV group at one query block, and
+// where their number is not a multiple of four the next query block's heads after them (a
+// wave whose row has ended then only helps to load).
+// ROWMASK: an additive mask without a query dimension (a key-padding row), p.sam[2] == 0. A
+// lane's score registers are keys, so it needs the same 32 mask values for all its query
+// rows: eight 16-byte loads a block, issued before the next block's DMA.
+// EVEN: the heads of a group fill whole workgroups, so that all waves' rows are equally long;
+// without the per-wave limit the loop measured 5% faster.
+template <int D, int DT, bool ROWMASK, bool EVEN>
+__global__ void __launch_bounds__(kW1Waves * 64) __attribute__((amdgpu_waves_per_eu(2)))
 gate_target_bs64_w1_kernel(const GateTargetParams p) {
   constexpr int BS = 64;
   constexpr int KSTEPS = D / 16;
   constexpr int ROWB = D * 2;
   constexpr int TILE = BS * ROWB;
   constexpr int UNITS = TILE / 1024;
-  static_assert(UNITS % HPW == 0, "equal DMA units per wave");
-  constexpr int UPW = UNITS / HPW;
+  static_assert(UNITS % kW1Waves == 0, "equal DMA units per wave");
+  constexpr int UPW = UNITS / kW1Waves;
   __shared__ __attribute__((aligned(1024))) uint8_t k0[TILE];
   __shared__ __attribute__((aligned(1024))) uint8_t k1[TILE];
   __shared__ __attribute__((aligned(1024))) uint8_t k2[TILE];
 
   const int tid = threadIdx.x;
   const int lane = tid & 63;
-  const int wave = tid >> 6;  // head within the workgroup
+  const int wave = __builtin_amdgcn_readfirstlane(tid >> 6);
   const int col = lane & 31;
   const int half = lane >> 5;
 
-  const int chunks = p.G / HPW;
+  // Row r of a group is head r % G at query slot r / G; the longest causal rows come first.
   const int64_t idx = blockIdx.x;
   const int64_t groups = (int64_t)p.B * p.Hkv;
-  const int64_t per_group = (int64_t)chunks * p.NB;
+  const int rows = p.G * p.NB;
+  const int64_t per_group = (rows + kW1Waves - 1) / kW1Waves;
   int64_t grp, r;
-  if ((groups & 7) == 0) {
+  if (p.interleave) {
+    grp = idx % groups;
+    r = idx / groups;
+  } else if ((groups & 7) == 0) {
     const int64_t j = idx >> 3;
     grp = (idx & 7) + 8 * (j / per_group);
     r = j % per_group;
@@ -412,11 +425,13 @@ gate_target_bs64_w1_kernel(const GateTargetParams p) {
     grp = idx / per_group;
     r = idx % per_group;
   }
-  const int qslot = (int)(r / chunks);
+  const int row0 = (int)r * kW1Waves, row = min(row0 + wave, rows - 1);
+  const bool has_row = EVEN || row0 + wave < rows;
+  const int qslot = row / p.G;
   const int qb = p.causal ? (p.NB - 1 - qslot) : qslot;
   const int b = (int)(grp / p.Hkv);
   const int kvh = (int)(grp % p.Hkv);
-  const int h = kvh * p.G + (int)(r % chunks) * HPW + wave;
+  const int h = kvh * p.G + row % p.G;
 
   const uint16_t* qbase = p.q + b * p.sq[0] + h * p.sq[1];
   const uint16_t* kbase = p.k + b * p.sk[0] + kvh * p.sk[1];
@@ -440,11 +455,11 @@ gate_target_bs64_w1_kernel(const GateTargetParams p) {
         qf[rt][ks] = val;
       }
   };
-  // DMA units of this wave: u = wave, wave + HPW, ...
+  // DMA units of this wave: u = wave, wave + kW1Waves, ...
   int koff[UPW];
 #pragma unroll
   for (int i = 0; i < UPW; ++i) {
-    const int u = wave + i * HPW;
+    const int u = wave + i * kW1Waves;
     const int byte = u * 1024 + lane * 16;
     const int row = byte / ROWB, pos = (byte % ROWB) / 16;
     koff[i] = (row * (int)p.sk[2] + gt_swz<D>(row, pos) * 8) * 2;
@@ -456,7 +471,18 @@ gate_target_bs64_w1_kernel(const GateTargetParams p) {
         (void*)(kbase + (int64_t)key0 * p.sk[2]), (short)0,
         bytes > 0x7fffffff ? 0x7fffffff : (int)bytes, 0x00020000);
 #pragma unroll
-    for (int i = 0; i < UPW; ++i) gt_dma16(rs, kt + (wave + i * HPW) * 1024, koff[i]);
+    for (int i = 0; i < UPW; ++i) gt_dma16(rs, kt + (wave + i * kW1Waves) * 1024, koff[i]);
+  };
+  const float* mrow = ROWMASK ? p.amask + b * p.sam[0] + h * p.sam[1] + 4 * half : nullptr;
+  const float post_scale = ROWMASK ? 1.f : p.scale;
+  f32x4_t mv[2][4];  // mask values of this lane's keys
+  auto load_mask = [&](int kb) {
+    if constexpr (ROWMASK) {
+#pragma unroll
+      for (int t = 0; t < 2; ++t)
+#pragma unroll
+        for (int g4 = 0; g4 < 4; ++g4) mv[t][g4] = *(const f32x4_t*)(mrow + kb * BS + 32 * t + 8 * g4);
+    }
   };
   // Block kb from stage kt: its maximum (or, for 32-token output blocks, the maxima of its
   // four 32 x 32 quarters), written by lane 0.
@@ -478,6 +504,14 @@ gate_target_bs64_w1_kernel(const GateTargetParams p) {
       }
     }
     const int key0 = kb * BS;
+    if constexpr (ROWMASK) {
+#pragma unroll
+      for (int rt = 0; rt < 2; ++rt)
+#pragma unroll
+        for (int t = 0; t < 2; ++t)
+#pragma unroll
+          for (int rr = 0; rr < 16; ++rr) s[rt][t][rr] = s[rt][t][rr] * p.scale + mv[t][rr >> 2][rr & 3];
+    }
     if ((p.causal && kb == qb) || (key0 + BS > p.S) || qb * BS + BS > p.S) {
 #pragma unroll
       for (int rt = 0; rt < 2; ++rt)
@@ -512,14 +546,14 @@ gate_target_bs64_w1_kernel(const GateTargetParams p) {
           const int rq = 2 * qb + rt;
           if (rq >= p.NBO) continue;
           float* o = p.out + (((int64_t)b * p.Hq + h) * p.NBO + rq) * p.NBO + 2 * kb;
-          o[0] = m[rt][0] * p.scale;
-          if (2 * kb + 1 < p.NBO) o[1] = m[rt][1] * p.scale;
+          o[0] = m[rt][0] * post_scale;
+          if (2 * kb + 1 < p.NBO) o[1] = m[rt][1] * post_scale;
         }
       }
       return;
     }
     // Scaling by scale > 0 after the max is exact: rounding is monotonic.
-    const float mx = wave_max_dpp(fmaxf(fmaxf(m[0][0], m[0][1]), fmaxf(m[1][0], m[1][1]))) * p.scale;
+    const float mx = wave_max_dpp(fmaxf(fmaxf(m[0][0], m[0][1]), fmaxf(m[1][0], m[1][1]))) * post_scale;
     if (lane == 0) {
       if (p.pool)
         gt_atomic_fmax(orow + (kb >> 1), mx);
@@ -528,23 +562,30 @@ gate_target_bs64_w1_kernel(const GateTargetParams p) {
     }
   };
 
-  const int kb_end = p.causal ? qb + 1 : p.NB;
-  if (!p.pool && !p.fine)
-    for (int kb = kb_end + lane; kb < p.NB; kb += kWave) orow[kb] = -INFINITY;
+  // The run's blocks of this wave, and those the workgroup loads (wave 0's row is the
+  // longest). Runs past the end of the rows have nothing to do.
+  const int kb_first = (int)blockIdx.y * p.run;
+  const int kb_row = p.causal ? qb + 1 : p.NB;
+  const int kb_mine = has_row ? min(kb_row, kb_first + p.run) : 0;
+  const int kb_end = min(p.causal ? p.NB - row0 / p.G : p.NB, kb_first + p.run);
+  if (!p.pool && !p.fine && has_row && blockIdx.y == 0)
+    for (int kb = kb_row + lane; kb < p.NB; kb += kWave) orow[kb] = -INFINITY;
+  if (kb_first >= kb_end) return;
   // Three stages, two blocks in flight; past the last block the last one is loaded again,
   // so every wave has exactly UPW later DMA units outstanding when it waits for a block.
   constexpr int kWaitBlock = (UPW & 15) | ((UPW >> 4) << 14) | 0x0070;  // vmcnt(UPW)
   auto step = [&](int kb, const uint8_t* cur, uint8_t* nxt) {
     __builtin_amdgcn_s_waitcnt(kWaitBlock);  // this wave's DMA of block kb landed
     asm volatile("s_barrier" ::: "memory");  // every wave's; stage nxt is free
+    if (EVEN || kb < kb_mine) load_mask(kb);
     issue(nxt, min(kb + 2, kb_end - 1));
-    block_max(cur, kb);
+    if (EVEN || kb < kb_mine) block_max(cur, kb);
   };
-  issue(k0, 0);
+  issue(k0, kb_first);
   load_q();
   __builtin_amdgcn_s_waitcnt(0x0f70);  // vmcnt(0)
-  issue(k1, min(1, kb_end - 1));
-  for (int kb = 0; kb < kb_end; kb += 3) {
+  issue(k1, min(kb_first + 1, kb_end - 1));
+  for (int kb = kb_first; kb < kb_end; kb += 3) {
     step(kb, k0, k2);
     if (kb + 1 >= kb_end) break;
     step(kb + 1, k1, k0);
@@ -554,26 +595,36 @@ gate_target_bs64_w1_kernel(const GateTargetParams p) {
   __builtin_amdgcn_s_waitcnt(0x0070);  // vmcnt(0) lgkmcnt(0): no DMA outlives the workgroup
 }
 
+template <int D, int DT, bool ROWMASK>
+static hipError_t launch_blockmax_w1(const GateTargetParams& p, hipStream_t stream) {
+  const int64_t per_group = ((int64_t)p.G * p.NB + kW1Waves - 1) / kW1Waves;
+  const dim3 grid((unsigned)((int64_t)p.B * p.Hkv * per_group), (unsigned)((p.NB + p.run - 1) / p.run));
+  if (p.G % kW1Waves == 0)
+    hipLaunchKernelGGL((gate_target_bs64_w1_kernel<D, DT, ROWMASK, true>), grid, dim3(kW1Waves * 64), 0, stream, p);
+  else
+    hipLaunchKernelGGL((gate_target_bs64_w1_kernel<D, DT, ROWMASK, false>), grid, dim3(kW1Waves * 64), 0, stream, p);
+  return hipGetLastError();
+}
+
 template <int D, bool MASKED, int DT>
 static hipError_t launch_blockmax_bs64(const GateTargetParams& p, hipStream_t stream) {
-  const int hpw = (p.G % 4 == 0) ? 4 : (p.G % 2 == 0 ? 2 : 1);
-  const int64_t grid = (int64_t)p.NB * p.B * p.Hq / hpw;
   if constexpr (!MASKED) {
+    return launch_blockmax_w1<D, DT, false>(p, stream);
+  } else {
+    // A key-padding row runs the one-wave kernel (its mask values are a lane's own), a mask
+    // with a query dimension the two-wave one: the values of 64 rows do not fit beside 64
+    // rows' scores. Both give the same bits.
+    if (p.sam[2] == 0) return launch_blockmax_w1<D, DT, true>(p, stream);
+    const int hpw = (p.G % 4 == 0) ? 4 : (p.G % 2 == 0 ? 2 : 1);
+    const dim3 grid((unsigned)((int64_t)p.NB * p.B * p.Hq / hpw));
     if (hpw == 4)
-      hipLaunchKernelGGL((gate_target_bs64_w1_kernel<D, 4, DT>), dim3((unsigned)grid), dim3(4 * 64), 0, stream, p);
+      hipLaunchKernelGGL((gate_target_bs64_kernel<D, 4, DT>), grid, dim3(4 * 128), 0, stream, p);
     else if (hpw == 2)
-      hipLaunchKernelGGL((gate_target_bs64_w1_kernel<D, 2, DT>), dim3((unsigned)grid), dim3(2 * 64), 0, stream, p);
+      hipLaunchKernelGGL((gate_target_bs64_kernel<D, 2, DT>), grid, dim3(2 * 128), 0, stream, p);
     else
-      hipLaunchKernelGGL((gate_target_bs64_w1_kernel<D, 1, DT>), dim3((unsigned)grid), dim3(64), 0, stream, p);
+      hipLaunchKernelGGL((gate_target_bs64_kernel<D, 1, DT>), grid, dim3(128), 0, stream, p);
     return hipGetLastError();
   }
-  if (hpw == 4)
-    hipLaunchKernelGGL((gate_target_bs64_kernel<D, 4, MASKED, DT>), dim3((unsigned)grid), dim3(4 * 128), 0, stream, p);
-  else if (hpw == 2)
-    hipLaunchKernelGGL((gate_target_bs64_kernel<D, 2, MASKED, DT>), dim3((unsigned)grid), dim3(2 * 128), 0, stream, p);
-  else
-    hipLaunchKernelGGL((gate_target_bs64_kernel<D, 1, MASKED, DT>), dim3((unsigned)grid), dim3(128), 0, stream, p);
-  return hipGetLastError();
 }
 
 template <bool MASKED, int DT>
@@ -877,6 +928,17 @@ extern "C" int tasft_gate_target_fwd(const void* q, const void* k, const float* 
   p.pool = pool;
   p.NBO = (int)nb;
   p.fine = fine;
+  // One-wave kernel. Groups in turn when an XCD's share of K fits half its 4 MB L2 (B=4,
+  // 32/8 heads, S=1500, key-padding row: 73 us against 89 group by group).
+  const int64_t group_rows = (num_q_heads / num_kv_heads * nb_run + kW1Waves - 1) / kW1Waves;
+  p.interleave = (batch * num_kv_heads + 7) / 8 * seq_len * head_dim * 2 <= (2 << 20) ? 1 : 0;
+  // Rows are cut into runs when there are too few of them to even out over the 512 workgroups
+  // that run at once: about 640 runs' worth of blocks each, at least 8 (the start of a run, its
+  // Q and first K tile, costs about three blocks). B=2, 28/4, 16/16 and 8/2 heads, S=4096: 112,
+  // 85 and 45 us against 113, 103 and 67 uncut; B=1, 32/8 heads, S=1024: 14 against 21;
+  // B=4, S=4096 stays uncut (225 us, in runs of 32 blocks 235).
+  const int64_t all_blocks = batch * num_kv_heads * group_rows * (causal ? (nb_run + 1) / 2 : nb_run);
+  p.run = (int)std::min<int64_t>(nb_run, std::max<int64_t>(8, (all_blocks + 639) / 640));
 
   hipStream_t s = (hipStream_t)stream;
   hipError_t err;
