@@ -156,12 +156,20 @@ bsfa_decode_split_kernel(const DecodeParams p) {
   const int kv_len = p.kv_lens ? min(max(p.kv_lens[b], 0), p.S_kv) : p.S_kv;
   const int nb_valid = (kv_len + BS - 1) / BS;
 
-  // Mask bits of key block t for the group's heads.
+  // Mask bits of key block t for the group's heads: eight heads' bytes in flight at a time
+  // (heads past G read head G-1 again and are dropped).
   const uint8_t* mbase = p.mask + b * p.sm[0] + (int64_t)h0 * p.sm[1];
   auto head_bits = [&](int t) -> uint32_t {
+    const uint8_t* m = mbase + (int64_t)(t >> p.mshift) * p.sm[2];
     uint32_t bitsv = 0;
-    for (int gg = 0; gg < G; ++gg)
-      if (mbase[(int64_t)gg * p.sm[1] + (int64_t)(t >> p.mshift) * p.sm[2]]) bitsv |= 1u << gg;
+    for (int g0 = 0; g0 < G; g0 += 8) {
+      uint8_t by[8];
+#pragma unroll
+      for (int i = 0; i < 8; ++i) by[i] = m[(int64_t)min(g0 + i, G - 1) * p.sm[1]];
+#pragma unroll
+      for (int i = 0; i < 8; ++i)
+        if (by[i] != 0 && g0 + i < G) bitsv |= 1u << (g0 + i);
+    }
     return bitsv;
   };
   // Q^T as the B operand: lane (hc, g4) holds head h0+hc, head dims 32 ks + 8 g4 .. +7.
@@ -207,9 +215,11 @@ bsfa_decode_split_kernel(const DecodeParams p) {
   // Balanced splits: the blocks selected by any head of the group are numbered over the
   // whole row in block order, and split s takes entries [s*n/P, (s+1)*n/P). With one split
   // the count pass is skipped.
+  // Rows of at most NTH blocks are read once: the ballots of the one pass give both the
+  // number of selected blocks and each block's position.
   constexpr int NTH = kDecodeWaves * kWave;
   int start = 0, end = 0x7fffffff;
-  if (p.P > 1) {
+  if (p.P > 1 && nb_valid > NTH) {
     int cnt = 0;
     for (int t = tid; t < nb_valid; t += NTH) cnt += head_bits(t) != 0u ? 1 : 0;
 #pragma unroll
@@ -228,13 +238,18 @@ bsfa_decode_split_kernel(const DecodeParams p) {
     const uint64_t bal = __ballot(bv != 0u);
     if (lane == 0) wsum[wave] = __popcll(bal);
     __syncthreads();
+    const int n_chunk = (wsum[0] + wsum[1]) + (wsum[2] + wsum[3]);
+    if (p.P > 1 && nb_valid <= NTH) {
+      start = (int)(((int64_t)s * n_chunk) / p.P);
+      end = (int)(((int64_t)(s + 1) * n_chunk) / p.P);
+    }
     int pos = base + __popcll(bal & ((1ull << lane) - 1ull));
     for (int w = 0; w < wave; ++w) pos += wsum[w];
     if (bv != 0u && pos >= start && pos < end) {
       sel[pos - start] = t;
       hb[pos - start] = (uint16_t)bv;
     }
-    base += (wsum[0] + wsum[1]) + (wsum[2] + wsum[3]);
+    base += n_chunk;
     __syncthreads();
   }
   const int nsel = __builtin_amdgcn_readfirstlane(min(end, base) - start);
@@ -468,24 +483,72 @@ bsfa_decode_split_kernel(const DecodeParams p) {
   }
 }
 
-// Merge the P split partials of every (b, h) and write the output row.
+// Merge the P split partials of every (b, h) and write the output row: kCombineGroups threads
+// per output column, each over a share of the splits, eight splits' loads in flight at a time
+// (past the last one it is read again, and dropped). The partials come from other XCDs'
+// workgroups, so a load is a trip past L2 and a serial walk over the splits was its cost:
+// 32 splits 6 us (10.6 in one thread, a load at a time), 128 splits 10 us (36).
+constexpr int kCombineGroups = 4;
+
 template <int D, int DT>
-__global__ void __launch_bounds__(D)
+__global__ void __launch_bounds__(kCombineGroups * D)
 bsfa_decode_combine_kernel(const DecodeParams p) {
+  __shared__ float red_m[kCombineGroups];
+  __shared__ float red_l[kCombineGroups];
+  __shared__ float red_o[kCombineGroups][D];
   const int64_t bh = blockIdx.x;
   const int b = (int)(bh / p.Hq);
   const int h = (int)(bh % p.Hq);
-  const int d = threadIdx.x;
+  const int d = threadIdx.x % D, grp = threadIdx.x / D;
   const float* ml = p.ws_ml + bh * p.P * 2;
   const float* os = p.ws_o + bh * p.P * D;
+  const int first = grp * p.P / kCombineGroups, last = (grp + 1) * p.P / kCombineGroups;
+  float m[8], l[8], o[8];
+  auto load = [&](int s0) {
+#pragma unroll
+    for (int i = 0; i < 8; ++i) {
+      const int sp = min(s0 + i, p.P - 1);
+      m[i] = ml[2 * sp];
+      l[i] = ml[2 * sp + 1];
+      o[i] = os[(int64_t)sp * D + d];
+    }
+  };
+  load(first);
   float M = -INFINITY;
-  for (int sp = 0; sp < p.P; ++sp) M = fmaxf(M, ml[2 * sp]);
+#pragma unroll
+  for (int i = 0; i < 8; ++i)
+    if (first + i < last) M = fmaxf(M, m[i]);
+  for (int s0 = first + 8; s0 < last; s0 += 8) {
+    float mm[8];
+#pragma unroll
+    for (int i = 0; i < 8; ++i) mm[i] = ml[2 * min(s0 + i, last - 1)];
+#pragma unroll
+    for (int i = 0; i < 8; ++i) M = fmaxf(M, mm[i]);
+  }
+  if (d == 0) red_m[grp] = M;
+  __syncthreads();
+#pragma unroll
+  for (int g = 0; g < kCombineGroups; ++g) M = fmaxf(M, red_m[g]);
   const float Mu = (M == -INFINITY) ? 0.f : M;
   float L = 0.f, O = 0.f;
-  for (int sp = 0; sp < p.P; ++sp) {
-    const float f = __builtin_amdgcn_exp2f(ml[2 * sp] - Mu);
-    L += ml[2 * sp + 1] * f;
-    O += os[(int64_t)sp * D + d] * f;
+  for (int s0 = first; s0 < last; s0 += 8) {
+    if (s0 > first) load(s0);
+#pragma unroll
+    for (int i = 0; i < 8; ++i) {
+      if (s0 + i >= last) break;
+      const float f = __builtin_amdgcn_exp2f(m[i] - Mu);
+      L += l[i] * f;
+      O += o[i] * f;
+    }
+  }
+  if (d == 0) red_l[grp] = L;
+  red_o[grp][d] = O;
+  __syncthreads();
+  if (grp != 0) return;
+#pragma unroll
+  for (int g = 1; g < kCombineGroups; ++g) {
+    L += red_l[g];
+    O += red_o[g][d];
   }
   const float r = O / (L > 0.f ? L : 1.f);  // empty rows: O = 0; NaN rows stay NaN
   p.o[b * p.so[0] + h * p.so[1] + d] = f32_to16<DT>(r);
@@ -498,8 +561,8 @@ static hipError_t launch_decode_dt(const DecodeParams& p, hipStream_t stream) {
                      dim3(kDecodeWaves * kWave), 0, stream, p);
   hipError_t err = hipGetLastError();
   if (err != hipSuccess || p.P == 1) return err;
-  hipLaunchKernelGGL((bsfa_decode_combine_kernel<D, DT>), dim3((unsigned)((int64_t)p.B * p.Hq)), dim3(D),
-                     0, stream, p);
+  hipLaunchKernelGGL((bsfa_decode_combine_kernel<D, DT>), dim3((unsigned)((int64_t)p.B * p.Hq)),
+                     dim3(kCombineGroups * D), 0, stream, p);
   return hipGetLastError();
 }
 
