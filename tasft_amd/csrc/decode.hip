@@ -25,6 +25,7 @@
 #include "common.h"
 
 #include <mutex>
+#include <type_traits>
 
 #include "../../include/tasft_amd.h"
 
@@ -156,21 +157,27 @@ bsfa_decode_split_kernel(const DecodeParams p) {
   const int kv_len = p.kv_lens ? min(max(p.kv_lens[b], 0), p.S_kv) : p.S_kv;
   const int nb_valid = (kv_len + BS - 1) / BS;
 
-  // Mask bits of key block t for the group's heads: eight heads' bytes in flight at a time
-  // (heads past G read head G-1 again and are dropped).
+  // Mask bits of key block t for the group's heads: the bytes of one, four or eight heads in
+  // flight at a time (heads past G read head G-1 again and are dropped).
   const uint8_t* mbase = p.mask + b * p.sm[0] + (int64_t)h0 * p.sm[1];
-  auto head_bits = [&](int t) -> uint32_t {
+  auto bytes_at = [&](int t, auto n) -> uint32_t {
+    constexpr int N = decltype(n)::value;
     const uint8_t* m = mbase + (int64_t)(t >> p.mshift) * p.sm[2];
     uint32_t bitsv = 0;
-    for (int g0 = 0; g0 < G; g0 += 8) {
-      uint8_t by[8];
+    for (int g0 = 0; g0 < G; g0 += N) {
+      uint8_t by[N];
 #pragma unroll
-      for (int i = 0; i < 8; ++i) by[i] = m[(int64_t)min(g0 + i, G - 1) * p.sm[1]];
+      for (int i = 0; i < N; ++i) by[i] = m[(int64_t)min(g0 + i, G - 1) * p.sm[1]];
 #pragma unroll
-      for (int i = 0; i < 8; ++i)
+      for (int i = 0; i < N; ++i)
         if (by[i] != 0 && g0 + i < G) bitsv |= 1u << (g0 + i);
     }
     return bitsv;
+  };
+  auto head_bits = [&](int t) -> uint32_t {
+    if (G == 1) return bytes_at(t, std::integral_constant<int, 1>{});
+    if (G <= 4) return bytes_at(t, std::integral_constant<int, 4>{});
+    return bytes_at(t, std::integral_constant<int, 8>{});
   };
   // Q^T as the B operand: lane (hc, g4) holds head h0+hc, head dims 32 ks + 8 g4 .. +7.
   u32x4_t qf[KS];
