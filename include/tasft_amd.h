@@ -317,6 +317,22 @@ int tasft_gate_decode_rows_fwd(const void* q_new, const void* k_new, const int64
                                void* stream);
 
 /*
+ * The state tasft_gate_decode_rows_fwd starts from, after a prompt of seq_len tokens: uk
+ * [B, Hkv, capacity, hidden] receives the prompt's key units (key_units [B, Hkv,
+ * ceil(seq_len/block_size), hidden], the second half of tasft_gate_fwd's workspace) and zeros
+ * behind them, q_sum [B, Hq, D] and k_sum [B, Hkv, D] the sums of the tokens from
+ * seq_len / block_size * block_size on, wq_t and wk_t [D, hidden] the halves of w_in
+ * [hidden, 2 D] transposed and divided by block_size. q and k as in tasft_gate_fwd (any token
+ * strides, D contiguous). No reference counterpart.
+ */
+int tasft_gate_decode_state(const void* q, const void* k, const int64_t* q_strides,
+                            const int64_t* k_strides, const float* key_units, const float* w_in,
+                            float* uk, float* q_sum, float* k_sum, float* wq_t, float* wk_t,
+                            int64_t batch, int64_t num_q_heads, int64_t num_kv_heads,
+                            int64_t seq_len, int64_t head_dim, int64_t block_size, int64_t hidden,
+                            int64_t capacity, int dtype, void* stream);
+
+/*
  * Backward of the gate's pairwise MLP, for gate training: the gradient the reference gets
  * from autograd through AttnGate.forward (tasft/modules/attn_gate.py:248-273), without the
  * [B, H, NB, NB, hidden] activations.

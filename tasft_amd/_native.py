@@ -34,6 +34,7 @@ EXPORTED_SYMBOLS = (
     "tasft_gate_debug_wait_fault",
     "tasft_gate_rows_fwd",
     "tasft_gate_decode_rows_fwd",
+    "tasft_gate_decode_state",
     "tasft_gate_bwd_workspace_bytes",
     "tasft_gate_bwd",
     "tasft_gate_grads_workspace_bytes",
@@ -103,6 +104,11 @@ _SIGNATURES: dict[str, tuple[object, list[object]]] = {
         _I,
         [_P, _P, _I64P, _I64P, _P, _P, _P, _I64, _P, _P, _P, _P, _P, _P, _P, _P, _I64, _I64,
          _I64, _I64, _I64, _I64, _I, _I, _I, _P],
+    ),
+    "tasft_gate_decode_state": (
+        _I,
+        [_P, _P, _I64P, _I64P, _P, _P, _P, _P, _P, _P, _P, _I64, _I64, _I64, _I64, _I64, _I64,
+         _I64, _I64, _I, _P],
     ),
     "tasft_gate_bwd_workspace_bytes": (_SZ, [_I64, _I64, _I64, _I64, _I64]),
     "tasft_gate_bwd": (

@@ -811,7 +811,7 @@ gate_sync_reset_kernel(unsigned int* done, int n, unsigned long long* counter) {
 // folded in, so a zero-padded block mean is sum x W), stores the key unit of the
 // current block `row` among the kept units, and evaluates the rows of the G heads against
 // key blocks 0 .. row: logit = w_out . relu(u + v_j), sigmoid, per-head tau, the forced
-// diagonal. Thread j takes key block j (and j + 256, ...), all G heads at once.
+// diagonal.
 constexpr int kRowMaxG = 8;
 constexpr int kRowMaxHid = 256;
 
@@ -834,31 +834,75 @@ struct GateDecodeRowParams {
   int B, Hq, Hkv, G, D, hidden, row, reset, force_diag;
 };
 
+// One workgroup of 1024 threads per (b, KV head). A step is one short dependent chain (sums,
+// projections, rows), so what counts is its latency: every weight and every kept key unit of
+// the first 128 key blocks is requested before the sums are formed, and each reduction is
+// split so that a thread has one batch of loads. Thread (c, part) projects unit c over its
+// share of the head dims, the shares meet in LDS; then eight neighbouring lanes share a key
+// block, four units at a time each. B=2, 32/8 heads, D=128, hidden 128, 32 key blocks:
+// 7.7 us (13.4 with 256 threads, two per unit and one per key block).
 // MG: the query heads per KV head rounded up to 1, 2, 4 or 8; heads G .. MG - 1 are zero and
 // never stored, so the loops carry no per-head branch.
+constexpr int kRowThreads = 1024;
+constexpr int kRowBatch = 16;  // head dims loaded ahead
+constexpr int kRowKeys = kRowThreads / 8;
+
 template <int DT, int MG>
-__global__ void __launch_bounds__(256)
+__global__ void __launch_bounds__(kRowThreads)
 gate_decode_row_kernel(const GateDecodeRowParams p) {
   __shared__ float ks[kGateMaxD];
   __shared__ float qs[MG][kGateMaxD];
+  __shared__ float part[MG + 1][kRowThreads];
   __shared__ __attribute__((aligned(16))) float u[MG][kRowMaxHid];
   __shared__ __attribute__((aligned(16))) float vrow[kRowMaxHid];
-  __shared__ float wo[kRowMaxHid];
-  __shared__ unsigned int wave_count[4];
+  __shared__ __attribute__((aligned(16))) float wo[kRowMaxHid];
+  __shared__ unsigned int wave_count[kRowThreads / kWave];
 
   const int tid = threadIdx.x;
   const int wave = tid / kWave, lane = tid % kWave;
   const int b = blockIdx.x / p.Hkv, kvh = blockIdx.x % p.Hkv;
   const int h0 = kvh * p.G;
   const int D = p.D, hid = p.hidden;
-  for (int d = tid; d < D; d += 256) {
+  const int nbk = p.row + 1;
+  float* ukb = p.uk + ((int64_t)b * p.Hkv + kvh) * p.uk_stride;
+
+  // Projection role: unit c, head dims d0 .. d1 - 1.
+  const int hp = hid <= 32 ? 32 : (hid <= 64 ? 64 : (hid <= 128 ? 128 : 256));
+  const int nparts = kRowThreads / hp;
+  const int c = tid & (hp - 1), dp = tid / hp;
+  const int d0 = dp * D / nparts, d1 = (dp + 1) * D / nparts;
+  const int cc = min(c, hid - 1);
+  float wk[kRowBatch], wq[kRowBatch];
+  auto load_w = [&](int d) {
+#pragma unroll
+    for (int i = 0; i < kRowBatch; ++i) {
+      const int64_t o = (int64_t)min(d + i, D - 1) * hid + cc;
+      wk[i] = p.wk_t[o];
+      wq[i] = p.wq_t[o];
+    }
+  };
+  // Row role: key block j0 + tid / 8, units 4 (tid % 8 + 8 i) .. +3.
+  constexpr int kPre = 4;  // 16-byte loads held across the projections
+  const int kj = tid >> 3, p8 = tid & 7;
+  f32x4_t kv[kPre];
+  auto load_kv = [&](int j, int i0) {
+#pragma unroll
+    for (int i = 0; i < kPre; ++i) {
+      const int c4 = 4 * (p8 + 8 * (i0 + i));
+      kv[i] = (j < p.row && c4 < hid) ? *(const f32x4_t*)(ukb + (int64_t)j * hid + c4) : (f32x4_t){};
+    }
+  };
+  load_w(d0);
+  load_kv(kj, 0);
+
+  for (int d = tid; d < D; d += kRowThreads) {
     const float kn = bits16_to_f32<DT>(p.k_new[b * p.sk[0] + kvh * p.sk[1] + d]);
     float* ksp = p.k_sum + ((int64_t)b * p.Hkv + kvh) * D + d;
     const float v = (p.reset ? 0.f : *ksp) + kn;
     *ksp = v;
     ks[d] = v;
   }
-  for (int e = tid; e < MG * D; e += 256) {
+  for (int e = tid; e < MG * D; e += kRowThreads) {
     const int g = e / D, d = e % D, h = h0 + g;
     if (g >= p.G) {
       qs[g][d] = 0.f;
@@ -870,80 +914,74 @@ gate_decode_row_kernel(const GateDecodeRowParams p) {
     *qsp = v;
     qs[g][d] = v;
   }
-  for (int c = tid; c < hid; c += 256) wo[c] = p.w_out[c];
+  for (int e = tid; e < hid; e += kRowThreads) wo[e] = p.w_out[e];
   __syncthreads();
-  float* ukb = p.uk + ((int64_t)b * p.Hkv + kvh) * p.uk_stride;
   {
-    // Projections. Up to 128 hidden units, two threads per unit, each over half of d
-    // (partial sums meet in LDS); above that one thread per unit. The loads of eight d run
-    // ahead of their FMAs.
-    const int per = hid <= 128 ? 128 : 256;
-    const int nsp = 256 / per;
-    const int c = tid % per, sp = tid / per;
-    const int d0 = sp * D / nsp, d1 = (sp + 1) * D / nsp;
-    float vk = 0.f;
-    float acc[MG];
+    float acc[MG + 1];
 #pragma unroll
-    for (int g = 0; g < MG; ++g) acc[g] = 0.f;
-    if (c < hid) {
-#pragma unroll 8
-      for (int d = d0; d < d1; ++d) {
-        const float wk = p.wk_t[(int64_t)d * hid + c];
-        const float wq = p.wq_t[(int64_t)d * hid + c];
-        vk = fmaf(ks[d], wk, vk);
+    for (int m = 0; m <= MG; ++m) acc[m] = 0.f;
+    for (int d = d0; d < d1; d += kRowBatch) {
+      if (d > d0) load_w(d);
 #pragma unroll
-        for (int g = 0; g < MG; ++g)
-          acc[g] = fmaf(qs[g][d], wq, acc[g]);
+      for (int i = 0; i < kRowBatch; ++i) {
+        if (d + i >= d1) break;
+        acc[MG] = fmaf(ks[d + i], wk[i], acc[MG]);
+#pragma unroll
+        for (int g = 0; g < MG; ++g) acc[g] = fmaf(qs[g][d + i], wq[i], acc[g]);
       }
     }
-    if (nsp == 2 && sp == 1 && c < hid) {
-      vrow[c] = vk;
 #pragma unroll
-      for (int g = 0; g < MG; ++g)
-        u[g][c] = acc[g];
-    }
-    __syncthreads();
-    if (sp == 0 && c < hid) {
-      if (nsp == 2) {
-        vk += vrow[c];
-#pragma unroll
-        for (int g = 0; g < MG; ++g)
-          acc[g] += u[g][c];
-      }
-      vrow[c] = vk;
-      ukb[(int64_t)p.row * hid + c] = vk;
-      const float bias = p.b_in[c];
-#pragma unroll
-      for (int g = 0; g < MG; ++g)
-        u[g][c] = acc[g] + bias;
+    for (int m = 0; m <= MG; ++m) part[m][tid] = acc[m];
+  }
+  __syncthreads();
+  for (int e = tid; e < (MG + 1) * hid; e += kRowThreads) {
+    const int m = e / hid, x = e % hid;
+    float v = 0.f;
+    for (int s = 0; s < nparts; ++s) v += part[m][s * hp + x];
+    if (m == MG) {
+      vrow[x] = v;
+      ukb[(int64_t)p.row * hid + x] = v;
+    } else {
+      u[m][x] = v + p.b_in[x];
     }
   }
   __syncthreads();
-  const int nbk = p.row + 1;
   unsigned int active = 0;
-  for (int j = tid; j < nbk; j += 256) {
+  for (int j0 = 0; j0 < nbk; j0 += kRowKeys) {
+    const int j = j0 + kj;
     float acc[MG];
 #pragma unroll
     for (int g = 0; g < MG; ++g) acc[g] = 0.f;
-    // Block `row` was stored above by this workgroup (visible after the barrier), so every
-    // key block is read from the kept units with plain global loads.
-    const float* vj = ukb + (int64_t)j * hid;
-#pragma unroll 8
-    for (int c = 0; c < hid; c += 4) {
-      const f32x4_t v4 = *(const f32x4_t*)(vj + c);
+    for (int i0 = 0; 32 * i0 < hid; i0 += kPre) {
+      if (j0 > 0 || i0 > 0) load_kv(j, i0);
 #pragma unroll
-      for (int e = 0; e < 4; ++e) {
-        const float w = wo[c + e];
+      for (int i = 0; i < kPre; ++i) {
+        const int c4 = 4 * (p8 + 8 * (i0 + i));
+        if (c4 >= hid) break;
+        // The current block's unit is this call's own.
+        const f32x4_t v4 = j == p.row ? *(const f32x4_t*)&vrow[c4] : kv[i];
+        const f32x4_t w4 = *(const f32x4_t*)&wo[c4];
 #pragma unroll
-        for (int g = 0; g < MG; ++g)
-          acc[g] = fmaf(w, fmaxf(u[g][c + e] + v4[e], 0.f), acc[g]);
+        for (int g = 0; g < MG; ++g) {
+          const f32x4_t u4 = *(const f32x4_t*)&u[g][c4];
+#pragma unroll
+          for (int e = 0; e < 4; ++e) acc[g] = fmaf(w4[e], fmaxf(u4[e] + v4[e], 0.f), acc[g]);
+        }
       }
     }
 #pragma unroll
     for (int g = 0; g < MG; ++g) {
-      if (g >= p.G) break;
-      const int h = h0 + g;
-      const float sv = 1.f / (1.f + expf(-acc[g]));
+      acc[g] += __shfl_xor(acc[g], 1, kWave);
+      acc[g] += __shfl_xor(acc[g], 2, kWave);
+      acc[g] += __shfl_xor(acc[g], 4, kWave);
+    }
+    // Lane p8 of the eight writes head p8.
+    float logit = acc[0];
+#pragma unroll
+    for (int g = 1; g < MG; ++g) logit = p8 == g ? acc[g] : logit;
+    if (p8 < p.G && j < nbk) {
+      const int h = h0 + p8;
+      const float sv = 1.f / (1.f + expf(-logit));
       const bool on = sv >= p.tau[h] || (p.force_diag && j == p.row);
       const int64_t o = ((int64_t)b * p.Hq + h) * nbk + j;
       p.soft[o] = sv;
@@ -951,12 +989,83 @@ gate_decode_row_kernel(const GateDecodeRowParams p) {
       active += on ? 1u : 0u;
     }
   }
+  if (!p.counter) return;
   const float tot = wave_sum((float)active);
   if (lane == 0) wave_count[wave] = (unsigned int)(tot + 0.5f);
   __syncthreads();
   if (tid == 0) {
-    const unsigned int t = (wave_count[0] + wave_count[1]) + (wave_count[2] + wave_count[3]);
-    if (t && p.counter) atomicAdd(p.counter, (unsigned long long)t);
+    unsigned int t = 0;
+    for (int w = 0; w < kRowThreads / kWave; ++w) t += wave_count[w];
+    if (t) atomicAdd(p.counter, (unsigned long long)t);
+  }
+}
+
+// The state a cached decode starts from, after a prompt of S tokens, in one launch (what took
+// about twenty small torch kernels): the prompt's key units at the front of the kept ones and
+// zeros behind them, the sums of the queries and keys of the block the next token falls in,
+// and the two halves of W_in transposed and divided by the block size. The first `sum_wgs`
+// workgroups form the sums, a thread per (head, dim); the others copy.
+struct DecodeStateParams {
+  const uint16_t* q;
+  const uint16_t* k;
+  int64_t sq[3], sk[3];
+  const float* units;  // [B, Hkv, nb, hidden]
+  const float* w_in;   // [hidden, 2 D]
+  float* uk;           // [B, Hkv, cap, hidden]
+  float* q_sum;        // [B, Hq, D]
+  float* k_sum;        // [B, Hkv, D]
+  float* wq_t;         // [D, hidden]
+  float* wk_t;         // [D, hidden]
+  int64_t n_units;     // elements of uk
+  int B, Hq, Hkv, D, nb, cap, hidden, row0, S, sum_wgs;
+  float block;
+};
+
+template <int DT>
+__global__ void __launch_bounds__(256)
+gate_decode_state_kernel(const DecodeStateParams p) {
+  if ((int)blockIdx.x < p.sum_wgs) {
+    const int64_t e = (int64_t)blockIdx.x * 256 + threadIdx.x;
+    const int64_t nq = (int64_t)p.B * p.Hq * p.D;
+    if (e >= nq + (int64_t)p.B * p.Hkv * p.D) return;
+    const bool is_q = e < nq;
+    const int64_t r = is_q ? e : e - nq;
+    const int heads = is_q ? p.Hq : p.Hkv;
+    const int d = (int)(r % p.D);
+    const int64_t bh = r / p.D;
+    const int64_t b = bh / heads, h = bh % heads;
+    const int64_t stride = is_q ? p.sq[2] : p.sk[2];
+    const uint16_t* src = (is_q ? p.q + b * p.sq[0] + h * p.sq[1] : p.k + b * p.sk[0] + h * p.sk[1]) + d;
+    // Sixteen rows in flight at a time, added pairwise.
+    float acc = 0.f;
+    for (int t = p.row0; t < p.S; t += 16) {
+      float x[16];
+#pragma unroll
+      for (int i = 0; i < 16; ++i)
+        x[i] = t + i < p.S ? bits16_to_f32<DT>(src[(int64_t)(t + i) * stride]) : 0.f;
+#pragma unroll
+      for (int w = 8; w >= 1; w >>= 1)
+#pragma unroll
+        for (int i = 0; i < w; ++i) x[i] += x[i + w];
+      acc += x[0];
+    }
+    (is_q ? p.q_sum : p.k_sum)[r] = acc;
+    return;
+  }
+  const int64_t step = (int64_t)(gridDim.x - p.sum_wgs) * 256;
+  const int64_t n_w = (int64_t)p.hidden * 2 * p.D;
+  for (int64_t e = ((int64_t)blockIdx.x - p.sum_wgs) * 256 + threadIdx.x; e < p.n_units + n_w; e += step) {
+    if (e < p.n_units) {
+      const int c = (int)(e % p.hidden);
+      const int64_t r = e / p.hidden;
+      const int j = (int)(r % p.cap);
+      p.uk[e] = j < p.nb ? p.units[((r / p.cap) * p.nb + j) * p.hidden + c] : 0.f;
+    } else {
+      const int64_t w = e - p.n_units;
+      const int c = (int)(w % p.hidden), x = (int)(w / p.hidden);
+      (x < p.D ? p.wq_t : p.wk_t - (int64_t)p.D * p.hidden)[(int64_t)x * p.hidden + c] =
+          p.w_in[(int64_t)c * 2 * p.D + x] / p.block;
+    }
   }
 }
 
@@ -1529,9 +1638,9 @@ extern "C" int tasft_gate_decode_rows_fwd(
   auto launch = [&](auto mg) {
     constexpr int MG = decltype(mg)::value;
     if (dtype == kF16)
-      hipLaunchKernelGGL((gate_decode_row_kernel<kF16, MG>), grid, dim3(256), 0, s, rp);
+      hipLaunchKernelGGL((gate_decode_row_kernel<kF16, MG>), grid, dim3(kRowThreads), 0, s, rp);
     else
-      hipLaunchKernelGGL((gate_decode_row_kernel<kBf16, MG>), grid, dim3(256), 0, s, rp);
+      hipLaunchKernelGGL((gate_decode_row_kernel<kBf16, MG>), grid, dim3(kRowThreads), 0, s, rp);
   };
   if (G == 1)
     launch(std::integral_constant<int, 1>());
@@ -1544,5 +1653,71 @@ extern "C" int tasft_gate_decode_rows_fwd(
   const hipError_t err = hipGetLastError();
   if (err != hipSuccess)
     return set_error(kErrLaunch, "gate_decode_rows: launch failed: %s", hipGetErrorString(err));
+  return kOk;
+}
+
+extern "C" int tasft_gate_decode_state(const void* q, const void* k, const int64_t* q_strides,
+                                       const int64_t* k_strides, const float* key_units,
+                                       const float* w_in, float* uk, float* q_sum, float* k_sum,
+                                       float* wq_t, float* wk_t, int64_t batch,
+                                       int64_t num_q_heads, int64_t num_kv_heads, int64_t seq_len,
+                                       int64_t head_dim, int64_t block_size, int64_t hidden,
+                                       int64_t capacity, int dtype, void* stream) {
+  if (!q || !k || !q_strides || !k_strides || !key_units || !w_in || !uk || !q_sum || !k_sum ||
+      !wq_t || !wk_t)
+    return set_error(kErrInvalidArgument, "gate_decode_state: null pointer argument");
+  if (dtype != kBf16 && dtype != kF16)
+    return set_error(kErrUnsupported, "gate_decode_state: dtype must be bf16 (0) or fp16 (1), got %d",
+                     dtype);
+  if (batch <= 0 || num_q_heads <= 0 || num_kv_heads <= 0 || seq_len <= 0 || head_dim <= 0 ||
+      block_size <= 0 || hidden <= 0)
+    return set_error(kErrInvalidArgument, "gate_decode_state: sizes must be positive");
+  if (!strides_nonneg(q_strides, 4) || !strides_nonneg(k_strides, 4))
+    return set_error(kErrInvalidArgument, "gate_decode_state: strides must be non-negative");
+  if (q_strides[3] != 1 || k_strides[3] != 1)
+    return set_error(kErrInvalidArgument, "gate_decode_state: head_dim must be the contiguous dimension");
+  const int64_t nb = (seq_len + block_size - 1) / block_size;
+  if (capacity < nb)
+    return set_error(kErrInvalidArgument, "gate_decode_state: capacity of %lld blocks for a prompt of %lld",
+                     (long long)capacity, (long long)nb);
+  const int64_t n_sum = batch * (num_q_heads + num_kv_heads) * head_dim;
+  if (n_sum > 0x7fffffffLL * 128 || seq_len > 0x3fffffffLL || capacity > 0x3fffffffLL)
+    return set_error(kErrUnsupported, "gate_decode_state: problem too large for one launch");
+  DecodeStateParams p;
+  p.q = (const uint16_t*)q;
+  p.k = (const uint16_t*)k;
+  for (int j = 0; j < 3; ++j) {
+    p.sq[j] = q_strides[j];
+    p.sk[j] = k_strides[j];
+  }
+  p.units = key_units;
+  p.w_in = w_in;
+  p.uk = uk;
+  p.q_sum = q_sum;
+  p.k_sum = k_sum;
+  p.wq_t = wq_t;
+  p.wk_t = wk_t;
+  p.n_units = batch * num_kv_heads * capacity * hidden;
+  p.B = (int)batch;
+  p.Hq = (int)num_q_heads;
+  p.Hkv = (int)num_kv_heads;
+  p.D = (int)head_dim;
+  p.nb = (int)nb;
+  p.cap = (int)capacity;
+  p.hidden = (int)hidden;
+  p.row0 = (int)(seq_len / block_size * block_size);
+  p.S = (int)seq_len;
+  p.sum_wgs = (int)((n_sum + 255) / 256);
+  p.block = (float)block_size;
+  const int64_t copy = p.n_units + hidden * 2 * head_dim;
+  const int64_t copy_wgs = std::min<int64_t>((copy + 255) / 256, 2048);
+  const dim3 grid((unsigned)(p.sum_wgs + copy_wgs));
+  if (dtype == kF16)
+    hipLaunchKernelGGL(gate_decode_state_kernel<kF16>, grid, dim3(256), 0, (hipStream_t)stream, p);
+  else
+    hipLaunchKernelGGL(gate_decode_state_kernel<kBf16>, grid, dim3(256), 0, (hipStream_t)stream, p);
+  const hipError_t err = hipGetLastError();
+  if (err != hipSuccess)
+    return set_error(kErrLaunch, "gate_decode_state: launch failed: %s", hipGetErrorString(err));
   return kOk;
 }

@@ -87,23 +87,26 @@ class SparseAttentionDecoder:
         hid = self.gate.gate_hidden_dim
         nb = r["nb"]
         cap = math.ceil(self.max_len / bs)
-        self._vk = torch.zeros((B, Hkv, cap, hid), dtype=torch.float32, device=q.device)
-        uq_bytes = B * Hq * nb * hid * 4
-        uk = r["workspace"][uq_bytes:uq_bytes + B * Hkv * nb * hid * 4].view(torch.float32)
-        self._vk[:, :, :nb] = uk.view(B, Hkv, nb, hid)
-        last0 = (S // bs) * bs  # first token of the block the next token falls in
-        if last0 < S:
-            self._ksum = k[:, :, last0:S].float().sum(2)
-            self._qsum = q[:, :, last0:S].float().sum(2)
-        else:
-            self._ksum = torch.zeros((B, Hkv, D), dtype=torch.float32, device=q.device)
-            self._qsum = torch.zeros((B, Hq, D), dtype=torch.float32, device=q.device)
+        # The decode state: kept key units, the current block's sums, and the per-step constants
+        # read from the gate once (the W_in halves with the 1/block of the zero-padded mean
+        # folded in, the bias, w_out, the thresholds and the flags).
+        dev = q.device
+        self._vk = torch.empty((B, Hkv, cap, hid), dtype=torch.float32, device=dev)
+        self._ksum = torch.empty((B, Hkv, D), dtype=torch.float32, device=dev)
+        self._qsum = torch.empty((B, Hq, D), dtype=torch.float32, device=dev)
+        self._wk_t = torch.empty((D, hid), dtype=torch.float32, device=dev)
+        self._wq_t = torch.empty((D, hid), dtype=torch.float32, device=dev)
+        qc = q if q.stride(-1) == 1 else q.contiguous()
+        kc = k if k.stride(-1) == 1 else k.contiguous()
+        lib = _native.load_library()
+        status = lib.tasft_gate_decode_state(
+            qc.data_ptr(), kc.data_ptr(), self._strides(qc), self._strides(kc),
+            r["workspace"].data_ptr() + B * Hq * nb * hid * 4, r["w_in"].data_ptr(),
+            self._vk.data_ptr(), self._qsum.data_ptr(), self._ksum.data_ptr(), self._wq_t.data_ptr(),
+            self._wk_t.data_ptr(), B, Hq, Hkv, S, D, bs, hid, cap,
+            _native.dtype_code(q.dtype, "decode state"), _native.stream_handle(dev))
+        _native.check(status, "tasft_gate_decode_state", {"shape": [B, Hq, S, D]})
         self.length = S
-        # Per-step constants, read from the gate once: the W_in halves with the 1/block of
-        # the zero-padded mean folded in, the bias, w_out, the thresholds and the flags.
-        w_in = self.gate.gate_proj_in.weight.detach().float()
-        self._wk_t = (w_in[:, D:] / bs).t().contiguous()
-        self._wq_t = (w_in[:, :D] / bs).t().contiguous()
         self._b_in = self.gate.gate_proj_in.bias.detach().float().contiguous()
         self._w_out = self.gate.gate_proj_out.weight.detach().float().reshape(-1).contiguous()
         self._taus = taus
