@@ -7,6 +7,7 @@ to load, every kernel entry point raises ``KernelError``.
 from __future__ import annotations
 
 import ctypes
+import functools
 import threading
 from pathlib import Path
 
@@ -173,14 +174,16 @@ def is_available() -> bool:
     return True
 
 
+@functools.lru_cache(maxsize=4096)
+def strides_array(values: tuple[int, ...]) -> ctypes.Array:
+    """Element strides as a C int64 array. Arrays are kept by their values (the library only
+    reads them): building the five of a call took as long as the call."""
+    return (ctypes.c_int64 * len(values))(*values)
+
+
 def strides(t: torch.Tensor) -> ctypes.Array:
     """Element strides of a tensor as a C int64 array."""
-    return (ctypes.c_int64 * t.dim())(*t.stride())
-
-
-def strides_array(values) -> ctypes.Array:
-    """A list of element strides as a C int64 array."""
-    return (ctypes.c_int64 * len(values))(*values)
+    return strides_array(t.stride())
 
 
 # Element types of the 16-bit tensors (TASFT_DTYPE_BF16 / TASFT_DTYPE_F16).
@@ -204,9 +207,27 @@ def ptr(t: torch.Tensor | None) -> int | None:
     return None if t is None else t.data_ptr()
 
 
+# hipStream_t of a device's current stream without building a torch Stream object.
+_raw_stream = getattr(torch._C, "_cuda_getCurrentRawStream", None)
+
+
 def stream_handle(device: torch.device) -> int:
     """hipStream_t of torch's current stream on ``device``."""
+    if _raw_stream is not None and device.index is not None:
+        return _raw_stream(device.index)
     return torch.cuda.current_stream(device).cuda_stream
+
+
+def kernel_layout(t: torch.Tensor, align: bool = True) -> bool:
+    """True if the kernels read ``t`` in place: unit stride on the last dim, the others
+    multiples of 8 elements and (with ``align``) a 16-byte aligned base."""
+    st = t.stride()
+    if st[-1] != 1:
+        return False
+    low = 0
+    for s in st[:-1]:
+        low |= s
+    return low & 7 == 0 and not (align and t.data_ptr() & 15)
 
 
 def check(status: int, what: str, context: dict[str, object] | None = None) -> None:
@@ -217,5 +238,5 @@ def check(status: int, what: str, context: dict[str, object] | None = None) -> N
 
 
 __all__ = ["DTYPE_BF16", "DTYPE_F16", "EXPORTED_SYMBOLS", "KERNEL_DTYPES", "LIB_PATH", "check",
-           "dtype_code", "is_available", "load_library", "ptr", "stream_handle", "strides",
+           "dtype_code", "is_available", "kernel_layout", "load_library", "ptr", "stream_handle", "strides",
            "strides_array"]

@@ -55,18 +55,8 @@ class SparseAttentionDecoder:
         self._vk = None
         self._ksum = None
         self._qsum = None
-        self._ws: dict[int, tuple[torch.Tensor, int]] = {}  # decode workspace per split count
-        # ctypes stride arrays per stride tuple: a step's tensors keep their strides, and
-        # building the arrays was a measurable share of a step's host time.
-        self._stride_arrays: dict[tuple[int, ...], object] = {}
-
-    def _strides(self, t: torch.Tensor):
-        st = t.stride()
-        arr = self._stride_arrays.get(st)
-        if arr is None:
-            arr = _native.strides_array(st)
-            self._stride_arrays[st] = arr
-        return arr
+        # Decode workspaces by (batch, query heads, head dim, splits), of the last prompt.
+        self._ws: dict[tuple[int, ...], tuple[torch.Tensor, int]] = {}
 
     # ------------------------------------------------------------------ prefill
     @torch.no_grad()
@@ -81,7 +71,7 @@ class SparseAttentionDecoder:
                               context={"seq_len": S, "max_len": self.max_len})
         taus = self.gate._thresholds(self.threshold, q.device)
         r = _launch_gate(self.gate, q, k, taus, False, self.force_diagonal, keep=False)
-        g = GateOutput(soft_scores=r["soft"], hard_mask=r["mask"].view(torch.bool), num_blocks_q=r["nb"],
+        g = GateOutput(soft_scores=r["soft"], hard_mask=r["mask"], num_blocks_q=r["nb"],
                        num_blocks_k=r["nb"], active_count=r["active"])
         out = self.bsfa.forward(q, k, v, g.hard_mask, causal=self.gate.is_causal)
         hid = self.gate.gate_hidden_dim
@@ -100,13 +90,14 @@ class SparseAttentionDecoder:
         kc = k if k.stride(-1) == 1 else k.contiguous()
         lib = _native.load_library()
         status = lib.tasft_gate_decode_state(
-            qc.data_ptr(), kc.data_ptr(), self._strides(qc), self._strides(kc),
+            qc.data_ptr(), kc.data_ptr(), _native.strides(qc), _native.strides(kc),
             r["workspace"].data_ptr() + B * Hq * nb * hid * 4, r["w_in"].data_ptr(),
             self._vk.data_ptr(), self._qsum.data_ptr(), self._ksum.data_ptr(), self._wq_t.data_ptr(),
             self._wk_t.data_ptr(), B, Hq, Hkv, S, D, bs, hid, cap,
             _native.dtype_code(q.dtype, "decode state"), _native.stream_handle(dev))
         _native.check(status, "tasft_gate_decode_state", {"shape": [B, Hq, S, D]})
         self.length = S
+        self._ws = {}
         self._b_in = self.gate.gate_proj_in.bias.detach().float().contiguous()
         self._w_out = self.gate.gate_proj_out.weight.detach().float().reshape(-1).contiguous()
         self._taus = taus
@@ -114,14 +105,17 @@ class SparseAttentionDecoder:
         return out, g
 
     # ------------------------------------------------------------------ decode
-    @torch.no_grad()
     def select(self, q_new: torch.Tensor, k_new: torch.Tensor) -> GateOutput:
         """Advance the state by one token and return its gate row ``[B, Hq, 1, NB]``
         (``NB = ceil((t + 1) / block)`` for the new position ``t``)."""
+        return self._select(q_new, k_new, 0)
+
+    def _select(self, q_new: torch.Tensor, k: torch.Tensor, at: int) -> GateOutput:
+        """``select`` with the new token's keys at position ``at`` of ``k [B, Hkv, ., D]``."""
         if self._vk is None:
             raise KernelError("SparseAttentionDecoder.select before prefill", context={})
         B, Hq, _, D = q_new.shape
-        Hkv = k_new.shape[1]
+        Hkv = k.shape[1]
         bs = self.gate.block_size
         t = self.length
         if t >= self.max_len:
@@ -131,19 +125,21 @@ class SparseAttentionDecoder:
         nbk = i + 1
         dev = q_new.device
         soft = torch.empty((B, Hq, 1, nbk), dtype=torch.float32, device=dev)
-        mask = torch.empty((B, Hq, 1, nbk), dtype=torch.uint8, device=dev)
+        mask = torch.empty((B, Hq, 1, nbk), dtype=torch.bool, device=dev)
         active = None
         lib = _native.load_library()
+        q_st, k_st = q_new.stride(), k.stride()
         if (Hq // Hkv <= 8 and D <= 256 and hid <= 256 and hid % 4 == 0
-                and q_new.dtype in (torch.bfloat16, torch.float16) and k_new.dtype == q_new.dtype
-                and q_new.stride(-1) == 1 and k_new.stride(-1) == 1):
+                and q_new.dtype in _native.KERNEL_DTYPES and k.dtype == q_new.dtype
+                and q_st[-1] == 1 and k_st[-1] == 1):
             # One launch per (b, KV head): block sums, both projections, the kept key unit of
             # block i and the rows (tasft_gate_decode_rows_fwd).
             status = lib.tasft_gate_decode_rows_fwd(
-                q_new.data_ptr(), k_new.data_ptr(), self._strides(q_new), self._strides(k_new),
-                self._qsum.data_ptr(), self._ksum.data_ptr(), self._vk.data_ptr(),
-                self._vk.shape[2] * hid, self._wq_t.data_ptr(), self._wk_t.data_ptr(),
-                self._b_in.data_ptr(), self._w_out.data_ptr(), self._taus.data_ptr(),
+                q_new.data_ptr(), k.data_ptr() + 2 * at * k_st[2], _native.strides_array(q_st),
+                _native.strides_array(k_st), self._qsum.data_ptr(), self._ksum.data_ptr(),
+                self._vk.data_ptr(), self._vk.shape[2] * hid, self._wq_t.data_ptr(),
+                self._wk_t.data_ptr(), self._b_in.data_ptr(), self._w_out.data_ptr(),
+                self._taus.data_ptr(),
                 # No device count: the row's sparsity is counted from the mask if asked for.
                 soft.data_ptr(), mask.data_ptr(), None, B, Hq, Hkv, D, hid, i,
                 1 if t % bs == 0 else 0, self._flags, _native.dtype_code(q_new.dtype, "decode rows"),
@@ -151,23 +147,23 @@ class SparseAttentionDecoder:
             _native.check(status, "tasft_gate_decode_rows_fwd", {"position": t})
         else:
             active = torch.empty((1,), dtype=torch.int64, device=dev)
-            if t % bs == 0:
-                self._ksum.zero_()
-                self._qsum.zero_()
-            self._ksum.add_(k_new[:, :, 0])
-            self._qsum.add_(q_new[:, :, 0])
-            self._vk[:, :, i] = torch.matmul(self._ksum, self._wk_t)
-            uq = torch.addmm(self._b_in, self._qsum.view(B * Hq, D), self._wq_t).view(B, Hq, 1, hid)
+            with torch.no_grad():
+                if t % bs == 0:
+                    self._ksum.zero_()
+                    self._qsum.zero_()
+                self._ksum.add_(k[:, :, at])
+                self._qsum.add_(q_new[:, :, 0])
+                self._vk[:, :, i] = torch.matmul(self._ksum, self._wk_t)
+                uq = torch.addmm(self._b_in, self._qsum.view(B * Hq, D), self._wq_t).view(B, Hq, 1, hid)
             status = lib.tasft_gate_rows_fwd(
                 uq.data_ptr(), self._vk.data_ptr(), self._w_out.data_ptr(), self._taus.data_ptr(),
                 soft.data_ptr(), None, mask.data_ptr(), active.data_ptr(), B, Hq, Hkv, 1, nbk, i, hid,
                 self._vk.shape[2] * hid, self._flags, _native.stream_handle(dev))
             _native.check(status, "tasft_gate_rows_fwd", {"position": t})
         self.length = t + 1
-        return GateOutput(soft_scores=soft, hard_mask=mask.view(torch.bool), num_blocks_q=1,
+        return GateOutput(soft_scores=soft, hard_mask=mask, num_blocks_q=1,
                           num_blocks_k=nbk, active_count=active)
 
-    @torch.no_grad()
     def step(self, q_new: torch.Tensor, k_cache: torch.Tensor, v_cache: torch.Tensor
              ) -> tuple[torch.Tensor, GateOutput]:
         """One cached decode step: ``q_new [B, Hq, 1, D]``; ``k_cache``/``v_cache``
@@ -177,7 +173,7 @@ class SparseAttentionDecoder:
         if k_cache.shape[2] != t + 1:
             raise KernelError(f"KV cache holds {k_cache.shape[2]} tokens, expected {t + 1}",
                               context={"cache_len": k_cache.shape[2], "length": t})
-        row = self.select(q_new, k_cache[:, :, t:t + 1])
+        row = self._select(q_new, k_cache, t)
         return self._decode(q_new, k_cache, v_cache, row.hard_mask), row
 
     def _decode(self, q: torch.Tensor, k_cache: torch.Tensor, v_cache: torch.Tensor,
@@ -187,28 +183,28 @@ class SparseAttentionDecoder:
         the workspace kept between steps; ``forward_decode`` (validation, copies) otherwise."""
         B, Hq, _, D = q.shape
         Hkv, S_kv = k_cache.shape[1], k_cache.shape[2]
-        ready = (D in _VALID_HEAD_DIMS and q.dtype in (torch.bfloat16, torch.float16)
-                 and k_cache.dtype == q.dtype and v_cache.dtype == q.dtype and q.is_cuda
-                 and all(t.stride(-1) == 1 and all(st % 8 == 0 for st in t.stride()[:-1])
-                         and t.data_ptr() % 16 == 0 for t in (q, k_cache, v_cache)))
+        dtype = q.dtype
+        ready = (D in _VALID_HEAD_DIMS and dtype in _native.KERNEL_DTYPES and k_cache.dtype == dtype
+                 and v_cache.dtype == dtype and q.is_cuda and _native.kernel_layout(q)
+                 and _native.kernel_layout(k_cache) and _native.kernel_layout(v_cache))
         if not ready:
-            return self.bsfa.forward_decode(q, k_cache, v_cache, mask)
+            with torch.no_grad():
+                return self.bsfa.forward_decode(q, k_cache, v_cache, mask)
         lib = _native.load_library()
-        nb = mask.shape[-1]
-        splits = default_decode_splits(B, Hkv, nb, Hq // Hkv)
-        ws = self._ws.get(splits)
+        splits = default_decode_splits(B, Hkv, mask.shape[-1], Hq // Hkv)
+        key = (B, Hq, D, splits)
+        ws = self._ws.get(key)
         if ws is None:
             n = lib.tasft_bsfa_decode_workspace_bytes(B, Hq, D, splits)
             ws = (torch.empty(n, dtype=torch.uint8, device=q.device), n)
-            self._ws[splits] = ws
-        out = torch.empty((B, Hq, 1, D), dtype=q.dtype, device=q.device)
-        m8 = mask.view(torch.uint8)
+            self._ws[key] = ws
+        out = torch.empty((B, Hq, 1, D), dtype=dtype, device=q.device)
         status = lib.tasft_bsfa_decode_fwd(
-            q.data_ptr(), k_cache.data_ptr(), v_cache.data_ptr(), out.data_ptr(), m8.data_ptr(),
+            q.data_ptr(), k_cache.data_ptr(), v_cache.data_ptr(), out.data_ptr(), mask.data_ptr(),
             None, ws[0].data_ptr(), ws[1], B, Hq, Hkv, S_kv, D, self.bsfa.block_size, splits,
-            self._strides(q), self._strides(k_cache), self._strides(v_cache),
-            self._strides(out), self._strides(m8), 1.0 / math.sqrt(D),
-            _native.dtype_code(q.dtype, "decode"), _native.stream_handle(q.device))
+            _native.strides(q), _native.strides(k_cache), _native.strides(v_cache),
+            _native.strides(out), _native.strides(mask), 1.0 / math.sqrt(D),
+            _native.dtype_code(dtype, "decode"), _native.stream_handle(q.device))
         _native.check(status, "tasft_bsfa_decode_fwd", {"shape": [B, Hq, S_kv, D]})
         return out
 

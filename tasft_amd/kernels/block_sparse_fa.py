@@ -85,21 +85,19 @@ def _kv_compatible(q: torch.Tensor, kv: torch.Tensor) -> bool:
 def _kernel_dtype(**tensors: torch.Tensor) -> int:
     """The C-ABI ``dtype`` code shared by the given tensors (bf16 or fp16, all the same, as the
     reference's ``tl.dot`` needs, ``block_sparse_fa.py:228, 252``)."""
-    items = list(tensors.items())
-    first_name, first = items[0]
-    for name, t in items[1:]:
-        if t.dtype != first.dtype:
-            raise KernelError(f"{name} is {t.dtype} but {first_name} is {first.dtype}",
-                              context={"tensor": name, "dtype": str(t.dtype), "expected": str(first.dtype)})
-    return _native.dtype_code(first.dtype, "block-sparse attention")
+    first_name, first = None, None
+    for name, t in tensors.items():
+        if first is None:
+            first_name, first = name, t.dtype
+        elif t.dtype != first:
+            raise KernelError(f"{name} is {t.dtype} but {first_name} is {first}",
+                              context={"tensor": name, "dtype": str(t.dtype), "expected": str(first)})
+    return _native.dtype_code(first, "block-sparse attention")
 
 
 def _kernel_ready(t: torch.Tensor) -> torch.Tensor:
     """Return ``t`` if its layout suits the kernels (unit d stride, 16-byte rows), else a copy."""
-    st = t.stride()
-    if st[-1] == 1 and all(s % 8 == 0 for s in st[:-1]) and t.data_ptr() % 16 == 0:
-        return t
-    return t.contiguous()
+    return t if _native.kernel_layout(t) else t.contiguous()
 
 
 def _mask_bytes(mask: torch.Tensor) -> torch.Tensor:
@@ -109,6 +107,13 @@ def _mask_bytes(mask: torch.Tensor) -> torch.Tensor:
     if mask.dtype in (torch.uint8, torch.int8):
         return mask.view(torch.uint8) if mask.dtype == torch.int8 else mask
     return (mask != 0).view(torch.uint8)
+
+
+def _int32_on(t: torch.Tensor, device: torch.device) -> torch.Tensor:
+    """``t`` as a contiguous int32 tensor on ``device``, itself if it is one."""
+    if t.dtype == torch.int32 and t.device == device and t.is_contiguous():
+        return t
+    return t.to(device=device, dtype=torch.int32).contiguous()
 
 
 class BlockSparseFlashAttention:
@@ -244,15 +249,17 @@ class BlockSparseFlashAttention:
         q = _kernel_ready(q)
         k = _kernel_ready(k)
         v = _kernel_ready(v)
-        mask = _mask_bytes(block_mask.to(q.device))
+        mask = _mask_bytes(block_mask if block_mask.device == q.device else block_mask.to(q.device))
         out = torch.empty((B, H, S, D), dtype=q.dtype, device=q.device)
         scale = 1.0 / math.sqrt(D)
-        # Workspace for the persistent launch's work-queue counters.
-        ws_bytes = lib.tasft_bsfa_prefill_workspace_bytes(B, H, S, self.block_size)
-        workspace = torch.empty(ws_bytes, dtype=torch.uint8, device=q.device)
+        workspace, ws_bytes = None, 0
+        if D == 64 and self.block_size != 32:
+            # Work-queue counters of the persistent launch.
+            ws_bytes = lib.tasft_bsfa_prefill_workspace_bytes(B, H, S, self.block_size)
+            workspace = torch.empty(ws_bytes, dtype=torch.uint8, device=q.device)
         status = lib.tasft_bsfa_prefill_fwd(
             q.data_ptr(), k.data_ptr(), v.data_ptr(), out.data_ptr(), mask.data_ptr(),
-            workspace.data_ptr(), ws_bytes, B, H, k.shape[1], S, D, self.block_size,
+            _native.ptr(workspace), ws_bytes, B, H, k.shape[1], S, D, self.block_size,
             _native.strides(q), _native.strides(k), _native.strides(v), _native.strides(out),
             _native.strides(mask), scale, 1 if causal else 0, dtype, _native.stream_handle(q.device),
         )
@@ -366,8 +373,8 @@ class BlockSparseFlashAttention:
         q = _kernel_ready(q)
         k = _kernel_ready(k)
         v = _kernel_ready(v)
-        mask = _mask_bytes(block_mask.to(q.device))
-        cu_dev = cu_seqlens.to(device=q.device, dtype=torch.int32).contiguous()
+        mask = _mask_bytes(block_mask if block_mask.device == q.device else block_mask.to(q.device))
+        cu_dev = _int32_on(cu_seqlens, q.device)
         out = torch.empty_like(q)
         status = lib.tasft_bsfa_prefill_varlen_fwd(
             q.data_ptr(), k.data_ptr(), v.data_ptr(), out.data_ptr(), mask.data_ptr(),
@@ -468,10 +475,10 @@ class BlockSparseFlashAttention:
         q = q.contiguous()
         k_cache = _kernel_ready(k_cache)
         v_cache = _kernel_ready(v_cache)
-        mask = _mask_bytes(block_mask.to(q.device))
+        mask = _mask_bytes(block_mask if block_mask.device == q.device else block_mask.to(q.device))
         lens = None
         if kv_lens is not None:
-            lens = kv_lens.to(device=q.device, dtype=torch.int32).contiguous()
+            lens = _int32_on(kv_lens, q.device)
             if lens.shape != (B,):
                 raise KernelError(f"kv_lens must have shape ({B},), got {tuple(lens.shape)}",
                                   context={"kv_lens": list(lens.shape)})
@@ -583,10 +590,10 @@ class BlockSparseFlashAttention:
         q = q.contiguous()
         k_pages = _kernel_ready(k_pages)
         v_pages = _kernel_ready(v_pages)
-        mask = _mask_bytes(block_mask.to(q.device))
+        mask = _mask_bytes(block_mask if block_mask.device == q.device else block_mask.to(q.device))
         # The kernel reads the table with a unit column stride.
-        table = block_table.to(device=q.device, dtype=torch.int32).contiguous()
-        lens = kv_lens.to(device=q.device, dtype=torch.int32).contiguous()
+        table = _int32_on(block_table, q.device)
+        lens = _int32_on(kv_lens, q.device)
         ws_bytes = lib.tasft_bsfa_decode_workspace_bytes(B, H, D, num_splits)
         workspace = torch.empty(ws_bytes, dtype=torch.uint8, device=q.device)
         out = torch.empty((B, H, 1, D), dtype=q.dtype, device=q.device)

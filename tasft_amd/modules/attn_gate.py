@@ -192,7 +192,10 @@ class AttnGate(nn.Module):
     def _needs_grad(self, q: torch.Tensor, k: torch.Tensor) -> bool:
         if not torch.is_grad_enabled():
             return False
-        return q.requires_grad or k.requires_grad or any(p.requires_grad for p in self.parameters())
+        proj_in = self.gate_proj_in
+        return (q.requires_grad or k.requires_grad or proj_in.weight.requires_grad
+                or (proj_in.bias is not None and proj_in.bias.requires_grad)
+                or self.gate_proj_out.weight.requires_grad)
 
     def forward(
         self,
@@ -247,6 +250,9 @@ class AttnGate(nn.Module):
 
     def _thresholds(self, tau: float | torch.Tensor, device: torch.device) -> torch.Tensor:
         if isinstance(tau, torch.Tensor):
+            if (tau.dtype == torch.float32 and tau.device == device and tau.ndim == 1
+                    and tau.shape[0] == self.num_heads and tau.is_contiguous()):
+                return tau
             t = tau.to(device=device, dtype=torch.float32).reshape(-1)
             if t.numel() == 1:
                 return t.expand(self.num_heads).contiguous()
@@ -261,7 +267,7 @@ class AttnGate(nn.Module):
                      return_logits: bool, force_diagonal: bool) -> GateOutput:
         r = _launch_gate(self, q, k, self._thresholds(tau, q.device), return_logits,
                          force_diagonal, keep=False)
-        return GateOutput(soft_scores=r["soft"], hard_mask=r["mask"].view(torch.bool),
+        return GateOutput(soft_scores=r["soft"], hard_mask=r["mask"],
                           num_blocks_q=r["nb"], num_blocks_k=r["nb"], logits=r["logits"],
                           active_count=r["active"])
 
@@ -275,7 +281,7 @@ class AttnGate(nn.Module):
             q, k, self.gate_proj_in.weight, self.gate_proj_in.bias, self.gate_proj_out.weight,
             self, taus, force_diagonal)
         nb = soft.shape[-1]
-        return GateOutput(soft_scores=soft, hard_mask=mask.view(torch.bool), num_blocks_q=nb,
+        return GateOutput(soft_scores=soft, hard_mask=mask, num_blocks_q=nb,
                           num_blocks_k=nb, logits=None, active_count=active)
 
     def _forward_torch(self, q: torch.Tensor, k: torch.Tensor, tau: float | torch.Tensor,
@@ -392,7 +398,15 @@ class AttnGate(nn.Module):
 
 
 def _kernel_layout(t: torch.Tensor) -> torch.Tensor:
-    return t if (t.stride(-1) == 1 and all(s % 8 == 0 for s in t.stride()[:-1])) else t.contiguous()
+    return t if _native.kernel_layout(t, align=False) else t.contiguous()
+
+
+def _f32_on(t: torch.Tensor, device: torch.device) -> torch.Tensor:
+    """A parameter as the kernels read it (fp32, contiguous, on ``device``), without autograd."""
+    t = t.detach()
+    if t.dtype == torch.float32 and t.device == device and t.is_contiguous():
+        return t
+    return t.to(device=device, dtype=torch.float32).contiguous()
 
 
 def _launch_gate(gate: AttnGate, q: torch.Tensor, k: torch.Tensor, taus: torch.Tensor,
@@ -405,13 +419,14 @@ def _launch_gate(gate: AttnGate, q: torch.Tensor, k: torch.Tensor, taus: torch.T
     dev = q.device
     q = _kernel_layout(q.detach())
     k = _kernel_layout(k.detach())
-    w_in = gate.gate_proj_in.weight.detach().to(device=dev, dtype=torch.float32).contiguous()
-    b_in = gate.gate_proj_in.bias.detach().to(device=dev, dtype=torch.float32).contiguous()
-    w_out = gate.gate_proj_out.weight.detach().to(device=dev, dtype=torch.float32).reshape(-1).contiguous()
+    proj_in = gate.gate_proj_in
+    w_in = _f32_on(proj_in.weight, dev)
+    b_in = _f32_on(proj_in.bias, dev)
+    w_out = _f32_on(gate.gate_proj_out.weight, dev).view(-1)
     nb = math.ceil(S / gate.block_size)
     hidden = gate.gate_hidden_dim
     soft = torch.empty((B, H, nb, nb), dtype=torch.float32, device=dev)
-    mask = torch.empty((B, H, nb, nb), dtype=torch.uint8, device=dev)
+    mask = torch.empty((B, H, nb, nb), dtype=torch.bool, device=dev)  # one byte a block
     logits = torch.empty((B, H, nb, nb), dtype=torch.float32, device=dev) if return_logits else None
     active = torch.empty((1,), dtype=torch.int64, device=dev)
     qm = torch.empty((B, H, nb, D), dtype=torch.float32, device=dev) if keep else None
@@ -467,10 +482,14 @@ class _HipGateFunction(torch.autograd.Function):
         ctx.save_for_backward(r["soft"], r["workspace"], r["q_means"], r["k_means"], r["w_in"],
                               r["w_out"])
         ctx.mark_non_differentiable(r["mask"], r["active"])
+        # No zero gradients for the mask and the count (two fills of their size per backward).
+        ctx.set_materialize_grads(False)
         return r["soft"], r["mask"], r["active"]
 
     @staticmethod
     def backward(ctx, grad_soft, _grad_mask, _grad_active):
+        if grad_soft is None:
+            return (None,) * 8
         soft, workspace, qm, km, w_in, w_out = ctx.saved_tensors
         bs, hidden, causal = ctx.gate_cfg
         (B, H, S, D), (_, Hkv, _, _) = ctx.shapes

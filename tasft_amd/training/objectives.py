@@ -176,8 +176,8 @@ def _launch_gate_target(q, k, block_size, causal, scale, normalize, temperature,
     B, H, S, D = q.shape
     dtype = _native.dtype_code(q.dtype, "gate target kernel")
     lib = _native.load_library()
-    q = q if (q.stride(-1) == 1 and all(s % 8 == 0 for s in q.stride()[:-1])) else q.contiguous()
-    k = k if (k.stride(-1) == 1 and all(s % 8 == 0 for s in k.stride()[:-1])) else k.contiguous()
+    q = q if _native.kernel_layout(q, align=False) else q.contiguous()
+    k = k if _native.kernel_layout(k, align=False) else k.contiguous()
     nb = math.ceil(S / block_size)
     mask_buf, mask_strides = None, None
     if attention_mask is not None:
@@ -221,7 +221,7 @@ def _padded_attention_mask(mask: torch.Tensor, B: int, H: int, S: int, padded: i
         status.data_ptr(), _native.stream_handle(device))
     _native.check(code, "tasft_gate_mask_pad", {"attention_mask": list(mask.shape)})
     st = buf.stride()
-    strides = [st[0] if mb > 1 else 0, st[1] if mh > 1 else 0, st[2] if rows > 1 else 0]
+    strides = (st[0] if mb > 1 else 0, st[1] if mh > 1 else 0, st[2] if rows > 1 else 0)
     return buf, _native.strides_array(strides)
 
 
