@@ -17,8 +17,8 @@
 // optional logits, the uint8 hard mask and the active count. Flag bit 1 forces the
 // diagonal blocks on in the hard mask (soft scores unchanged).
 //
-// Block size 64, D in {64, 128}, hidden a multiple of 32 up to 128 (the benchmarked gate):
-// one kernel, gate_fused64_kernel, after a one-workgroup reset of its completion counters.
+// Block size 64, D in {64, 128}, hidden a multiple of 32 up to 128, more than one workgroup of
+// 16 blocks per CU (the benchmarked gate): one kernel, gate_fused64_kernel, after a one-workgroup reset of its completion counters.
 // Its first workgroups pool and project the key chunks; every other workgroup pools and
 // projects one query chunk, waits for its KV group's key units and evaluates the chunk's
 // rows. Otherwise one pooling launch (streaming for blocks 32, 64 and 128 with D in
@@ -155,6 +155,7 @@ gate_pool_project_kernel(const GatePoolParams p) {
 // computes one hidden unit for 8 of the blocks from one read of its W_in row (the W_in
 // halves are L2-resident), so the projection adds no HBM traffic and no launch.
 constexpr int kFusePB = 16;
+constexpr int kSmallPB = 4;  // blocks per workgroup in small launches: one load group
 // Cache policy of the pooling loads: sc0 + nt (streamed: every byte of Q and K is read
 // once here), measured 5% faster than the default policy.
 constexpr int kStreamLoad = 3;
@@ -164,10 +165,11 @@ __device__ __forceinline__ __amdgpu_buffer_rsrc_t gate_rsrc(const void* base, in
   return __builtin_amdgcn_make_buffer_rsrc((void*)base, (short)0, n, 0x00020000);
 }
 
-// Pools kFusePB blocks (chunk `chunk`) of BSZ rows (32, 64 or 128) of one (b, head) row stream
-// of Q (is_q) or K and projects their means; `red` is the workgroup's LDS (4 x kFusePB x D
+// Pools PB blocks (chunk `chunk`) of BSZ rows (32, 64 or 128) of one (b, head) row stream of Q
+// (is_q) or K and projects their means: kFusePB of them, or one load group in small launches,
+// whose W_in rows are then requested first; `red` is the workgroup's LDS (4 x kFusePB x D
 // floats).
-template <int D, int DT, int BSZ = 64, bool PUBLISH = false>
+template <int D, int DT, int BSZ = 64, bool PUBLISH = false, int PB = kFusePB>
 __device__ __forceinline__ void pool_proj64(const GatePoolParams& p, bool is_q, int64_t bh,
                                             int chunk, float (&red)[4][kFusePB][D]) {
   static_assert(BSZ == 32 || BSZ == 64 || BSZ == 128, "block rows");
@@ -184,14 +186,30 @@ __device__ __forceinline__ void pool_proj64(const GatePoolParams& p, bool is_q, 
   const int h = (int)(bh % heads);
   const uint16_t* src = is_q ? p.q + b * p.sq[0] + h * p.sq[1] : p.k + b * p.sk[0] + h * p.sk[1];
   const int srow = (int)(is_q ? p.sq[2] : p.sk[2]);
-  const int blk0 = chunk * kFusePB;
-  const int nblk = min(kFusePB, p.NB - blk0);
+  const int blk0 = chunk * PB;
+  const int nblk = min(PB, p.NB - blk0);
   const int row0 = blk0 * BSZ;
   const __amdgpu_buffer_rsrc_t r =
       gate_rsrc(src + (int64_t)row0 * srow, (int64_t)(p.S - row0) * srow * 2);
 
   const int dc = tid % DOCT, rg = tid / DOCT;
   const int wave = tid / kWave;
+  // W_in staging role: 16-byte chunk e % WCH of row e / WCH of a 16-row tile (rows past hidden
+  // read row 0; their results are not stored).
+  constexpr int WCH = D / 4;  // 16-byte chunks per staged row
+  constexpr int WPL = (16 * WCH) / kWave;
+  const int lane = tid % kWave;
+  const int off = is_q ? 0 : D;
+  f32x4_t wt[WPL];
+  auto load_w = [&](int nt) {
+#pragma unroll
+    for (int i = 0; i < WPL; ++i) {
+      const int e = i * kWave + lane, r = e / WCH, k = e % WCH;
+      const int row = nt * 16 + r < p.hidden ? nt * 16 + r : 0;
+      wt[i] = *(const f32x4_t*)(p.w_in + (int64_t)row * 2 * D + off + 4 * k);
+    }
+  };
+  if constexpr (PB < kFusePB) load_w(wave);
   for (int g = 0; g < nblk; g += GB) {
     u32x4_t v[GB][RPT];
 #pragma unroll
@@ -220,7 +238,7 @@ __device__ __forceinline__ void pool_proj64(const GatePoolParams& p, bool is_q, 
         if (WRG == 8) x += __shfl_xor(x, 8, 64);
         acc[j] = x;
       }
-      if ((tid % kWave) < DOCT && g + bi < kFusePB) {
+      if ((tid % kWave) < DOCT && g + bi < PB) {
 #pragma unroll
         for (int j = 0; j < 8; ++j) red[wave][g + bi][dc * 8 + j] = acc[j];
       }
@@ -251,9 +269,8 @@ __device__ __forceinline__ void pool_proj64(const GatePoolParams& p, bool is_q, 
   // 64 cache lines per load.
   static_assert(kFusePB == 16, "one 16-row MFMA tile of blocks");
   constexpr int KQ = D / 4;      // k-steps per lane group
-  constexpr int WCH = D / 4;     // 16-byte chunks per staged row
   static_assert(4 * 16 * D <= 4 * kFusePB * D, "W staging fits the pooling LDS");
-  const int lane = tid % kWave, lr = lane % 16, lq = lane / 16;
+  const int lr = lane % 16, lq = lane / 16;
   float a[KQ];
 #pragma unroll
   for (int s4 = 0; s4 < KQ; s4 += 4) {
@@ -264,17 +281,14 @@ __device__ __forceinline__ void pool_proj64(const GatePoolParams& p, bool is_q, 
   // This wave's staging area: 16 rows x D floats, 16-byte chunk k of row r at position
   // k ^ (r & 7) (conflict-free operand reads).
   float* wst = &red[0][0][0] + wave * 16 * D;
-  const int off = is_q ? 0 : D;
   float* dst = (is_q ? p.uq : p.uk) + (bh * p.NB + blk0) * (int64_t)p.hidden;
   const int ntiles = (p.hidden + 15) / 16;
   for (int nt = wave; nt < ntiles; nt += 4) {
-    // Copy rows nt*16 .. +15 (rows past hidden read row 0; their results are not stored).
+    if (PB == kFusePB || nt != wave) load_w(nt);
 #pragma unroll
-    for (int i = 0; i < (16 * WCH) / kWave; ++i) {
+    for (int i = 0; i < WPL; ++i) {
       const int e = i * kWave + lane, r = e / WCH, k = e % WCH;
-      const int row = nt * 16 + r < p.hidden ? nt * 16 + r : 0;
-      const f32x4_t v = *(const f32x4_t*)(p.w_in + (int64_t)row * 2 * D + off + 4 * k);
-      *(f32x4_t*)(wst + r * D + 4 * (k ^ (r & 7))) = v;
+      *(f32x4_t*)(wst + r * D + 4 * (k ^ (r & 7))) = wt[i];
     }
     const int c = nt * 16 + lr;
     f32x4_t acc = {0.f, 0.f, 0.f, 0.f};
@@ -307,21 +321,21 @@ __device__ __forceinline__ void pool_proj64(const GatePoolParams& p, bool is_q, 
 
 // Workgroup wg0 + blockIdx.x pools query chunks first (B x Hq x chunks, see query_chunk),
 // then key chunks.
-template <int D, int DT, int BSZ = 64>
+template <int D, int DT, int BSZ, int PB>
 __global__ void __launch_bounds__(256)
 gate_pool_proj64_kernel(const GatePoolParams p) {
   __shared__ __attribute__((aligned(16))) float red[4][kFusePB][D];  // per-wave sums, then means
   if (blockIdx.x == 0 && threadIdx.x == 0 && p.counter) *p.counter = 0ull;
-  const int chunks = (p.NB + kFusePB - 1) / kFusePB;
+  const int chunks = (p.NB + PB - 1) / PB;
   const int64_t nq = (int64_t)p.B * p.Hq * chunks;
   const int64_t wg = (int64_t)blockIdx.x + p.wg0;
   if (wg < nq) {
     int64_t bh;
     int chunk;
     query_chunk(p, wg, chunks, bh, chunk);
-    pool_proj64<D, DT, BSZ>(p, true, bh, chunk, red);
+    pool_proj64<D, DT, BSZ, false, PB>(p, true, bh, chunk, red);
   } else {
-    pool_proj64<D, DT, BSZ>(p, false, (wg - nq) / chunks, (int)((wg - nq) % chunks), red);
+    pool_proj64<D, DT, BSZ, false, PB>(p, false, (wg - nq) / chunks, (int)((wg - nq) % chunks), red);
   }
 }
 
@@ -1245,6 +1259,36 @@ static int gate_device_cus() {
   return cached[dev];
 }
 
+// The pooling and projection launch: a chunk of kFusePB blocks per workgroup; with SMALL (block
+// 64) one load group.
+template <int D, int DT, bool SMALL>
+static hipError_t launch_pool_proj_dt(const GatePoolParams& p, int64_t block_size, hipStream_t s) {
+  constexpr int PB = SMALL ? kSmallPB : kFusePB;
+  const int64_t chunks = (p.NB + PB - 1) / PB;
+  const dim3 g((unsigned)((int64_t)p.B * (p.Hq + p.Hkv) * chunks));
+  if constexpr (SMALL) {
+    hipLaunchKernelGGL((gate_pool_proj64_kernel<D, DT, 64, PB>), g, dim3(256), 0, s, p);
+  } else {
+    if (block_size == 32)
+      hipLaunchKernelGGL((gate_pool_proj64_kernel<D, DT, 32, PB>), g, dim3(256), 0, s, p);
+    else if (block_size == 128)
+      hipLaunchKernelGGL((gate_pool_proj64_kernel<D, DT, 128, PB>), g, dim3(256), 0, s, p);
+    else
+      hipLaunchKernelGGL((gate_pool_proj64_kernel<D, DT, 64, PB>), g, dim3(256), 0, s, p);
+  }
+  return hipGetLastError();
+}
+
+template <bool SMALL>
+static hipError_t launch_pool_proj(const GatePoolParams& p, int64_t head_dim, int64_t block_size,
+                                   int dtype, hipStream_t s) {
+  if (head_dim == 128)
+    return dtype == kF16 ? launch_pool_proj_dt<128, kF16, SMALL>(p, block_size, s)
+                         : launch_pool_proj_dt<128, kBf16, SMALL>(p, block_size, s);
+  return dtype == kF16 ? launch_pool_proj_dt<64, kF16, SMALL>(p, block_size, s)
+                       : launch_pool_proj_dt<64, kBf16, SMALL>(p, block_size, s);
+}
+
 // Diagnostic switch of tasft_gate_debug_wait_fault: while set, the one-launch gate's key
 // workgroups publish nothing and each query workgroup's wait gives up after kGateFaultTicks.
 static std::atomic<int> g_gate_wait_fault{0};
@@ -1382,7 +1426,15 @@ extern "C" int tasft_gate_fwd(const void* q, const void* k, const float* w_in, c
     // Block 64 with hidden a multiple of kFuseHid, at most kFuseMaxHid: the whole gate in
     // gate_fused64_kernel. Otherwise one launch pools and projects Q and K, and
     // gate_pairwise_kernel follows.
-    const bool fused = block_size == 64 && hidden % kFuseHid == 0 && hidden <= kFuseMaxHid;
+    // Small launches (at most one workgroup of 16 blocks per CU) pool four blocks per workgroup
+    // instead and run the pairwise tiles as a second launch: a workgroup's 16 blocks are four
+    // trips to memory in a row, and few workgroups share a CU to hide them. 32/8 heads, hidden
+    // 32 / 128: S=1000 12.3 / 16.8 us against 18.4 / 26.3 in one kernel (with its counter reset);
+    // S=4096 (160 workgroups) 23.8 against 28.8; B=1, S=8192 (320) 37.9 against 37.4.
+    // The diagnostic of the one kernel's wait keeps to that kernel.
+    const bool small = block_size == 64 && !g_gate_wait_fault &&
+                       batch * (num_q_heads + num_kv_heads) * fchunks <= 256;
+    const bool fused = block_size == 64 && hidden % kFuseHid == 0 && hidden <= kFuseMaxHid && !small;
     if (fused) {
       // One launch: key chunks, then query chunks (gate_fused64_kernel), after the
       // completion counters and the active count are zeroed.
@@ -1407,35 +1459,9 @@ extern "C" int tasft_gate_fwd(const void* q, const void* k, const float* w_in, c
         return set_error(kErrLaunch, "gate: fused launch failed: %s", hipGetErrorString(err));
       return kOk;
     }
-    const dim3 g1((unsigned)(batch * (num_q_heads + num_kv_heads) * fchunks));
-    if (block_size == 32) {
-      if (head_dim == 128 && dtype == kF16)
-        hipLaunchKernelGGL((gate_pool_proj64_kernel<128, kF16, 32>), g1, dim3(256), 0, s, pp);
-      else if (head_dim == 128)
-        hipLaunchKernelGGL((gate_pool_proj64_kernel<128, kBf16, 32>), g1, dim3(256), 0, s, pp);
-      else if (dtype == kF16)
-        hipLaunchKernelGGL((gate_pool_proj64_kernel<64, kF16, 32>), g1, dim3(256), 0, s, pp);
-      else
-        hipLaunchKernelGGL((gate_pool_proj64_kernel<64, kBf16, 32>), g1, dim3(256), 0, s, pp);
-    } else if (block_size == 128) {
-      // Blocks 32 and 128: the same streaming pool, then gate_pairwise_kernel.
-      if (head_dim == 128 && dtype == kF16)
-        hipLaunchKernelGGL((gate_pool_proj64_kernel<128, kF16, 128>), g1, dim3(256), 0, s, pp);
-      else if (head_dim == 128)
-        hipLaunchKernelGGL((gate_pool_proj64_kernel<128, kBf16, 128>), g1, dim3(256), 0, s, pp);
-      else if (dtype == kF16)
-        hipLaunchKernelGGL((gate_pool_proj64_kernel<64, kF16, 128>), g1, dim3(256), 0, s, pp);
-      else
-        hipLaunchKernelGGL((gate_pool_proj64_kernel<64, kBf16, 128>), g1, dim3(256), 0, s, pp);
-    } else if (head_dim == 128 && dtype == kF16)
-      hipLaunchKernelGGL((gate_pool_proj64_kernel<128, kF16>), g1, dim3(256), 0, s, pp);
-    else if (head_dim == 128)
-      hipLaunchKernelGGL((gate_pool_proj64_kernel<128, kBf16>), g1, dim3(256), 0, s, pp);
-    else if (dtype == kF16)
-      hipLaunchKernelGGL((gate_pool_proj64_kernel<64, kF16>), g1, dim3(256), 0, s, pp);
-    else
-      hipLaunchKernelGGL((gate_pool_proj64_kernel<64, kBf16>), g1, dim3(256), 0, s, pp);
-    if ((err = hipGetLastError()) != hipSuccess)
+    err = small ? launch_pool_proj<true>(pp, head_dim, block_size, dtype, s)
+                : launch_pool_proj<false>(pp, head_dim, block_size, dtype, s);
+    if (err != hipSuccess)
       return set_error(kErrLaunch, "gate: pool launch failed: %s", hipGetErrorString(err));
   } else {
     const dim3 g1((unsigned)(batch * (num_q_heads + num_kv_heads) * chunks));

@@ -402,11 +402,10 @@ def _kernel_layout(t: torch.Tensor) -> torch.Tensor:
 
 
 def _f32_on(t: torch.Tensor, device: torch.device) -> torch.Tensor:
-    """A parameter as the kernels read it (fp32, contiguous, on ``device``), without autograd."""
-    t = t.detach()
+    """A parameter as the kernels read it: fp32, contiguous, on ``device`` (itself if it is)."""
     if t.dtype == torch.float32 and t.device == device and t.is_contiguous():
         return t
-    return t.to(device=device, dtype=torch.float32).contiguous()
+    return t.detach().to(device=device, dtype=torch.float32).contiguous()
 
 
 def _launch_gate(gate: AttnGate, q: torch.Tensor, k: torch.Tensor, taus: torch.Tensor,
@@ -417,12 +416,12 @@ def _launch_gate(gate: AttnGate, q: torch.Tensor, k: torch.Tensor, taus: torch.T
     Hkv = k.shape[1]
     lib = _native.load_library()
     dev = q.device
-    q = _kernel_layout(q.detach())
-    k = _kernel_layout(k.detach())
+    q = _kernel_layout(q)
+    k = _kernel_layout(k)
     proj_in = gate.gate_proj_in
     w_in = _f32_on(proj_in.weight, dev)
     b_in = _f32_on(proj_in.bias, dev)
-    w_out = _f32_on(gate.gate_proj_out.weight, dev).view(-1)
+    w_out = _f32_on(gate.gate_proj_out.weight, dev)
     nb = math.ceil(S / gate.block_size)
     hidden = gate.gate_hidden_dim
     soft = torch.empty((B, H, nb, nb), dtype=torch.float32, device=dev)
