@@ -60,13 +60,8 @@ int tasft_abi_version(void);
  * head_dim in {64, 128}; block_size in {32, 64, 128}; strides of b/h/s multiples of 8.
  * Block size 128 runs on the block-64 kernels, each 128-token block as its four 64-token
  * quarters (the same tokens attend to the same keys).
- * workspace: NULL (one workgroup per query-block row), or >=
- * tasft_bsfa_prefill_workspace_bytes(...) bytes, 16-byte aligned: then (block size 64 or
- * 128, head_dim 64) a persistent launch keeps every CU slot busy, pulling rows from ticket
- * counters kept in the workspace (zeroed on `stream` by the call itself). head_dim 128
- * always runs one workgroup per row (its two-wave kernel fills four slots per CU) and
- * leaves the workspace untouched. The output does not depend on it.
- * Calls that share one workspace must be ordered on one stream.
+ * workspace: NULL, or >= tasft_bsfa_prefill_workspace_bytes(...) bytes, 16-byte aligned; it
+ * is checked and left untouched (every launch runs one workgroup per query-block row).
  */
 int tasft_bsfa_prefill_fwd(const void* q, const void* k, const void* v, void* out,
                            const uint8_t* block_mask, void* workspace, size_t workspace_bytes,
@@ -116,9 +111,7 @@ int tasft_bsfa_varlen_zero_tail(void* out, const int32_t* cu_seqlens, int64_t nu
                                 const int64_t* o_strides, void* stream);
 
 /*
- * Bytes of the optional workspace of tasft_bsfa_prefill_fwd (work-queue counters).
- * No reference counterpart: the reference launches one program per query block in
- * grid order (tasft/kernels/block_sparse_fa.py:517-550).
+ * Bytes of the optional workspace of tasft_bsfa_prefill_fwd, for callers that pass one.
  */
 size_t tasft_bsfa_prefill_workspace_bytes(int64_t batch, int64_t num_q_heads, int64_t seq_len,
                                           int64_t block_size);

@@ -14,7 +14,7 @@
 // tasft/modules/tasft_attention.py:725-729).
 //
 // Mapping onto CDNA4. A wave owns 32 query rows (block 32: the workgroup is one such wave;
-// blocks 64 and 128: two or four waves per 64 rows). Each key tile is computed as
+// blocks 64 and 128: two waves per 64 rows). Each key tile is computed as
 // S^T = K . Q^T with v_mfma_f32_32x32x16_bf16 (_f16 for fp16 inputs), so a lane owns one query column of S^T:
 // its running max and sum live in that lane (plus the lane 32 away), and the P^T
 // accumulator registers feed the PV product O^T = V^T . P^T directly as the B operand
@@ -42,10 +42,7 @@ struct PrefillParams {
   float scale_log2;  // softmax scale * log2(e)
   int causal;
   int small_spans;   // S * row bytes of K and V below 2^31: 32-bit DMA address math
-  int small_q;       // the same of Q (block 32)
-  int* queue;        // per-partition ticket counters of the persistent launch, or null
-  int parts;         // work partitions: 8 (one per XCD) or 1
-  int wg_per_part;   // persistent workgroups per partition
+  int small_q;       // the same of Q (block 32, head dim 64)
   // Packed variable-length batch: sequence b holds tokens cu_seqlens[b] .. cu_seqlens[b+1]-1
   // of dimension s (the b strides are 0), S is the longest length and NB its block count.
   // Null for a dense [B, H, S, D] launch.
@@ -104,35 +101,14 @@ __device__ __forceinline__ SeqSpan seq_span(const PrefillParams& p, int b) {
   return {len, (len + BS - 1) / BS, (int64_t)t0};
 }
 
-// Persistent launch (block size 64). Rows differ widely in cost (a gate can light whole
-// rows), and a grid of one workgroup per row leaves CU slots idle while heavy and light
-// rows are dispatched side by side. Instead, two workgroups per CU stay resident and
-// pull rows from a ticket counter per partition (one partition per XCD: item
-// x + 8j belongs to XCD x, so the static group-major order and its L2 locality are
-// kept). The counters live in the caller's workspace and are zeroed by
-// bsfa_queue_reset_kernel on the same stream before every launch.
-constexpr int kQueueSlots = 8;
-
-__global__ void bsfa_queue_reset_kernel(int* queue) {
-  if (threadIdx.x < kQueueSlots) queue[threadIdx.x] = 0;
-}
-
-// ---------------------------------------------------------------------------------------
-// Block size 64: the tuned kernel.
-//
-// Four waves per (batch, query head, query block): wave w owns query rows 32*(w&1)..+31
-// and the key half 32*(w>>1)..+31 of every key block, so each wave issues 8 + D/16 MFMAs
-// per block and two waves share a SIMD. The two key-half partial results of a row are
-// merged once at the end. K and V of the next active block are copied HBM -> LDS by
-// buffer_load_dwordx4 ... lds (no staging registers) into the other of two LDS stages
-// while the current block is computed (one barrier per block), row-major with a 16-byte
-// XOR swizzle (conflict-free without padding). V^T operands come from
-// ds_read_b64_tr_b16, so V is never transposed by VALU. The softmax rescale is lazy: the running maximum used
-// for exp2 is only moved when a new score exceeds it by more than kRescaleLog2 (so P
-// stays <= 2^8); numerator and denominator share the same reference, so the normalised
-// output is unchanged.
-// ---------------------------------------------------------------------------------------
+// The softmax rescale is lazy where it pays: the running maximum used for exp2 is only moved
+// when a new score exceeds it by more than this (so P stays <= 2^8); numerator and denominator
+// share the same reference, so the normalised output is unchanged.
 constexpr float kRescaleLog2 = 8.f;
+// Head dim 64: moving it earlier keeps the largest probabilities of a row near a power of two,
+// with less rounding error (8: 1% more error against 64 bits than one reference per 32 keys,
+// 2: less, at 1-2% of the time).
+constexpr float kRescale64Log2 = 2.f;
 
 // 16-byte chunk position of chunk `cc` of K row `r` in LDS.
 template <int D>
@@ -162,25 +138,6 @@ __device__ __forceinline__ int next_active_block(const uint8_t* mrow, int64_t st
   return kb;
 }
 
-// One 64 x D 16-bit tile in LDS, written by buffer_load_dwordx4 ... lds (DMA, no VGPRs).
-// Unit u (1 KB, one instruction of one wave) covers bytes u*1024 .. +1023 of the tile;
-// lane l of that instruction lands at byte u*1024 + 16*l, i.e. row (u*1024+16l)/ROWB,
-// 16-byte position ((u*1024+16l)%ROWB)/16. The lane therefore loads the global chunk
-// that the swizzle maps to that position (the XOR swizzles are involutions). The
-// buffer resource starts at the tile's first row and ends after row S-1, so rows past
-// the end of the sequence are out of range and land in LDS as zeros.
-template <int D>
-__device__ __forceinline__ void dma_tile(uint8_t* tile, __amdgpu_buffer_rsrc_t rsrc,
-                                         const int* voff, int wave) {
-  constexpr int UNITS_PER_WAVE = (64 * D * 2 / 1024) / 4;
-#pragma unroll
-  for (int i = 0; i < UNITS_PER_WAVE; ++i) {
-    const int u = wave * UNITS_PER_WAVE + i;
-    __builtin_amdgcn_raw_ptr_buffer_load_lds(rsrc, (TASFT_LDS void*)(tile + u * 1024), 16, voff[i], 0,
-                                             0, 0);
-  }
-}
-
 // Raw buffer resource (stride 0) over `bytes` bytes starting at `base`.
 __device__ __forceinline__ __amdgpu_buffer_rsrc_t tile_rsrc(const void* base, int64_t bytes) {
   const int n = bytes > 0x7fffffff ? 0x7fffffff : (bytes < 0 ? 0 : (int)bytes);
@@ -193,310 +150,8 @@ __device__ __forceinline__ void dma16_lds(__amdgpu_buffer_rsrc_t r, uint8_t* dst
   __builtin_amdgcn_raw_ptr_buffer_load_lds(r, (TASFT_LDS void*)dst, 16, voff, 0, 0, AUX);
 }
 
-template <int D, int DT>
-__global__ void __launch_bounds__(256, 2)
-bsfa_prefill_bs64_kernel(const PrefillParams p) {
-  constexpr int BS = 64;
-  constexpr int KSTEPS = D / 16;
-  constexpr int DTILES = D / 32;
-  constexpr int ROWB = D * 2;                        // bytes per K/V row in LDS
-  constexpr int TILE = BS * ROWB;                    // one K or V tile
-  constexpr int UNITS_PER_WAVE = (TILE / 1024) / 4;  // DMA instructions per wave per tile
-
-  // Two stages (A, B) of K and V tiles, each its own LDS object so that reads of one
-  // stage are not ordered behind DMA into the other.
-  __shared__ __attribute__((aligned(1024))) uint8_t kA[TILE];
-  __shared__ __attribute__((aligned(1024))) uint8_t vA[TILE];
-  __shared__ __attribute__((aligned(1024))) uint8_t kB[TILE];
-  __shared__ __attribute__((aligned(1024))) uint8_t vB[TILE];
-  __shared__ float xch_ml[2][2][2][32];  // (m, l) by row half, key half
-  __shared__ int next_slot;
-  static_assert(DTILES * 16 * kWave * 4 == TILE, "merge buffer size");
-
-  const int tid = threadIdx.x;
-  const int lane = tid & 63;
-  const int wave = __builtin_amdgcn_readfirstlane(tid >> 6);  // uniform: scalar DMA addresses
-  const int rh = wave & 1;   // row half
-  const int kh = wave >> 1;  // key half
-  const int col = lane & 31;
-  const int half = lane >> 5;
-
-  // Per-lane byte offsets (within a tile's rows) of this wave's DMA units.
-  int kvoff[UNITS_PER_WAVE], vvoff[UNITS_PER_WAVE];
-#pragma unroll
-  for (int i = 0; i < UNITS_PER_WAVE; ++i) {
-    const int byte = (wave * UNITS_PER_WAVE + i) * 1024 + lane * 16;
-    const int row = byte / ROWB, pos = (byte % ROWB) / 16;
-    kvoff[i] = (row * (int)p.sk[2] + swz_k<D>(row, pos) * 8) * 2;
-    vvoff[i] = (row * (int)p.sv[2] + swz_v<D>(row, pos) * 8) * 2;
-  }
-  const int krow_l = kh * 32 + col;
-  const int grp16 = lane >> 4, t16 = lane & 15;  // ds_read_tr group and lane in group
-  const int tr_row = t16 >> 2;                   // source row offset within a 4-row run
-  const int tr_cb = t16 & 3;                     // source 8-byte column block
-
-  // Work distribution: one item per workgroup, or the persistent ticket loop.
-  const bool persistent = p.queue != nullptr;
-  const int part = persistent ? (int)(blockIdx.x % p.parts) : 0;
-  const int64_t per_part = persistent ? (int64_t)p.B * p.Hq * p.NB / p.parts : 1;
-  int64_t slot = persistent ? (int64_t)(blockIdx.x / p.parts) : 0;
-  // A workgroup knows its next item one item ahead: the second is static (slot +
-  // wg_per_part), later ones come from tickets. The next item's first 64 mask bytes are
-  // loaded during this item, so its first K/V DMA starts without a mask round trip.
-  int64_t slot_nx = persistent ? slot + p.wg_per_part : per_part;
-  bool pre = false;   // mbyte holds the first 64 mask bytes of this item's row, item_nx its item
-  uint8_t mbyte = 0;
-  PrefillItem item_nx = {0, 0, 0, 0};
-  while (slot < per_part) {
-  const int64_t idx = !persistent ? (int64_t)blockIdx.x : (p.parts == 8 ? part + 8 * slot : slot);
-  const PrefillItem item = pre ? item_nx : prefill_item(p, idx);
-  const int qb = item.qb, b = item.b, kvh = item.kvh, h = item.h;
-  // Varlen launch: items past the last query block of a shorter sequence have no work.
-  const SeqSpan span = seq_span<BS>(p, b);
-  if (qb >= span.NB) return;  // (never in a persistent launch, which is dense)
-  const int S = span.S, NB = span.NB;
-
-
-  const uint16_t* qbase = p.q + b * p.sq[0] + span.tok0 * p.sq[2] + h * p.sq[1];
-  const uint16_t* kbase = p.k + b * p.sk[0] + span.tok0 * p.sk[2] + kvh * p.sk[1];
-  const uint16_t* vbase = p.v + b * p.sv[0] + span.tok0 * p.sv[2] + kvh * p.sv[1];
-  uint16_t* obase = p.o + b * p.so[0] + span.tok0 * p.so[2] + h * p.so[1];
-  const uint8_t* mrow = p.mask + b * p.sm[0] + h * p.sm[1] + (int64_t)(qb >> p.mshift) * p.sm[2];
-
-  const int qrow = qb * BS + rh * 32 + col;
-  const bool qvalid = qrow < S;
-  const int kb_end = p.causal ? qb + 1 : NB;
-  // Blocks from here on need element masks: the causal diagonal (the last block of a
-  // causal row, which is also the partial block if there is one) or the partial block.
-  const int mask_from = p.causal ? qb : ((S % BS) != 0 ? NB - 1 : NB);
-  // Loads go out in the order their results are needed, since waits are in issue order:
-  // this row's mask bytes (unless the previous item fetched them) and Q; the first K/V
-  // DMA follows once the mask bytes are in, and only then the next item's mask bytes and
-  // the ticket of the item after the next, which the first wait also covers.
-  uint8_t mb = mbyte;
-  if (!pre && lane < kb_end) mb = mrow[(int64_t)(lane >> p.mshift) * p.sm[3]];
-  u32x4_t qf[KSTEPS];
-  {
-    // Rows past the end read row S-1: per-row results, never stored.
-    const uint16_t* qr = qbase + (int64_t)(qvalid ? qrow : S - 1) * p.sq[2] + half * 8;
-#pragma unroll
-    for (int ks = 0; ks < KSTEPS; ++ks) qf[ks] = *(const u32x4_t*)(qr + ks * 16);
-  }
-  // Start the DMA of key block kb into one stage (rows >= S arrive as zeros). With
-  // small spans the resource base and size take 32-bit scalar math only.
-  const uint32_t krb = (uint32_t)p.sk[2] * 2u, vrb = (uint32_t)p.sv[2] * 2u;
-  auto issue = [&](uint8_t* kt, uint8_t* vt, int kb) {
-    if (p.small_spans) {
-      const uint32_t key0 = (uint32_t)kb * BS, left = (uint32_t)S - key0;
-      dma_tile<D>(kt, __builtin_amdgcn_make_buffer_rsrc((void*)((const uint8_t*)kbase + key0 * krb),
-                                                        (short)0, (int)(left * krb), 0x00020000),
-                  kvoff, wave);
-      dma_tile<D>(vt, __builtin_amdgcn_make_buffer_rsrc((void*)((const uint8_t*)vbase + key0 * vrb),
-                                                        (short)0, (int)(left * vrb), 0x00020000),
-                  vvoff, wave);
-    } else {
-      const int key0 = kb * BS;
-      const int64_t rows_left = (int64_t)(S - key0);
-      dma_tile<D>(kt, tile_rsrc(kbase + (int64_t)key0 * p.sk[2], rows_left * p.sk[2] * 2), kvoff, wave);
-      dma_tile<D>(vt, tile_rsrc(vbase + (int64_t)key0 * p.sv[2], rows_left * p.sv[2] * 2), vvoff, wave);
-    }
-  };
-
-  f32x16_t oacc[DTILES];
-#pragma unroll
-  for (int dt = 0; dt < DTILES; ++dt) oacc[dt] = (f32x16_t){};
-  float m_ref = -INFINITY;  // exp2 reference of this lane's query row (log2 domain)
-  float l_run = 0.f;
-
-  // One key block from stage (kt, vt): S^T MFMAs, online softmax, PV MFMAs.
-  auto compute = [&](const uint8_t* kt, const uint8_t* vt, int kb) {
-    // Every LDS operand of the block is requested before the first MFMA: the K fragments,
-    // then (behind a scheduling fence) the V^T fragments, whose reads the S MFMAs cover.
-    u32x4_t kf[KSTEPS];
-#pragma unroll
-    for (int ks = 0; ks < KSTEPS; ++ks) {
-      const int cc = ks * 2 + half;
-      kf[ks] = *(const u32x4_t*)(kt + krow_l * ROWB + swz_k<D>(krow_l, cc) * 16);
-    }
-    __builtin_amdgcn_sched_barrier(0);
-    u32x2_t vlo[2][DTILES], vhi[2][DTILES];
-#pragma unroll
-    for (int pp = 0; pp < 2; ++pp) {
-      const int kbase_k = kh * 32 + 16 * pp + 4 * (grp16 >> 1);  // first key of run 1
-#pragma unroll
-      for (int dt = 0; dt < DTILES; ++dt) {
-        const int d0 = dt * 32 + 16 * (grp16 & 1) + 4 * tr_cb;  // source column of this lane
-        const int cc = d0 >> 3, sub = (d0 & 7) * 2;
-        const int r1 = kbase_k + tr_row, r2 = r1 + 8;
-        vlo[pp][dt] = ds_read_tr16_b64((const void*)(vt + r1 * ROWB + swz_v<D>(r1, cc) * 16 + sub));
-        vhi[pp][dt] = ds_read_tr16_b64((const void*)(vt + r2 * ROWB + swz_v<D>(r2, cc) * 16 + sub));
-      }
-    }
-    f32x16_t s = (f32x16_t){};
-#pragma unroll
-    for (int ks = 0; ks < KSTEPS; ++ks) s = mfma16<DT>(kf[ks], qf[ks], s);
-    // Each S MFMA followed by two V^T reads.
-#pragma unroll
-    for (int ks = 0; ks < KSTEPS; ++ks) {
-      __builtin_amdgcn_sched_group_barrier(0x008, 1, 0);
-      __builtin_amdgcn_sched_group_barrier(0x100, 2, 0);
-    }
-    const int key0 = kb * BS;
-    // Causal diagonal block or partial last block: mask in one uniform branch.
-    if (kb >= mask_from) {
-#pragma unroll
-      for (int rr = 0; rr < 16; ++rr) {
-        const int key = key0 + kh * 32 + 8 * (rr >> 2) + 4 * half + (rr & 3);
-        s[rr] = (key >= S || (p.causal && key > qrow)) ? -INFINITY : s[rr];
-      }
-    }
-    // Scores stay unscaled: scale > 0 commutes with max, and exp2 takes one FMA.
-    float mraw = s[0];
-#pragma unroll
-    for (int rr = 1; rr < 16; ++rr) mraw = fmaxf(mraw, s[rr]);
-    const float mloc = pair_max32(mraw) * p.scale_log2;
-    // Lazy rescale: move the reference only when a score exceeds it by kRescaleLog2.
-    const bool move = mloc > m_ref + kRescaleLog2;
-    if (__ballot(move)) {
-      // exp2(-inf) = 0 clears the (empty) accumulators on a row's first finite score.
-      const float alpha = move ? __builtin_amdgcn_exp2f(m_ref - mloc) : 1.f;
-      l_run *= alpha;
-#pragma unroll
-      for (int dt = 0; dt < DTILES; ++dt) oacc[dt] *= alpha;
-      m_ref = move ? mloc : m_ref;
-    }
-    const float m_use = (m_ref == -INFINITY) ? 0.f : m_ref;
-    float lsum = 0.f;
-#pragma unroll
-    for (int rr = 0; rr < 16; ++rr) {
-      const float e = __builtin_amdgcn_exp2f(fmaf(s[rr], p.scale_log2, -m_use));
-      s[rr] = e;
-      lsum += e;
-    }
-    l_run += lsum;
-    // O^T += V^T P^T over this wave's 32 keys: two k-steps of 16 keys.
-#pragma unroll
-    for (int pp = 0; pp < 2; ++pp) {
-      const u32x4_t w = {pack16x2<DT>(s[8 * pp + 0], s[8 * pp + 1]),
-                         pack16x2<DT>(s[8 * pp + 2], s[8 * pp + 3]),
-                         pack16x2<DT>(s[8 * pp + 4], s[8 * pp + 5]),
-                         pack16x2<DT>(s[8 * pp + 6], s[8 * pp + 7])};
-      const u32x4_t pb = w;
-#pragma unroll
-      for (int dt = 0; dt < DTILES; ++dt) {
-        const u32x4_t a = {vlo[pp][dt][0], vlo[pp][dt][1], vhi[pp][dt][0], vhi[pp][dt][1]};
-        oacc[dt] = mfma16<DT>(a, pb, oacc[dt]);
-      }
-    }
-  };
-
-  int chunk = 0;
-  uint64_t bits = __ballot(mb != 0);
-  int kb = next_active_block(mrow, p.sm[3], kb_end, lane, chunk, bits, p.mshift);
-  if (kb >= 0) issue(kA, vA, kb);
-  mbyte = 0;
-  pre = slot_nx < per_part;
-  if (pre) {
-    item_nx = prefill_item(p, p.parts == 8 ? part + 8 * slot_nx : slot_nx);
-    const int kb_end_nx = p.causal ? item_nx.qb + 1 : p.NB;
-    const uint8_t* mrow_nx =
-        p.mask + item_nx.b * p.sm[0] + item_nx.h * p.sm[1] + (int64_t)(item_nx.qb >> p.mshift) * p.sm[2];
-    if (lane < kb_end_nx) mbyte = mrow_nx[(int64_t)(lane >> p.mshift) * p.sm[3]];
-  }
-  // atomicInc (not atomicAdd, which the compiler rewrites into a wave-aggregated form that
-  // waits for the result on the spot); the counter never reaches the wrap limit.
-  int ticket = 0;
-  if (persistent && tid == 0) ticket = (int)atomicInc((unsigned*)&p.queue[part], 0xffffffffu);
-  // Unrolled by two so each stage is a fixed LDS object.
-  while (kb >= 0) {
-    __builtin_amdgcn_s_waitcnt(0x0f70);  // vmcnt(0): this wave's DMA of block kb landed
-    __syncthreads();                      // every wave's DMA landed; stage B is free
-    int kb_next = next_active_block(mrow, p.sm[3], kb_end, lane, chunk, bits, p.mshift);
-    if (kb_next >= 0) issue(kB, vB, kb_next);
-    compute(kA, vA, kb);
-    kb = kb_next;
-    if (kb < 0) break;
-    __builtin_amdgcn_s_waitcnt(0x0f70);
-    __syncthreads();
-    kb_next = next_active_block(mrow, p.sm[3], kb_end, lane, chunk, bits, p.mshift);
-    if (kb_next >= 0) issue(kA, vA, kb_next);
-    compute(kB, vB, kb);
-    kb = kb_next;
-  }
-
-  // Merge the two key halves of each row. Each wave finalises half of the head dims (key
-  // half 0 the first DTILES/2 tiles, key half 1 the rest) and hands its partner the other
-  // half of its partial O^T and its (m, l), through stage A.
-  constexpr int HT = DTILES / 2;
-  const float l_tot = pair_sum32(l_run);
-  __syncthreads();  // every wave is done with stage A
-  float* xo = (float*)(rh == 0 ? kA : vA);  // 2 x HT tiles of 16 x 64 floats per row half
-  auto send = [&](auto khc) {
-    constexpr int KH = decltype(khc)::value;
-    float* out = xo + KH * (HT * 16 * kWave);
-#pragma unroll
-    for (int j = 0; j < HT; ++j)
-#pragma unroll
-      for (int rr = 0; rr < 16; ++rr) out[(j * 16 + rr) * kWave + lane] = oacc[(1 - KH) * HT + j][rr];
-    if (half == 0) {
-      xch_ml[rh][KH][0][col] = m_ref;
-      xch_ml[rh][KH][1][col] = l_tot;
-    }
-  };
-  auto finish = [&](auto khc) {
-    constexpr int KH = decltype(khc)::value;
-    const float* in = xo + (1 - KH) * (HT * 16 * kWave);
-    const float mp = xch_ml[rh][1 - KH][0][col], lp = xch_ml[rh][1 - KH][1][col];
-    // The same expressions in both waves, in key-half order.
-    const float m0 = KH == 0 ? m_ref : mp, m1 = KH == 0 ? mp : m_ref;
-    const float l0 = KH == 0 ? l_tot : lp, l1 = KH == 0 ? lp : l_tot;
-    const float M = fmaxf(m0, m1);
-    const float Mu = (M == -INFINITY) ? 0.f : M;
-    const float f0 = __builtin_amdgcn_exp2f(m0 - Mu);  // 0 for an empty half
-    const float f1 = __builtin_amdgcn_exp2f(m1 - Mu);
-    const float L = l0 * f0 + l1 * f1;
-    const float inv = 1.f / (L > 0.f ? L : 1.f);  // empty rows: O = 0; NaN rows stay NaN
-    if (qvalid) {
-      uint16_t* orow = obase + (int64_t)qrow * p.so[2];
-#pragma unroll
-      for (int j = 0; j < HT; ++j) {
-        const int dt = KH * HT + j;
-#pragma unroll
-        for (int gq = 0; gq < 4; ++gq) {
-          float o4[4];
-#pragma unroll
-          for (int e = 0; e < 4; ++e) {
-            const int rr = 4 * gq + e;
-            const float mine = oacc[dt][rr], theirs = in[(j * 16 + rr) * kWave + lane];
-            const float p0 = KH == 0 ? mine : theirs, p1 = KH == 0 ? theirs : mine;
-            o4[e] = (p0 * f0 + p1 * f1) * inv;
-          }
-          const int d0 = dt * 32 + 8 * gq + 4 * half;
-          const u32x2_t w = {pack16x2<DT>(o4[0], o4[1]), pack16x2<DT>(o4[2], o4[3])};
-          *(u32x2_t*)(orow + d0) = w;
-        }
-      }
-    }
-  };
-  if (kh == 0)
-    send(std::integral_constant<int, 0>{});
-  else
-    send(std::integral_constant<int, 1>{});
-  __syncthreads();
-  if (kh == 0)
-    finish(std::integral_constant<int, 0>{});
-  else
-    finish(std::integral_constant<int, 1>{});
-  if (!persistent) break;
-  if (tid == 0) next_slot = 2 * p.wg_per_part + ticket;
-  __syncthreads();  // merge buffer, stages and next_slot are free for the next item
-  slot = slot_nx;
-  slot_nx = __builtin_amdgcn_readfirstlane(next_slot);
-  }
-}
-
 // ---------------------------------------------------------------------------------------
-// Block size 64, head dim 128: two waves per query block.
+// Block size 64 (and 128, through the mask index shift): two waves per query block.
 //
 // Wave w owns query rows 32*w..+31 and all 64 keys of every active key block: 16 S MFMAs
 // (two 32-key tiles) and 16 PV MFMAs per block, so a row needs no merge of partial
@@ -513,6 +168,11 @@ bsfa_prefill_bs64_kernel(const PrefillParams p) {
 // read into the MFMA operand registers like K; O is written there per wave and stored as
 // whole rows, four per instruction. Loading Q and storing O directly in the MFMA layouts
 // touched 32 rows, 32 bytes each, per instruction (1 KB of data in 32 cache lines).
+//
+// Head dim 64 takes 16 KB of LDS and three waves per SIMD (129 registers; four, with 122,
+// measured 4% faster at B=4, S=8192 and 4% slower on dense masks). Against four waves per query
+// block with two LDS stages and a merge of key halves, 32/8 heads, a fifth of the blocks: B=2,
+// S=4096 53 us (66.5); B=4, S=8192 310 us (332); S=1000 14.5 us (17); blocks of 128 58 us (69).
 // ---------------------------------------------------------------------------------------
 // Workgroup barrier without a memory fence. The caller waits (s_waitcnt) for what the
 // barrier publishes; the memory clobber keeps the compiler from moving memory accesses
@@ -524,21 +184,26 @@ __device__ __forceinline__ void block_barrier() { asm volatile("s_barrier" ::: "
 template <int D, int AUX = 0>
 __device__ __forceinline__ void dma_tile_2w(uint8_t* tile, __amdgpu_buffer_rsrc_t rsrc,
                                             const int* voff, int wave) {
-  static_assert(D == 128, "eight 1 KB units per wave and tile");
-  TASFT_LDS void* b0 = (TASFT_LDS void*)(tile + wave * 8192);
-  TASFT_LDS void* b1 = (TASFT_LDS void*)(tile + wave * 8192 + 4096);
-  __builtin_amdgcn_raw_ptr_buffer_load_lds(rsrc, b0, 16, voff[0], 0, 0, AUX);
-  __builtin_amdgcn_raw_ptr_buffer_load_lds(rsrc, b0, 16, voff[1], 0, 1024, AUX);
-  __builtin_amdgcn_raw_ptr_buffer_load_lds(rsrc, b0, 16, voff[2], 0, 2048, AUX);
-  __builtin_amdgcn_raw_ptr_buffer_load_lds(rsrc, b0, 16, voff[3], 0, 3072, AUX);
-  __builtin_amdgcn_raw_ptr_buffer_load_lds(rsrc, b1, 16, voff[4], 0, 0, AUX);
-  __builtin_amdgcn_raw_ptr_buffer_load_lds(rsrc, b1, 16, voff[5], 0, 1024, AUX);
-  __builtin_amdgcn_raw_ptr_buffer_load_lds(rsrc, b1, 16, voff[6], 0, 2048, AUX);
-  __builtin_amdgcn_raw_ptr_buffer_load_lds(rsrc, b1, 16, voff[7], 0, 3072, AUX);
+  if constexpr (D == 128) {
+    TASFT_LDS void* b0 = (TASFT_LDS void*)(tile + wave * 8192);
+    TASFT_LDS void* b1 = (TASFT_LDS void*)(tile + wave * 8192 + 4096);
+    __builtin_amdgcn_raw_ptr_buffer_load_lds(rsrc, b0, 16, voff[0], 0, 0, AUX);
+    __builtin_amdgcn_raw_ptr_buffer_load_lds(rsrc, b0, 16, voff[1], 0, 1024, AUX);
+    __builtin_amdgcn_raw_ptr_buffer_load_lds(rsrc, b0, 16, voff[2], 0, 2048, AUX);
+    __builtin_amdgcn_raw_ptr_buffer_load_lds(rsrc, b0, 16, voff[3], 0, 3072, AUX);
+    __builtin_amdgcn_raw_ptr_buffer_load_lds(rsrc, b1, 16, voff[4], 0, 0, AUX);
+    __builtin_amdgcn_raw_ptr_buffer_load_lds(rsrc, b1, 16, voff[5], 0, 1024, AUX);
+    __builtin_amdgcn_raw_ptr_buffer_load_lds(rsrc, b1, 16, voff[6], 0, 2048, AUX);
+    __builtin_amdgcn_raw_ptr_buffer_load_lds(rsrc, b1, 16, voff[7], 0, 3072, AUX);
+  } else {
+    // Four units per wave, each with its own LDS base: row strides below 128 bytes stay legal.
+#pragma unroll
+    for (int i = 0; i < 4; ++i) dma16_lds<AUX>(rsrc, tile + wave * 4096 + i * 1024, voff[i]);
+  }
 }
 
 template <int D, int DT>
-__global__ void __launch_bounds__(128) __attribute__((amdgpu_waves_per_eu(2, 2)))
+__global__ void __launch_bounds__(128) __attribute__((amdgpu_waves_per_eu(D == 64 ? 3 : 2, D == 64 ? 3 : 2)))
 bsfa_prefill_bs64_2w_kernel(const PrefillParams p) {
   constexpr int BS = 64;
   constexpr int KSTEPS = D / 16;
@@ -546,6 +211,9 @@ bsfa_prefill_bs64_2w_kernel(const PrefillParams p) {
   constexpr int ROWB = D * 2;
   constexpr int TILE = BS * ROWB;
   constexpr int UPW = (TILE / 1024) / 2;  // DMA units per wave and tile
+  constexpr int kWaitTile = 0x0f70 | UPW;  // vmcnt: all but the last tile's units have landed
+  constexpr float kMove = D == 128 ? kRescaleLog2 : kRescale64Log2;
+  constexpr int LOW = D == 128 ? 1024 : 0;  // what dma_tile_2w's instruction offsets add per unit
 
   __shared__ __attribute__((aligned(1024))) uint8_t kS[TILE];
   __shared__ __attribute__((aligned(1024))) uint8_t vS[TILE];
@@ -555,7 +223,8 @@ bsfa_prefill_bs64_2w_kernel(const PrefillParams p) {
   const int col = lane & 31;
   const int half = lane >> 5;
 
-  // Per-lane source offsets of this wave's DMA units (see dma_tile), less the instruction
+  // Per-lane source offsets of this wave's DMA units (the lane loads the
+  // chunk that the self-inverse swizzle maps to its 16 bytes), less the instruction
   // offset that dma_tile_2w adds. Unit u starts at tile row 4u >= 4 (u & 3), so the
   // difference stays non-negative.
   int kvoff[UPW], vvoff[UPW];
@@ -563,8 +232,8 @@ bsfa_prefill_bs64_2w_kernel(const PrefillParams p) {
   for (int i = 0; i < UPW; ++i) {
     const int byte = (wave * UPW + i) * 1024 + lane * 16;
     const int row = byte / ROWB, pos = (byte % ROWB) / 16;
-    kvoff[i] = (row * (int)p.sk[2] + swz_k<D>(row, pos) * 8) * 2 - (i & 3) * 1024;
-    vvoff[i] = (row * (int)p.sv[2] + swz_v<D>(row, pos) * 8) * 2 - (i & 3) * 1024;
+    kvoff[i] = (row * (int)p.sk[2] + swz_k<D>(row, pos) * 8) * 2 - (i & 3) * LOW;
+    vvoff[i] = (row * (int)p.sv[2] + swz_v<D>(row, pos) * 8) * 2 - (i & 3) * LOW;
   }
   const int grp16 = lane >> 4, t16 = lane & 15;  // ds_read_tr group and lane in group
   const int tr_row = t16 >> 2;                   // source row offset within a 4-row run
@@ -601,20 +270,23 @@ bsfa_prefill_bs64_2w_kernel(const PrefillParams p) {
     for (int i = 0; i < UPW; ++i) {
       const int byte = (wave * UPW + i) * 1024 + lane * 16;
       const int row = byte / ROWB, pos = (byte % ROWB) / 16;
-      qvoff[i] = (row * (int)p.sq[2] + swz_k<D>(row, pos) * 8) * 2 - (i & 3) * 1024;
+      qvoff[i] = (row * (int)p.sq[2] + swz_k<D>(row, pos) * 8) * 2 - (i & 3) * LOW;
     }
-    dma_tile_2w<D, 2>(vS, tile_rsrc(qbase + (int64_t)qb * BS * p.sq[2], (int64_t)(S - qb * BS) * p.sq[2] * 2),
+    dma_tile_2w<D, 2>(vS, tile_rsrc(qbase + (int64_t)qb * BS * p.sq[2],
+                                    (int64_t)(S - qb * BS) * p.sq[2] * 2 + (D == 64 ? ROWB - p.sq[2] * 2 : 0)),
                       qvoff, wave);
   }
-  // Buffer resource of key block kb of K or V (rows >= S are out of range: zeros).
+  // Buffer resource of key block kb of K or V (rows >= S are out of range: zeros). At D=64 it
+  // ends exactly with row S-1, also when rows overlap (token strides below D).
   auto block_rsrc = [&](const uint16_t* base, uint32_t rb, int64_t stride, int kb) {
     if (p.small_spans) {
       const uint32_t key0 = (uint32_t)kb * BS, left = (uint32_t)S - key0;
       return __builtin_amdgcn_make_buffer_rsrc((void*)((const uint8_t*)base + key0 * rb), (short)0,
-                                               (int)(left * rb), 0x00020000);
+                                               (int)(left * rb + (D == 64 ? ROWB - rb : 0u)), 0x00020000);
     }
     const int key0 = kb * BS;
-    return tile_rsrc(base + (int64_t)key0 * stride, (int64_t)(S - key0) * stride * 2);
+    return tile_rsrc(base + (int64_t)key0 * stride,
+                     (int64_t)(S - key0) * stride * 2 + (D == 64 ? ROWB - stride * 2 : 0));
   };
 
   f32x16_t oacc[DTILES];
@@ -629,7 +301,7 @@ bsfa_prefill_bs64_2w_kernel(const PrefillParams p) {
   u32x4_t qf[KSTEPS];
   if (kb >= 0) {
     dma_tile_2w<D>(kS, block_rsrc(kbase, krb, p.sk[2], kb), kvoff, wave);
-    __builtin_amdgcn_s_waitcnt(0x0f78);  // vmcnt(8): own share of Q landed, K in flight
+    __builtin_amdgcn_s_waitcnt(kWaitTile);  // own share of Q landed, K in flight
   } else {
     __builtin_amdgcn_s_waitcnt(0x0f70);  // vmcnt(0)
   }
@@ -639,6 +311,12 @@ bsfa_prefill_bs64_2w_kernel(const PrefillParams p) {
 #pragma unroll
     for (int ks = 0; ks < KSTEPS; ++ks)
       qf[ks] = *(const u32x4_t*)(vS + r * ROWB + swz_k<D>(r, ks * 2 + half) * 16);
+  }
+  if (D == 64 && !p.small_q) {
+    // Token strides the DMA's 32-bit offsets do not cover: the rows again, from memory.
+    const uint16_t* qr = qbase + (int64_t)min(qrow, S - 1) * p.sq[2] + half * 8;
+#pragma unroll
+    for (int ks = 0; ks < KSTEPS; ++ks) qf[ks] = *(const u32x4_t*)(qr + ks * 16);
   }
 
   while (kb >= 0) {
@@ -662,7 +340,7 @@ bsfa_prefill_bs64_2w_kernel(const PrefillParams p) {
     __builtin_amdgcn_s_waitcnt(0xc07f);  // lgkmcnt(0): this wave's K reads returned
     block_barrier();                      // every wave has read K(kb): the K tile is free
     const int kb_next = next_active_block(mrow, p.sm[3], kb_end, lane, chunk, bits, p.mshift);
-    // Always eight DMA units after V(kb) (the last block of a row loads its own K tile
+    // Always one K tile's DMA units after V(kb) (the last block of a row loads its own K tile
     // again), so the V wait below is one fixed count.
     dma_tile_2w<D>(kS, block_rsrc(kbase, krb, p.sk[2], kb_next >= 0 ? kb_next : kb), kvoff, wave);
     if (kb >= mask_from) {
@@ -688,7 +366,7 @@ bsfa_prefill_bs64_2w_kernel(const PrefillParams p) {
     }
     const float mraw = fmaxf(fmaxf(ma, s0[15]), fmaxf(mb, s1[15]));
     const float mloc = pair_max32(mraw) * p.scale_log2;
-    const bool move = mloc > m_ref + kRescaleLog2;
+    const bool move = mloc > m_ref + kMove;
     if (__ballot(move)) {
       // exp2(-inf) = 0 clears the (empty) accumulators on a row's first finite score.
       const float alpha = move ? __builtin_amdgcn_exp2f(m_ref - mloc) : 1.f;
@@ -720,7 +398,7 @@ bsfa_prefill_bs64_2w_kernel(const PrefillParams p) {
                          pack16x2<DT>(sv[o + 4], sv[o + 5]), pack16x2<DT>(sv[o + 6], sv[o + 7])};
       pb[pp] = w;
     }
-    __builtin_amdgcn_s_waitcnt(0x0f78);  // vmcnt(8): own share of V(kb) landed, next K in flight
+    __builtin_amdgcn_s_waitcnt(kWaitTile);  // own share of V(kb) landed, next K in flight
     block_barrier();                      // V(kb) visible
     u32x2_t vlo[4][DTILES], vhi[4][DTILES];
 #pragma unroll
@@ -761,14 +439,14 @@ bsfa_prefill_bs64_2w_kernel(const PrefillParams p) {
       const int d0 = dt * 32 + 8 * gq + 4 * half;
       const u32x2_t w = {pack16x2<DT>(oacc[dt][4 * gq + 0] * inv, oacc[dt][4 * gq + 1] * inv),
                          pack16x2<DT>(oacc[dt][4 * gq + 2] * inv, oacc[dt][4 * gq + 3] * inv)};
-      *(u32x2_t*)(ost + col * ROWB + (((d0 >> 3) ^ (col & 15)) << 4) + (d0 & 7) * 2) = w;
+      *(u32x2_t*)(ost + col * ROWB + (((d0 >> 3) ^ (col & (ROWB / 16 - 1))) << 4) + (d0 & 7) * 2) = w;
     }
   constexpr int CPR = ROWB / 16;  // 16-byte chunks per row
   const int row0 = qb * BS + wave * 32;
 #pragma unroll
   for (int j = 0; j < 32 * CPR / kWave; ++j) {
     const int r = j * (kWave / CPR) + lane / CPR, c = lane % CPR;
-    const u32x4_t v = *(const u32x4_t*)(ost + r * ROWB + ((c ^ (r & 15)) << 4));
+    const u32x4_t v = *(const u32x4_t*)(ost + r * ROWB + ((c ^ (r & (CPR - 1))) << 4));
     // Non-temporal: the output is not read again here, and K/V stay in L2.
     if (row0 + r < S) __builtin_nontemporal_store(v, (u32x4_t*)(obase + (int64_t)(row0 + r) * p.so[2] + c * 8));
   }
@@ -1085,60 +763,17 @@ static hipError_t launch_prefill_bs32(const PrefillParams& p, hipStream_t stream
   return hipGetLastError();
 }
 
-// Compute units of the current device (cached per device).
-static int device_cus() {
-  static int cached[64] = {0};
-  int dev = 0;
-  if (hipGetDevice(&dev) != hipSuccess || dev < 0 || dev >= 64) return 256;
-  if (cached[dev] == 0) {
-    int n = 0;
-    if (hipDeviceGetAttribute(&n, hipDeviceAttributeMultiprocessorCount, dev) != hipSuccess || n <= 0)
-      n = 256;
-    cached[dev] = n;
-  }
-  return cached[dev];
-}
-
-// Resident workgroups per CU of a kernel (at least 1).
-template <typename K>
-static int resident_per_cu(K kernel, int threads) {
-  int n = 0;
-  if (hipOccupancyMaxActiveBlocksPerMultiprocessor(&n, kernel, threads, 0) != hipSuccess || n <= 0) n = 1;
-  return n;
-}
-
 template <int D, int DT>
-static hipError_t launch_prefill_bs64(PrefillParams p, int* queue, hipStream_t stream) {
-  const int64_t total = (int64_t)p.NB * p.B * p.Hq;
-  int64_t grid = total;
-  // Head dim 128 runs the two-wave kernel, one workgroup per item (measured faster than
-  // the persistent ticket loop with four such workgroups per CU); head dim 64 runs the
-  // four-wave one, persistent when the caller passes a workspace.
-  constexpr bool two_wave = D == 128;
-  constexpr int threads = two_wave ? 128 : 256;
-  if constexpr (two_wave) {
-    hipLaunchKernelGGL((bsfa_prefill_bs64_2w_kernel<D, DT>), dim3((unsigned)grid), dim3(threads), 0, stream, p);
-  } else {
-    if (queue) {
-      // Every resident workgroup slot filled once, a whole number per partition.
-      p.parts = (((int64_t)p.B * p.Hkv) % 8 == 0) ? 8 : 1;
-      static const int per_cu = resident_per_cu(bsfa_prefill_bs64_kernel<D, DT>, threads);
-      int64_t wg = std::min<int64_t>(total, (int64_t)per_cu * device_cus());
-      wg = std::max<int64_t>(p.parts, wg / p.parts * p.parts);
-      p.wg_per_part = (int)(wg / p.parts);
-      p.queue = queue;
-      grid = wg;
-      hipLaunchKernelGGL(bsfa_queue_reset_kernel, dim3(1), dim3(64), 0, stream, queue);
-    }
-    hipLaunchKernelGGL((bsfa_prefill_bs64_kernel<D, DT>), dim3((unsigned)grid), dim3(threads), 0, stream, p);
-  }
+static hipError_t launch_prefill_bs64(const PrefillParams& p, hipStream_t stream) {
+  const int64_t grid = (int64_t)p.NB * p.B * p.Hq;
+  hipLaunchKernelGGL((bsfa_prefill_bs64_2w_kernel<D, DT>), dim3((unsigned)grid), dim3(128), 0, stream, p);
   return hipGetLastError();
 }
 
 static bool aligned16(const void* ptr) { return ((uintptr_t)ptr & 15u) == 0; }
 
 template <int DT>
-static hipError_t launch_prefill_any(const PrefillParams& p, int* queue, int64_t head_dim,
+static hipError_t launch_prefill_any(const PrefillParams& p, int64_t head_dim,
                                      int64_t block_size, hipStream_t s) {
   if (block_size == 128 && (head_dim == 128 || head_dim == 64)) {
     // A block-128 mask on the block-64 kernels: each 128-token block is its four 64-token
@@ -1148,11 +783,11 @@ static hipError_t launch_prefill_any(const PrefillParams& p, int* queue, int64_t
     PrefillParams q = p;
     q.mshift = 1;
     q.NB = (p.S + 63) / 64;
-    return head_dim == 128 ? launch_prefill_bs64<128, DT>(q, queue, s)
-                           : launch_prefill_bs64<64, DT>(q, queue, s);
+    return head_dim == 128 ? launch_prefill_bs64<128, DT>(q, s)
+                           : launch_prefill_bs64<64, DT>(q, s);
   }
-  if (block_size == 64 && head_dim == 128) return launch_prefill_bs64<128, DT>(p, queue, s);
-  if (block_size == 64 && head_dim == 64) return launch_prefill_bs64<64, DT>(p, queue, s);
+  if (block_size == 64 && head_dim == 128) return launch_prefill_bs64<128, DT>(p, s);
+  if (block_size == 64 && head_dim == 64) return launch_prefill_bs64<64, DT>(p, s);
   if (head_dim == 128) return launch_prefill_bs32<128, 1, DT>(p, s);  // block 32
   return launch_prefill_bs32<64, 2, DT>(p, s);
 }
@@ -1161,10 +796,10 @@ static hipError_t launch_prefill_any(const PrefillParams& p, int* queue, int64_t
 
 using namespace tasft;
 
-static int dispatch_prefill(const PrefillParams& p, int* queue, int64_t head_dim,
+static int dispatch_prefill(const PrefillParams& p, int64_t head_dim,
                             int64_t block_size, int dtype, hipStream_t s, const char* what) {
-  const hipError_t err = dtype == kF16 ? launch_prefill_any<kF16>(p, queue, head_dim, block_size, s)
-                                       : launch_prefill_any<kBf16>(p, queue, head_dim, block_size, s);
+  const hipError_t err = dtype == kF16 ? launch_prefill_any<kF16>(p, head_dim, block_size, s)
+                                       : launch_prefill_any<kBf16>(p, head_dim, block_size, s);
   if (err != hipSuccess)
     return set_error(kErrLaunch, "%s: launch failed: %s", what, hipGetErrorString(err));
   return kOk;
@@ -1173,7 +808,7 @@ static int dispatch_prefill(const PrefillParams& p, int* queue, int64_t head_dim
 extern "C" size_t tasft_bsfa_prefill_workspace_bytes(int64_t batch, int64_t num_q_heads,
                                                      int64_t seq_len, int64_t block_size) {
   if (batch <= 0 || num_q_heads <= 0 || seq_len <= 0 || block_size <= 0) return 0;
-  return 256;  // the persistent launch's ticket counters
+  return 256;  // kept for callers that pass one; no kernel uses it
 }
 
 extern "C" int tasft_bsfa_prefill_fwd(const void* q, const void* k, const void* v, void* out,
@@ -1255,13 +890,9 @@ extern "C" int tasft_bsfa_prefill_fwd(const void* q, const void* k, const void* 
   p.small_spans = (seq_len * k_strides[2] * 2 < 0x7fffffffLL &&
                    seq_len * v_strides[2] * 2 < 0x7fffffffLL) ? 1 : 0;
   p.small_q = seq_len * q_strides[2] * 2 < 0x7fffffffLL ? 1 : 0;
-  p.queue = nullptr;
-  p.parts = 1;
-  p.wg_per_part = 1;
   p.cu_seqlens = nullptr;
   p.mshift = 0;
-  // Ticket counters of the persistent launch (block size 64).
-  return dispatch_prefill(p, (int*)workspace, head_dim, block_size, dtype, (hipStream_t)stream,
+  return dispatch_prefill(p, head_dim, block_size, dtype, (hipStream_t)stream,
                           "prefill");
 }
 
@@ -1389,12 +1020,8 @@ extern "C" int tasft_bsfa_prefill_varlen_fwd(const void* q, const void* k, const
   p.small_spans = (max_seqlen * k_strides[0] * 2 < 0x7fffffffLL &&
                    max_seqlen * v_strides[0] * 2 < 0x7fffffffLL) ? 1 : 0;
   p.small_q = max_seqlen * q_strides[0] * 2 < 0x7fffffffLL ? 1 : 0;
-  p.queue = nullptr;
-  p.parts = 1;
-  p.wg_per_part = 1;
   p.cu_seqlens = cu_seqlens;
   p.mshift = 0;
-  // One workgroup per (sequence, head, query block); never the persistent loop.
-  return dispatch_prefill(p, nullptr, head_dim, block_size, dtype, (hipStream_t)stream,
+  return dispatch_prefill(p, head_dim, block_size, dtype, (hipStream_t)stream,
                           "prefill_varlen");
 }

@@ -252,14 +252,9 @@ class BlockSparseFlashAttention:
         mask = _mask_bytes(block_mask if block_mask.device == q.device else block_mask.to(q.device))
         out = torch.empty((B, H, S, D), dtype=q.dtype, device=q.device)
         scale = 1.0 / math.sqrt(D)
-        workspace, ws_bytes = None, 0
-        if D == 64 and self.block_size != 32:
-            # Work-queue counters of the persistent launch.
-            ws_bytes = lib.tasft_bsfa_prefill_workspace_bytes(B, H, S, self.block_size)
-            workspace = torch.empty(ws_bytes, dtype=torch.uint8, device=q.device)
         status = lib.tasft_bsfa_prefill_fwd(
             q.data_ptr(), k.data_ptr(), v.data_ptr(), out.data_ptr(), mask.data_ptr(),
-            _native.ptr(workspace), ws_bytes, B, H, k.shape[1], S, D, self.block_size,
+            None, 0, B, H, k.shape[1], S, D, self.block_size,
             _native.strides(q), _native.strides(k), _native.strides(v), _native.strides(out),
             _native.strides(mask), scale, 1 if causal else 0, dtype, _native.stream_handle(q.device),
         )
