@@ -202,8 +202,15 @@ __device__ __forceinline__ void dma_tile_2w(uint8_t* tile, __amdgpu_buffer_rsrc_
   }
 }
 
-template <int D, int DT>
-__global__ void __launch_bounds__(128) __attribute__((amdgpu_waves_per_eu(D == 64 ? 3 : 2, D == 64 ? 3 : 2)))
+// PAIRS = 2 (few rows): such a launch is as long as its longest row, a chain of steps of one
+// pair of waves. A second pair takes every other active block, with tiles of its own, and the
+// pairs' (max, sum, output) meet in LDS after the row. Both pairs meet the same barriers; on
+// an odd last block the second pair runs an empty one (zero K and V, all keys masked). One
+// pair against two, D=128, 32/8 heads, a fifth of the blocks: S=1024 13.5 to 12.6 us; 8/2
+// heads, S=4096 31.4 to 23.7 us, half of the blocks 63.7 to 42.8 us; D=64, 32/8 heads, S=1024
+// 12.2 to 9.9 us.
+template <int D, int DT, int PAIRS>
+__global__ void __launch_bounds__(128 * PAIRS) __attribute__((amdgpu_waves_per_eu(D == 64 ? 3 : 2, D == 64 ? 3 : 2)))
 bsfa_prefill_bs64_2w_kernel(const PrefillParams p) {
   constexpr int BS = 64;
   constexpr int KSTEPS = D / 16;
@@ -215,11 +222,15 @@ bsfa_prefill_bs64_2w_kernel(const PrefillParams p) {
   constexpr float kMove = D == 128 ? kRescaleLog2 : kRescale64Log2;
   constexpr int LOW = D == 128 ? 1024 : 0;  // what dma_tile_2w's instruction offsets add per unit
 
-  __shared__ __attribute__((aligned(1024))) uint8_t kS[TILE];
-  __shared__ __attribute__((aligned(1024))) uint8_t vS[TILE];
+  __shared__ __attribute__((aligned(1024))) uint8_t k_lds[PAIRS * TILE];
+  __shared__ __attribute__((aligned(1024))) uint8_t v_lds[PAIRS * TILE];
 
   const int lane = threadIdx.x & 63;
-  const int wave = __builtin_amdgcn_readfirstlane(threadIdx.x >> 6);  // uniform: scalar DMA addresses
+  const int wave4 = __builtin_amdgcn_readfirstlane(threadIdx.x >> 6);  // uniform: scalar DMA addresses
+  const int wave = PAIRS == 1 ? wave4 : wave4 & 1;  // row half
+  const int pair = PAIRS == 1 ? 0 : wave4 >> 1;
+  uint8_t* const kS = k_lds + pair * TILE;
+  uint8_t* const vS = v_lds + pair * TILE;
   const int col = lane & 31;
   const int half = lane >> 5;
 
@@ -246,7 +257,6 @@ bsfa_prefill_bs64_2w_kernel(const PrefillParams p) {
   const SeqSpan span = seq_span<BS>(p, b);
   if (qb >= span.NB) return;
   const int S = span.S, NB = span.NB;
-
 
   const uint16_t* qbase = p.q + b * p.sq[0] + span.tok0 * p.sq[2] + h * p.sq[1];
   const uint16_t* kbase = p.k + b * p.sk[0] + span.tok0 * p.sk[2] + kvh * p.sk[1];
@@ -279,6 +289,8 @@ bsfa_prefill_bs64_2w_kernel(const PrefillParams p) {
   // Buffer resource of key block kb of K or V (rows >= S are out of range: zeros). At D=64 it
   // ends exactly with row S-1, also when rows overlap (token strides below D).
   auto block_rsrc = [&](const uint16_t* base, uint32_t rb, int64_t stride, int kb) {
+    if (PAIRS > 1 && kb < 0)  // the empty block: no rows, all zeros
+      return __builtin_amdgcn_make_buffer_rsrc((void*)base, (short)0, 0, 0x00020000);
     if (p.small_spans) {
       const uint32_t key0 = (uint32_t)kb * BS, left = (uint32_t)S - key0;
       return __builtin_amdgcn_make_buffer_rsrc((void*)((const uint8_t*)base + key0 * rb), (short)0,
@@ -297,9 +309,20 @@ bsfa_prefill_bs64_2w_kernel(const PrefillParams p) {
 
   int chunk = 0;
   uint64_t bits = __ballot(mb != 0);
-  int kb = next_active_block(mrow, p.sm[3], kb_end, lane, chunk, bits, p.mshift);
+  // The next active block, or with two pairs the next two: the first in `lead`, this pair's
+  // (-1: none) returned.
+  int lead = 0;
+  auto next_block = [&]() {
+    const int first = next_active_block(mrow, p.sm[3], kb_end, lane, chunk, bits, p.mshift);
+    lead = first;
+    if constexpr (PAIRS == 1) return first;
+    const int second =
+        first >= 0 ? next_active_block(mrow, p.sm[3], kb_end, lane, chunk, bits, p.mshift) : -1;
+    return pair == 0 ? first : second;
+  };
+  int kb = next_block();
   u32x4_t qf[KSTEPS];
-  if (kb >= 0) {
+  if (lead >= 0) {
     dma_tile_2w<D>(kS, block_rsrc(kbase, krb, p.sk[2], kb), kvoff, wave);
     __builtin_amdgcn_s_waitcnt(kWaitTile);  // own share of Q landed, K in flight
   } else {
@@ -319,7 +342,7 @@ bsfa_prefill_bs64_2w_kernel(const PrefillParams p) {
     for (int ks = 0; ks < KSTEPS; ++ks) qf[ks] = *(const u32x4_t*)(qr + ks * 16);
   }
 
-  while (kb >= 0) {
+  while (lead >= 0) {
     __builtin_amdgcn_s_waitcnt(0x0070);  // vmcnt(0) lgkmcnt(0): own share of K(kb) landed
     block_barrier();                      // K(kb) visible; every wave is done with the V tile
     dma_tile_2w<D>(vS, block_rsrc(vbase, vrb, p.sv[2], kb), vvoff, wave);
@@ -339,16 +362,17 @@ bsfa_prefill_bs64_2w_kernel(const PrefillParams p) {
     }
     __builtin_amdgcn_s_waitcnt(0xc07f);  // lgkmcnt(0): this wave's K reads returned
     block_barrier();                      // every wave has read K(kb): the K tile is free
-    const int kb_next = next_active_block(mrow, p.sm[3], kb_end, lane, chunk, bits, p.mshift);
+    const int kb_next = next_block();
     // Always one K tile's DMA units after V(kb) (the last block of a row loads its own K tile
     // again), so the V wait below is one fixed count.
-    dma_tile_2w<D>(kS, block_rsrc(kbase, krb, p.sk[2], kb_next >= 0 ? kb_next : kb), kvoff, wave);
-    if (kb >= mask_from) {
+    dma_tile_2w<D>(kS, block_rsrc(kbase, krb, p.sk[2], lead >= 0 ? kb_next : kb), kvoff, wave);
+    const bool empty = PAIRS > 1 && kb < 0;
+    if (empty || kb >= mask_from) {
       // Register rr of tile t holds key kb*BS + 32t + 4*half + off(rr), off = 8*(rr/4) +
       // rr%4; a key is admissible iff it is <= min(qrow, S-1) (causal) or S-1, i.e. iff
       // 32t + off <= lim below: one compare per score.
       const int last = p.causal ? min(qrow, S - 1) : S - 1;
-      const int lim = last - kb * BS - 4 * half;
+      const int lim = empty ? -1 : last - kb * BS - 4 * half;
 #pragma unroll
       for (int rr = 0; rr < 16; ++rr) {
         const int off = 8 * (rr >> 2) + (rr & 3);
@@ -424,13 +448,44 @@ bsfa_prefill_bs64_2w_kernel(const PrefillParams p) {
   }
   __builtin_amdgcn_s_waitcnt(0x0f70);  // no DMA into this workgroup's LDS outlives it
 
-  const float l_tot = pair_sum32(l_run);
+  float l_tot = pair_sum32(l_run);
+  if constexpr (PAIRS > 1) {
+    // The second pair's sums through its own K and V tiles (16 DTILES x 64 floats per wave).
+    static_assert(DTILES * 16 * kWave * 4 == TILE, "merge buffers");
+    __shared__ float x_m[2][kWave], x_l[2][kWave];
+    float* xo = (float*)(wave == 0 ? k_lds + TILE : v_lds + TILE);
+    __builtin_amdgcn_s_waitcnt(0xc07f);  // lgkmcnt(0): this wave's V reads returned
+    block_barrier();                      // every wave is done with the tiles
+    if (pair == 1) {
+#pragma unroll
+      for (int dt = 0; dt < DTILES; ++dt)
+#pragma unroll
+        for (int rr = 0; rr < 16; ++rr) xo[(dt * 16 + rr) * kWave + lane] = oacc[dt][rr];
+      x_m[wave][lane] = m_ref;
+      x_l[wave][lane] = l_tot;
+    }
+    __builtin_amdgcn_s_waitcnt(0xc07f);  // lgkmcnt(0): the stores above are in LDS
+    block_barrier();
+    if (pair == 1) return;
+    const float m1 = x_m[wave][lane], l1 = x_l[wave][lane];
+    const float m = fmaxf(m_ref, m1);
+    const float mu = (m == -INFINITY) ? 0.f : m;
+    const float f0 = __builtin_amdgcn_exp2f(m_ref - mu), f1 = __builtin_amdgcn_exp2f(m1 - mu);
+    l_tot = l_tot * f0 + l1 * f1;
+#pragma unroll
+    for (int dt = 0; dt < DTILES; ++dt)
+#pragma unroll
+      for (int rr = 0; rr < 16; ++rr)
+        oacc[dt][rr] = oacc[dt][rr] * f0 + xo[(dt * 16 + rr) * kWave + lane] * f1;
+  }
   const float inv = 1.f / (l_tot > 0.f ? l_tot : 1.f);  // empty rows: O = 0; NaN rows stay NaN
   // The output through LDS: each wave writes its 32 rows into its own 8 KB of the V tile
   // (16-byte chunk c of row r at position c ^ (r & 15)), then stores whole 256-byte rows,
   // four rows per instruction.
-  __builtin_amdgcn_s_waitcnt(0xc07f);  // lgkmcnt(0): this wave's V reads returned
-  block_barrier();                      // every wave is done with the V tile
+  if constexpr (PAIRS == 1) {
+    __builtin_amdgcn_s_waitcnt(0xc07f);  // lgkmcnt(0): this wave's V reads returned
+    block_barrier();                      // every wave is done with the V tile
+  }
   uint8_t* ost = vS + wave * (32 * ROWB);
 #pragma unroll
   for (int dt = 0; dt < DTILES; ++dt)
@@ -766,7 +821,14 @@ static hipError_t launch_prefill_bs32(const PrefillParams& p, hipStream_t stream
 template <int D, int DT>
 static hipError_t launch_prefill_bs64(const PrefillParams& p, hipStream_t stream) {
   const int64_t grid = (int64_t)p.NB * p.B * p.Hq;
-  hipLaunchKernelGGL((bsfa_prefill_bs64_2w_kernel<D, DT>), dim3((unsigned)grid), dim3(128), 0, stream, p);
+  // Two pairs of waves per row fill the card with two workgroups per CU (registers), 512 rows;
+  // with more, rows wait for a second fill (640 rows 16.8 us against 15.6, S=2048 with 1024
+  // rows 24.1 against 22.7), and rows of fewer than 8 blocks have nothing to share out
+  // (S=256 8.8 us against 8.4, S=512 10.7 against 11.6).
+  if (grid <= 512 && p.NB >= 8)
+    hipLaunchKernelGGL((bsfa_prefill_bs64_2w_kernel<D, DT, 2>), dim3((unsigned)grid), dim3(256), 0, stream, p);
+  else
+    hipLaunchKernelGGL((bsfa_prefill_bs64_2w_kernel<D, DT, 1>), dim3((unsigned)grid), dim3(128), 0, stream, p);
   return hipGetLastError();
 }
 
