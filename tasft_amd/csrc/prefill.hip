@@ -821,11 +821,14 @@ static hipError_t launch_prefill_bs32(const PrefillParams& p, hipStream_t stream
 template <int D, int DT>
 static hipError_t launch_prefill_bs64(const PrefillParams& p, hipStream_t stream) {
   const int64_t grid = (int64_t)p.NB * p.B * p.Hq;
-  // Two pairs of waves per row fill the card with two workgroups per CU (registers), 512 rows;
-  // with more, rows wait for a second fill (640 rows 16.8 us against 15.6, S=2048 with 1024
-  // rows 24.1 against 22.7), and rows of fewer than 8 blocks have nothing to share out
-  // (S=256 8.8 us against 8.4, S=512 10.7 against 11.6).
-  if (grid <= 512 && p.NB >= 8)
+  // Two pairs of waves per row fill the card with two workgroups per CU at head dim 128, 512
+  // rows; with more, rows wait for a second fill (640 rows of S=1280 16.8 us against 15.6,
+  // 1024 of S=2048 24.1 against 22.7; rows of 80 blocks and more still gain, up to 1024 of
+  // them and not with few active blocks). At head dim 64 three fit, and up to 1024 rows it is
+  // no slower (S=2048 16.4 us both, S=4096 23.2 against 27.5; 1536 rows of S=6144 with few
+  // active blocks 22.5 against 21.6). Rows of fewer than 8 blocks have nothing to share out
+  // (D=128, S=256 8.8 us against 8.4, S=512 10.7 against 11.6).
+  if (grid <= (D == 128 ? 512 : 1024) && p.NB >= 8)
     hipLaunchKernelGGL((bsfa_prefill_bs64_2w_kernel<D, DT, 2>), dim3((unsigned)grid), dim3(256), 0, stream, p);
   else
     hipLaunchKernelGGL((bsfa_prefill_bs64_2w_kernel<D, DT, 1>), dim3((unsigned)grid), dim3(128), 0, stream, p);

@@ -17,9 +17,11 @@ pytestmark = pytest.mark.gpu
 @pytest.mark.parametrize(("S", "Hq", "Hkv", "D", "bs", "causal"), [
     (448, 4, 2, 128, 64, True),      # 7 blocks: one pair
     (449, 4, 2, 128, 64, False),     # 8 blocks, one key in the last
-    (1024, 32, 8, 64, 64, True),     # 512 rows
-    (1025, 32, 8, 64, 64, True),     # 544 rows: one pair
-    (1000, 32, 8, 128, 64, True),
+    (1024, 32, 8, 128, 64, True),    # 512 rows
+    (1025, 32, 8, 128, 64, True),    # 544 rows: one pair
+    (2048, 32, 8, 64, 64, True),     # 1024 rows
+    (2049, 32, 8, 64, 64, True),     # 1056 rows: one pair
+    (1000, 32, 8, 64, 64, True),
     (4500, 2, 1, 128, 64, True),     # more than 64 key blocks per row
     (4200, 3, 3, 64, 128, False),
 ])
