@@ -732,7 +732,7 @@ __device__ __forceinline__ void pair_chunk64(const GatePairParams& q, int64_t bh
 // counter with a relaxed agent-scope atomic. Thread 0 of a query workgroup polls the
 // counter with relaxed agent-scope loads (device-level reads) and s_sleep, then runs one
 // agent-scope acquire fence (this CU's L1 and the XCD's L2 invalidated) before the barrier
-// that releases every thread's unit reads. Measured on the box with a bounded probe: a
+// that releases every thread's unit reads. Measured with a bounded probe: a
 // counter raised on one XCD is seen by pollers on all eight, and the data published with it
 // reads back exactly.
 //
