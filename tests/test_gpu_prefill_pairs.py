@@ -2,11 +2,12 @@
 blocks, rows with one block or none, ragged ends, and both sides of the rule that chooses it."""
 from __future__ import annotations
 
+import numpy as np
 import pytest
 import torch
 
 import attn_inputs as ai
-from helpers import assert_close_bf16, require_gpu, to_np
+from helpers import assert_close_bf16, bar, require_gpu, to_np
 from oracle import tasft_oracle as orc
 from tasft_amd.kernels import BlockSparseFlashAttention
 
@@ -39,3 +40,25 @@ def test_few_rows(S, Hq, Hkv, D, bs, causal, kind):
     torch.cuda.synchronize()
     ref = orc.attention_block_gather(to_np(q), to_np(k), to_np(v), mask.numpy(), bs, causal)
     assert_close_bf16(out, ref, f"prefill pairs S={S} D={D} block {bs} {kind}")
+
+
+@pytest.mark.parametrize("dtype", [torch.bfloat16, torch.float16])
+@pytest.mark.parametrize(("S", "D"), [(440, 128), (512, 128), (440, 64), (512, 64)])  # one pair, two pairs
+def test_nan_pattern(S, D, dtype):
+    """A NaN in Q, K or V reaches the same outputs as in the oracle, whichever pair meets it."""
+    dev = require_gpu()
+    Hq, Hkv, nb = 4, 2, -(-S // 64)
+    print(f"prefill pairs NaN S={S} D={D} {dtype}", flush=True)
+    q, k, v = (t.float().to(dtype) for t in ai.qkv("unit", (1, Hq, S, D), (1, Hkv, S, D), 31 + S + D, 64))
+    q[0, 0, 300, 5] = float("nan")
+    k[0, 1, 130, 1] = float("nan")
+    v[0, 0, 70, D - 1] = float("nan")
+    mask = torch.rand(1, Hq, nb, nb, generator=torch.Generator().manual_seed(S)) < 0.5
+    ref = orc.attention_block_gather(to_np(q), to_np(k), to_np(v), mask.numpy(), 64, True)
+    assert np.isnan(ref).any() and not np.isnan(ref).all()
+    out = BlockSparseFlashAttention(block_size=64, min_sparsity_for_speedup=0.0).forward(
+        q.to(dev), k.to(dev), v.to(dev), mask.to(dev), causal=True)
+    torch.cuda.synchronize()
+    got, clean = to_np(out), ~np.isnan(ref)
+    np.testing.assert_array_equal(np.isnan(got), ~clean)
+    assert_close_bf16(np.where(clean, got, 0.0), np.where(clean, ref, 0.0), f"NaN S={S} D={D}", **bar(dtype))
