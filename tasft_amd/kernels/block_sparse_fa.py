@@ -686,11 +686,13 @@ def default_decode_splits(batch: int, num_kv_heads: int, num_blocks: int,
                           q_per_kv: int = 1) -> int:
     """Split-K factor giving about one decode workgroup per CU (256 on MI355X), for every
     head count up to 16 query heads per KV head. Two workgroups fit per CU, but one per CU
-    measured fastest: at B=8 with 28/4 heads 8 splits took 20.8 us against 24.6 us for 16,
-    at B=8 with 32/8 heads 4 splits took 25.7 us against 27.5 us for 8, and at B=64 with
-    28/4 heads one split took 65.8 us against 70.9 us for two. Fewer splits also mean
-    fewer blocks scanned twice and, at one split, no combine pass. Never fewer than the
-    splits that keep every split within 1024 key blocks."""
+    is the fastest count or within 7% of it, merge included, over 1 to 32 splits: at B=8,
+    S=8192 with 28/4 heads 8 splits take 23.2 us (4: 27.6, 16: 23.5), with 32/8 heads 4 take
+    27.1 us (2: 32.7, 8: 25.3); at B=16, S=4096, 32/8 heads 2 take 28.6 us (1: 29.2, 4: 26.7,
+    8: 29.3); at B=2, S=2048 16 take 11.2 us (8: 12.4, 32: 12.1); at B=64 with 28/4 heads one
+    split takes 65.8 us (2: 70.9). Fewer splits also mean fewer blocks scanned twice and, at
+    one split, no combine pass. Never fewer than the splits that keep every split within
+    1024 key blocks."""
     del q_per_kv  # the kernel's occupancy does not depend on the head count
     groups = max(1, batch * num_kv_heads)
     resident = 256
