@@ -20,6 +20,7 @@ import math
 
 import torch
 import torch.nn.functional as F
+from torch.autograd.function import once_differentiable
 
 from tasft_amd import _native
 from tasft_amd.exceptions import KernelError, NaNDetectedError
@@ -251,6 +252,7 @@ class _GateKL(torch.autograd.Function):
         return loss
 
     @staticmethod
+    @once_differentiable
     def backward(ctx, grad_out: torch.Tensor):
         (grad,) = ctx.saved_tensors
         if grad is None:
