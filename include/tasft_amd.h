@@ -57,7 +57,9 @@ int tasft_abi_version(void);
  * AND j <= i inside the diagonal block when causal) and j < seq_len, else -inf.
  * Rows with no admissible key are 0. P is rounded to `dtype` before the PV product.
  * block_mask: [B, Hq, ceil(S/bs), ceil(S/bs)] bytes, strides in mask_strides (bytes).
- * head_dim in {64, 128}; block_size in {32, 64, 128}; strides of b/h/s multiples of 8.
+ * head_dim in {64, 128}; block_size in {32, 64, 128}; strides of b/h/s multiples of 8; at
+ * head_dim 128 with block_size 64 or 128 the token strides of q, k and v at least 128 (rows
+ * that overlap, such as one row repeated by a stride of 0, are rejected).
  * Block size 128 runs on the block-64 kernels, each 128-token block as its four 64-token
  * quarters (the same tokens attend to the same keys).
  * workspace: NULL, or >= tasft_bsfa_prefill_workspace_bytes(...) bytes, 16-byte aligned; it
@@ -83,7 +85,8 @@ int tasft_bsfa_prefill_fwd(const void* q, const void* k, const void* v, void* ou
  * first token).
  *
  * q, out [T, Hq, D]; k, v [T, Hkv, D] (strides of token, head, dim in elements, dim
- * contiguous, token and head strides multiples of 8). cu_seqlens: device int32
+ * contiguous, token and head strides multiples of 8, token strides otherwise as in
+ * tasft_bsfa_prefill_fwd). cu_seqlens: device int32
  * [num_seqs + 1], cu_seqlens[0] = 0, non-decreasing, every length <= max_seqlen.
  * block_mask: [num_seqs, Hq, NB, NB] bytes with NB = ceil(max_seqlen / bs); sequence n
  * uses its leading ceil(len_n / bs) x ceil(len_n / bs) corner. Lengths are clamped to

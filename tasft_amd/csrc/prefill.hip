@@ -837,6 +837,14 @@ static hipError_t launch_prefill_bs64(const PrefillParams& p, hipStream_t stream
 
 static bool aligned16(const void* ptr) { return ((uintptr_t)ptr & 15u) == 0; }
 
+// At head dim 128 the kernels of blocks 64 and 128 end a tensor's buffer `rows left` token
+// strides after a tile's first row, and their per-lane offsets count on whole rows before
+// each unit: rows closer than the head dim (0: one row repeated) would arrive as zeros.
+static bool rows_overlap(int64_t head_dim, int64_t block_size, int64_t q_token, int64_t k_token,
+                         int64_t v_token) {
+  return head_dim == 128 && block_size != 32 && std::min({q_token, k_token, v_token}) < head_dim;
+}
+
 template <int DT>
 static hipError_t launch_prefill_any(const PrefillParams& p, int64_t head_dim,
                                      int64_t block_size, hipStream_t s) {
@@ -930,6 +938,10 @@ extern "C" int tasft_bsfa_prefill_fwd(const void* q, const void* k, const void* 
     if (((uintptr_t)workspace) & 15u)
       return set_error(kErrInvalidArgument, "prefill: workspace must be 16-byte aligned");
   }
+  if (rows_overlap(head_dim, block_size, q_strides[2], k_strides[2], v_strides[2]))
+    return set_error(kErrInvalidArgument,
+                     "prefill: at head_dim 128 and block_size 64 or 128 the token strides of q, k "
+                     "and v must be at least head_dim");
 
   PrefillParams p;
   p.q = (const uint16_t*)q;
@@ -1058,6 +1070,10 @@ extern "C" int tasft_bsfa_prefill_varlen_fwd(const void* q, const void* k, const
   if (nb * (block_size == 128 ? 2 : 1) * num_seqs * num_q_heads > 0x7fffffffLL ||
       max_seqlen > 0x3fffffffLL)
     return set_error(kErrUnsupported, "prefill_varlen: problem too large for one launch");
+  if (rows_overlap(head_dim, block_size, q_strides[0], k_strides[0], v_strides[0]))
+    return set_error(kErrInvalidArgument,
+                     "prefill_varlen: at head_dim 128 and block_size 64 or 128 the token strides of "
+                     "q, k and v must be at least head_dim");
 
   PrefillParams p;
   p.q = (const uint16_t*)q;

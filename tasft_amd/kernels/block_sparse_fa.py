@@ -100,6 +100,16 @@ def _kernel_ready(t: torch.Tensor) -> torch.Tensor:
     return t if _native.kernel_layout(t) else t.contiguous()
 
 
+def _prefill_ready(t: torch.Tensor, token_dim: int, block_size: int) -> torch.Tensor:
+    """``_kernel_ready`` for the prefill kernels. At head dim 128 those of blocks 64 and 128 read
+    tiles whose rows do not overlap: a token stride below the head dim (0 in an expanded
+    tensor) is copied."""
+    t = _kernel_ready(t)
+    if t.shape[-1] == 128 and block_size != 32 and t.stride(token_dim) < 128:
+        return t.clone(memory_format=torch.contiguous_format)
+    return t
+
+
 def _mask_bytes(mask: torch.Tensor) -> torch.Tensor:
     """One byte per block, non-zero = attend, without a copy for bool masks."""
     if mask.dtype == torch.bool:
@@ -246,9 +256,9 @@ class BlockSparseFlashAttention:
             if t.device != q.device:
                 raise KernelError("Q, K, V must be on the same device", context={"device": str(t.device)})
         lib = _native.load_library()
-        q = _kernel_ready(q)
-        k = _kernel_ready(k)
-        v = _kernel_ready(v)
+        q = _prefill_ready(q, 2, self.block_size)
+        k = _prefill_ready(k, 2, self.block_size)
+        v = _prefill_ready(v, 2, self.block_size)
         mask = _mask_bytes(block_mask if block_mask.device == q.device else block_mask.to(q.device))
         out = torch.empty((B, H, S, D), dtype=q.dtype, device=q.device)
         scale = 1.0 / math.sqrt(D)
@@ -365,9 +375,9 @@ class BlockSparseFlashAttention:
                 raise KernelError("Q, K, V must be on the same GPU device",
                                   context={"tensor": name, "device": str(t.device)})
         lib = _native.load_library()
-        q = _kernel_ready(q)
-        k = _kernel_ready(k)
-        v = _kernel_ready(v)
+        q = _prefill_ready(q, 0, self.block_size)
+        k = _prefill_ready(k, 0, self.block_size)
+        v = _prefill_ready(v, 0, self.block_size)
         mask = _mask_bytes(block_mask if block_mask.device == q.device else block_mask.to(q.device))
         cu_dev = _int32_on(cu_seqlens, q.device)
         out = torch.empty_like(q)

@@ -1,0 +1,43 @@
+"""Token strides below the head dim (one row repeated by a stride of 0, rows that overlap): each
+call equals the one on contiguous copies."""
+from __future__ import annotations
+
+import pytest
+import torch
+
+from helpers import require_gpu
+from tasft_amd import workloads as wl
+from tasft_amd.kernels import BlockSparseFlashAttention
+
+pytestmark = pytest.mark.gpu
+
+
+def _views(heads, S, D, seed, dev):
+    """[1, heads, S, D] of one row a head, and of rows eight elements apart."""
+    row = wl.randn_bf16((1, heads, 1, D), seed, scale=1.0).to(dev).expand(1, heads, S, D)
+    pool = wl.randn_bf16((heads, 8 * S + D), seed + 1, scale=1.0).to(dev)
+    return row, pool.as_strided((1, heads, S, D), (0, pool.stride(0), 8, 1))
+
+
+@pytest.mark.parametrize("D", [64, 128])
+@pytest.mark.parametrize("bs", [32, 64, 128])
+def test_prefill(bs, D):
+    dev = require_gpu()
+    S, Hq, Hkv = 333, 4, 2
+    print(f"prefill token strides block {bs} D={D}", flush=True)
+    q, k, v = (wl.randn_bf16((1, h, S, D), 5 + i, scale=1.0).to(dev) for i, h in enumerate((Hq, Hkv, Hkv)))
+    nb = -(-S // bs)
+    mask = (torch.rand(1, Hq, nb, nb, generator=torch.Generator().manual_seed(bs)) < 0.7).to(dev)
+    mask |= torch.eye(nb, dtype=torch.bool, device=dev)
+    attn = BlockSparseFlashAttention(block_size=bs, min_sparsity_for_speedup=0.0)
+    cu = torch.tensor([0, S - 100, S], device=dev)
+    varlen_mask = mask[..., :nb, :nb].expand(2, Hq, nb, nb)
+    for i in range(3):
+        for view in _views((Hq, Hkv, Hkv)[i], S, D, 20 + i, dev):
+            t = [q, k, v]
+            t[i] = view
+            c = [x.contiguous() for x in t]
+            assert torch.equal(attn.forward(*t, mask, causal=True), attn.forward(*c, mask, causal=True))
+            t, c = ([x[0].transpose(0, 1) for x in y] for y in (t, c))
+            assert torch.equal(attn.forward_varlen(*t, varlen_mask, cu, S),
+                               attn.forward_varlen(*c, varlen_mask, cu, S))

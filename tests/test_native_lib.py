@@ -10,6 +10,7 @@ import re
 from pathlib import Path
 
 import pytest
+import torch
 
 from tasft_amd import _native
 
@@ -179,6 +180,37 @@ def test_negative_strides_are_rejected_before_any_launch():
         assert rc == -1 and b"non-negative" in lib.tasft_last_error(), name
     rc = lib.tasft_mask_compact(fake, 1, 2, 4, 4, neg, 1, fake, fake, 16, fake, 1 << 20, None)
     assert rc == -1 and b"non-negative" in lib.tasft_last_error()
+
+
+@pytest.mark.parametrize("block", [64, 128])
+@pytest.mark.parametrize("which", [0, 1, 2])
+def test_prefill_refuses_overlapping_rows_at_head_dim_128(which, block):
+    """The block-64 kernels' DMA would read such rows as zeros."""
+    lib = _native.load_library()
+    ok4, ok3, mask = _i64([0, 128, 128, 1]), _i64([128, 128, 1]), _i64([0, 0, 0, 1])
+    fake = ctypes.c_void_p(16)
+    for stride in (0, 120):
+        s4, s3 = [ok4] * 3, [ok3] * 3
+        s4[which], s3[which] = _i64([0, 128, stride, 1]), _i64([stride, 128, 1])
+        rc = lib.tasft_bsfa_prefill_fwd(fake, fake, fake, fake, fake, None, 0, 1, 32, 8, 128, 128, block,
+                                        *s4, ok4, mask, 1.0, 1, 0, None)
+        assert rc == -1 and b"at least head_dim" in lib.tasft_last_error()
+        rc = lib.tasft_bsfa_prefill_varlen_fwd(fake, fake, fake, fake, fake, fake, 2, 32, 8, 128, 128,
+                                               block, *s3, ok3, mask, 1.0, 1, 0, None)
+        assert rc == -1 and b"at least head_dim" in lib.tasft_last_error()
+
+
+def test_prefill_copies_overlapping_rows_at_head_dim_128():
+    from tasft_amd.kernels.block_sparse_fa import _prefill_ready
+    t = torch.randn(2, 1, 1, 128).bfloat16().expand(2, 3, 70, 128)
+    c = _prefill_ready(t, 2, 64)
+    assert c.stride(2) == 128 and torch.equal(c, t)
+    assert _prefill_ready(t, 2, 32) is t  # the block-32 kernel reads them in place
+    assert _prefill_ready(t[..., :64], 2, 64).stride(2) == 0  # and so does head dim 64
+    one = torch.randn(4, 128).bfloat16().as_strided((1, 4, 1, 128), (512, 128, 0, 1))
+    assert _prefill_ready(one, 2, 64).stride(2) == 128
+    rows = torch.randn(70, 3, 128).bfloat16().transpose(0, 1)[None]
+    assert _prefill_ready(rows, 2, 64) is rows
 
 
 def test_check_raises_kernel_error_with_message():
