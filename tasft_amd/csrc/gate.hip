@@ -1416,9 +1416,12 @@ extern "C" int tasft_gate_fwd(const void* q, const void* k, const float* w_in, c
 
   hipStream_t s = (hipStream_t)stream;
   hipError_t err;
-  // The streaming pool's 32-bit row offsets reach the end of a chunk's last load group.
+  // The streaming pool's 32-bit row offsets reach the end of a chunk's last load group, and its
+  // buffer ends `rows left` token strides after the chunk's first row: rows closer than the head
+  // dim (0: one row repeated) would read as zeros, and take the general pool.
   const bool fast = (block_size == 32 || block_size == 64 || block_size == 128) &&
                     (head_dim == 64 || head_dim == 128) &&
+                    std::min(q_strides[2], k_strides[2]) >= head_dim &&
                     std::max<int64_t>(seq_len, kFusePB * block_size) *
                             std::max(q_strides[2], k_strides[2]) * 2 < 0x7fffffffLL;
   if (fast) {

@@ -8,6 +8,7 @@ import torch
 from helpers import require_gpu
 from tasft_amd import workloads as wl
 from tasft_amd.kernels import BlockSparseFlashAttention
+from tasft_amd.modules import AttnGate
 
 pytestmark = pytest.mark.gpu
 
@@ -41,3 +42,23 @@ def test_prefill(bs, D):
             t, c = ([x[0].transpose(0, 1) for x in y] for y in (t, c))
             assert torch.equal(attn.forward_varlen(*t, varlen_mask, cu, S),
                                attn.forward_varlen(*c, varlen_mask, cu, S))
+
+
+@pytest.mark.parametrize("D", [64, 128])
+@pytest.mark.parametrize(("B", "bs"), [(1, 32), (1, 64), (8, 64), (1, 128)])  # 8: the one-launch form
+def test_gate(B, bs, D):
+    dev = require_gpu()
+    S, Hq, Hkv = 1100, 32, 8
+    print(f"gate token strides B={B} block {bs} D={D}", flush=True)
+    torch.manual_seed(bs + D)
+    gate = AttnGate(num_heads=Hq, head_dim=D, block_size=bs, gate_hidden_dim=32).to(dev).requires_grad_(False)
+    q, k = (wl.randn_bf16((B, h, S, D), 41 + i, scale=1.0).to(dev) for i, h in enumerate((Hq, Hkv)))
+    for i in range(2):
+        for view in _views((Hq, Hkv)[i], S, D, 50 + i, dev):
+            t = [q, k]
+            t[i] = view.expand(B, -1, -1, -1)
+            a = gate(*t, threshold=0.5)
+            b = gate(*(x.contiguous() for x in t), threshold=0.5)
+            # Another kernel pools such rows, with its fp32 sums in another order: bs + D + hidden
+            # terms of 2^-24 on logits of order one, and a sigmoid (slope 1/4).
+            torch.testing.assert_close(a.soft_scores, b.soft_scores, rtol=0, atol=2e-6)
