@@ -247,8 +247,8 @@ gate_target_bs64_kernel(const GateTargetParams p) {
   }
   auto issue = [&](uint8_t* kt, int kb) {
     const int key0 = kb * BS;
-    const int64_t rows_left = (int64_t)(p.S - key0);
-    const int64_t bytes = rows_left * p.sk[2] * 2;
+    // Ends with row S-1, also where rows overlap (token strides below D).
+    const int64_t bytes = (int64_t)(p.S - key0 - 1) * p.sk[2] * 2 + ROWB;
     const __amdgpu_buffer_rsrc_t rs = __builtin_amdgcn_make_buffer_rsrc(
         (void*)(kbase + (int64_t)key0 * p.sk[2]), (short)0,
         bytes > 0x7fffffff ? 0x7fffffff : (int)bytes, 0x00020000);
@@ -466,7 +466,8 @@ gate_target_bs64_w1_kernel(const GateTargetParams p) {
   }
   auto issue = [&](uint8_t* kt, int kb) {
     const int key0 = kb * BS;
-    const int64_t bytes = (int64_t)(p.S - key0) * p.sk[2] * 2;
+    // Ends with row S-1, also where rows overlap (token strides below D).
+    const int64_t bytes = (int64_t)(p.S - key0 - 1) * p.sk[2] * 2 + ROWB;
     const __amdgpu_buffer_rsrc_t rs = __builtin_amdgcn_make_buffer_rsrc(
         (void*)(kbase + (int64_t)key0 * p.sk[2]), (short)0,
         bytes > 0x7fffffff ? 0x7fffffff : (int)bytes, 0x00020000);

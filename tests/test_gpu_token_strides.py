@@ -9,6 +9,7 @@ from helpers import require_gpu
 from tasft_amd import workloads as wl
 from tasft_amd.kernels import BlockSparseFlashAttention
 from tasft_amd.modules import AttnGate
+from tasft_amd.training import gate_target_from_qk
 
 pytestmark = pytest.mark.gpu
 
@@ -62,3 +63,21 @@ def test_gate(B, bs, D):
             # Another kernel pools such rows, with its fp32 sums in another order: bs + D + hidden
             # terms of 2^-24 on logits of order one, and a sigmoid (slope 1/4).
             torch.testing.assert_close(a.soft_scores, b.soft_scores, rtol=0, atol=2e-6)
+
+
+@pytest.mark.parametrize("D", [64, 128])
+@pytest.mark.parametrize("bs", [32, 64, 128])
+def test_gate_target(bs, D):
+    dev = require_gpu()
+    S, Hq, Hkv = 333, 4, 2
+    print(f"gate target token strides block {bs} D={D}", flush=True)
+    q, k = (wl.randn_bf16((1, h, S, D), 61 + i, scale=1.0).to(dev) for i, h in enumerate((Hq, Hkv)))
+    per_query = torch.randn(1, 1, S, S, device=dev)
+    for i in range(2):
+        for view in _views((Hq, Hkv)[i], S, D, 70 + i, dev):
+            t = [q, k]
+            t[i] = view
+            c = [x.contiguous() for x in t]
+            for mask in (None, per_query[:, 0, 0], per_query):
+                assert torch.equal(gate_target_from_qk(*t, bs, normalize="none", attention_mask=mask),
+                                   gate_target_from_qk(*c, bs, normalize="none", attention_mask=mask))
