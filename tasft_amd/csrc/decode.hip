@@ -66,6 +66,12 @@ __device__ __forceinline__ __amdgpu_buffer_rsrc_t decode_rsrc(const void* base, 
   const int n = bytes > 0x7fffffff ? 0x7fffffff : (bytes < 0 ? 0 : (int)bytes);
   return __builtin_amdgcn_make_buffer_rsrc((void*)base, (short)0, n, 0x00020000);
 }
+// Bytes from the first of `rows` rows of D elements to the end of the last, `stride` elements
+// apart (also where rows overlap); none without a row.
+template <int D>
+__device__ __forceinline__ int64_t rows_bytes(int rows, int64_t stride) {
+  return rows > 0 ? ((rows - 1) * stride + D) * 2 : 0;
+}
 
 // s_waitcnt immediate waiting until at most n vector-memory operations are outstanding
 // (expcnt and lgkmcnt left at their maxima).
@@ -287,7 +293,7 @@ bsfa_decode_split_kernel(const DecodeParams p) {
           const int page = __builtin_amdgcn_readlane(pgv, row0 / ps);
           const int rows = min(16, kv_len - key0 - t * 16);
           const __amdgpu_buffer_rsrc_t kr = decode_rsrc(
-              kbase + (int64_t)page * p.sk[0] + (int64_t)(row0 % ps) * ks2, (int64_t)max(rows, 0) * ks2 * 2);
+              kbase + (int64_t)page * p.sk[0] + (int64_t)(row0 % ps) * ks2, rows_bytes<D>(rows, ks2));
 #pragma unroll
           for (int ks = 0; ks < KS; ++ks) ka[t][ks] = buf_load16(kr, k_voff + ks * 64, 0);
         }
@@ -303,7 +309,7 @@ bsfa_decode_split_kernel(const DecodeParams p) {
         }
       }
     } else {
-      const __amdgpu_buffer_rsrc_t kr = decode_rsrc(kbase + (int64_t)key0 * ks2, (int64_t)BS * ks2 * 2);
+      const __amdgpu_buffer_rsrc_t kr = decode_rsrc(kbase + (int64_t)key0 * ks2, rows_bytes<D>(BS, ks2));
       if (key0 + BS <= kv_len) {
 #pragma unroll
         for (int t = 0; t < NT; ++t)
@@ -333,13 +339,13 @@ bsfa_decode_split_kernel(const DecodeParams p) {
         const int page = __builtin_amdgcn_readlane(pgv, row / ps);
         const int rows = min(RPU, kv_len - key0 - u * RPU);
         const __amdgpu_buffer_rsrc_t vr = decode_rsrc(
-            vbase + (int64_t)page * p.sv[0] + (int64_t)(row % ps) * vs2, (int64_t)max(rows, 0) * vs2 * 2);
+            vbase + (int64_t)page * p.sv[0] + (int64_t)(row % ps) * vs2, rows_bytes<D>(rows, vs2));
         dma16(vr, v_lds[wave] + u * 1024, v_src_off(u) - u * RPU * vs2 * 2);
       }
     } else {
       // The resource ends at row kv_len-1, so rows past kv_len arrive as zeros.
       const __amdgpu_buffer_rsrc_t vr =
-          decode_rsrc(vbase + (int64_t)key0 * vs2, (int64_t)min(BS, kv_len - key0) * vs2 * 2);
+          decode_rsrc(vbase + (int64_t)key0 * vs2, rows_bytes<D>(min(BS, kv_len - key0), vs2));
 #pragma unroll
       for (int u = 0; u < VTILE / 1024; ++u) dma16(vr, v_lds[wave] + u * 1024, v_src_off(u));
     }

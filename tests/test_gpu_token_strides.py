@@ -81,3 +81,37 @@ def test_gate_target(bs, D):
             for mask in (None, per_query[:, 0, 0], per_query):
                 assert torch.equal(gate_target_from_qk(*t, bs, normalize="none", attention_mask=mask),
                                    gate_target_from_qk(*c, bs, normalize="none", attention_mask=mask))
+
+
+@pytest.mark.parametrize("D", [64, 128])
+@pytest.mark.parametrize("bs", [32, 64, 128])
+def test_decode(bs, D):
+    dev = require_gpu()
+    S, Hq, Hkv = 333, 8, 2
+    print(f"decode token strides block {bs} D={D}", flush=True)
+    nb = -(-S // bs)
+    q = wl.randn_bf16((1, Hq, 1, D), 81, scale=1.0).to(dev)
+    kv = [wl.randn_bf16((1, Hkv, S, D), 82 + i, scale=1.0).to(dev) for i in range(2)]
+    mask = torch.ones(1, Hq, 1, nb, dtype=torch.bool, device=dev)
+    lens = torch.tensor([S - 3], dtype=torch.int32, device=dev)
+    attn = BlockSparseFlashAttention(block_size=bs, min_sparsity_for_speedup=0.0)
+    for i in range(2):
+        for view in _views(Hkv, S, D, 90 + i, dev):
+            t = list(kv)
+            t[i] = view
+            c = [x.contiguous() for x in t]
+            for n in (None, lens):
+                assert torch.equal(attn.forward_decode(q, *t, mask, kv_lens=n),
+                                   attn.forward_decode(q, *c, mask, kv_lens=n))
+    for page in (8, 16, 64):  # page pools [pages, page, Hkv, D], each page one repeated row
+        pages = -(-S // page)
+        table = torch.randperm(pages, generator=torch.Generator().manual_seed(page)).view(1, -1)
+        table = table.to(dev, torch.int32)
+        pools = [wl.randn_bf16((pages, page, Hkv, D), 100 + i, scale=1.0).to(dev) for i in range(2)]
+        for i in range(2):
+            t = list(pools)
+            t[i] = pools[i][:, :1].expand(pages, page, Hkv, D)
+            c = [x.contiguous() for x in t]
+            m = torch.ones(1, Hq, 1, -(-pages * page // bs), dtype=torch.bool, device=dev)
+            assert torch.equal(attn.forward_decode_paged(q, *t, table, lens, m),
+                               attn.forward_decode_paged(q, *c, table, lens, m))
