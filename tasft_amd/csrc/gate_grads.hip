@@ -328,8 +328,11 @@ gate_grads_reduce_kernel(const GateGradParams p) {
   if (sl == 0 && dst) *dst = (float)((red[0][o] + red[1][o]) + (red[2][o] + red[3][o]));
 }
 
-// Workgroups of the weight products of du (and as many of dv): two per CU.
+// Workgroups of the weight products of du (and as many of dv), at least: two per CU.
 constexpr int64_t kGradGroups = 512;
+// Rows of a partial product, at most: a run is one serial fp32 sum, and its length sets the
+// rounding error whatever the batch (the partial products are added up in 64 bits).
+constexpr int64_t kGradRun = 128;
 
 // Sizes of a call: row chunks of 64 query blocks, fewer rows (down to 16) while the launch
 // would leave CUs without a workgroup.
@@ -351,7 +354,7 @@ static GateGradPlan gate_grad_plan(int64_t B, int64_t Hq, int64_t Hkv, int64_t S
   auto split = [&](int64_t rows, int64_t* parts, int64_t* span) {
     const int64_t want = std::max<int64_t>(1, kGradGroups / tiles);
     const int64_t batch = 4 * kGradBatch;
-    *span = ((rows + want - 1) / want + batch - 1) / batch * batch;
+    *span = std::min(((rows + want - 1) / want + batch - 1) / batch * batch, kGradRun);
     *parts = (rows + *span - 1) / *span;
   };
   split(B * Hq * g.nb, &g.qparts, &g.qspan);

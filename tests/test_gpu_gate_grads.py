@@ -1,6 +1,6 @@
 """tasft_gate_grads (the gate's parameter gradients) at the edges of its tiles: row chunks of
-16 to 64 query blocks, 16-key rounds, 64-unit tiles, 32-dim output tiles, the ends of the row
-runs of the weight products, and the block-diagonal cases, against the formula in 64 bits."""
+16 to 64 query blocks, 16-key rounds, 64-unit tiles, 64-dim output tiles, the ends of the row
+runs of the weight products (at most 128 rows each), and the block-diagonal cases, against the formula in 64 bits."""
 from __future__ import annotations
 
 import pytest
@@ -20,6 +20,7 @@ CASES = [
     (1, 8, 2, 16 * 65, 128, 16, 96, True),  # 65 blocks: a last chunk of one row
     (4, 32, 8, 32 * 66, 256, 32, 64, True), # 66 blocks in 64-row chunks, 256 dims, 2112 K rows
     (3, 6, 2, 700, 8, 64, 130, False),      # eight dims, a third unit tile of two units
+    (8, 32, 8, 16 * 128, 128, 16, 72, True),  # 32768 rows, four tiles: the longest run, 128 rows
 ]
 
 

@@ -47,6 +47,17 @@ def test_abi_version_and_workspace_sizes():
     assert lib.tasft_mask_compact_workspace_bytes(0, 32, 128) == 0
 
 
+def test_gate_gradient_runs_stay_short():
+    """The weight products of the gate's backward are sums over runs of at most 128 rows, also
+    where 512 workgroups would not need that many runs: the workspace holds them all."""
+    lib = _native.load_library()
+    for B, Hq, Hkv, S, D, hid in ((4, 32, 8, 8192, 256, 256), (16, 32, 8, 8192, 128, 128)):
+        rows, krows = B * Hq * S // 64, B * Hkv * S // 64
+        dv_heads = 2 * rows * hid  # two chunks of 64 query blocks
+        floats = lib.tasft_gate_grads_workspace_bytes(B, Hq, Hkv, S, D, 64, hid) // 4
+        assert floats - dv_heads >= (rows + krows) // 128 * hid * D
+
+
 def _i64(vals):
     return (ctypes.c_int64 * 4)(*vals)
 
