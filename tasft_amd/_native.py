@@ -9,6 +9,7 @@ from __future__ import annotations
 import ctypes
 import functools
 import threading
+from collections.abc import Sequence
 from pathlib import Path
 
 import torch
@@ -175,15 +176,20 @@ def is_available() -> bool:
 
 
 @functools.lru_cache(maxsize=4096)
-def strides_array(values: tuple[int, ...]) -> ctypes.Array:
-    """Element strides as a C int64 array. Arrays are kept by their values (the library only
-    reads them): building the five of a call took as long as the call."""
+def _kept_array(values: tuple[int, ...]) -> ctypes.Array:
     return (ctypes.c_int64 * len(values))(*values)
 
 
+def strides_array(values: Sequence[int]) -> ctypes.Array:
+    """A sequence of element strides as a C int64 array. Arrays are kept by their values (not to
+    be written to; the library only reads them): building the five of a call took as long as
+    the call."""
+    return _kept_array(tuple(values))
+
+
 def strides(t: torch.Tensor) -> ctypes.Array:
-    """Element strides of a tensor as a C int64 array."""
-    return strides_array(t.stride())
+    """Element strides of a tensor as a C int64 array (``strides_array``)."""
+    return _kept_array(t.stride())
 
 
 # Element types of the 16-bit tensors (TASFT_DTYPE_BF16 / TASFT_DTYPE_F16).

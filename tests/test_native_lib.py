@@ -58,6 +58,12 @@ def test_gate_gradient_runs_stay_short():
         assert floats - dv_heads >= (rows + krows) // 128 * hid * D
 
 
+def test_stride_arrays_take_any_sequence():
+    t = torch.empty(3, 5, 8).transpose(0, 1)
+    for values in ((8, 40, 1), [8, 40, 1], torch.Size((8, 40, 1))):
+        assert list(_native.strides_array(values)) == list(_native.strides(t)) == [8, 40, 1]
+
+
 def _i64(vals):
     return (ctypes.c_int64 * 4)(*vals)
 
