@@ -74,8 +74,10 @@ CASES = [
     (1, 2, 1, 777, 128, 48, 64, True),     # block size outside {32,64,128}
     (1, 4, 2, 700, 64, 64, 32, True),      # block 64, D=64, 11 blocks (partial pool chunk)
     (1, 4, 2, 1300, 128, 64, 200, False),  # block 64, 21 blocks, hidden > one staging tile
-    (1, 4, 2, 1300, 128, 64, 64, False),   # block 64, non-causal, fused query-pool + pairwise
-    (1, 2, 1, 9000, 128, 64, 32, True),    # 141 blocks: two 128-key groups per row
+    (1, 4, 2, 1300, 128, 64, 64, False),   # block 64, non-causal, 21 blocks
+    (1, 2, 1, 9000, 128, 64, 32, True),    # 141 blocks
+    (8, 28, 4, 1100, 128, 64, 64, False),  # block 64, 512 chunks: one launch, non-causal
+    (1, 28, 4, 9000, 64, 64, 32, True),    # 288 chunks: one launch, two 128-key groups per row
     (1, 4, 2, 1000, 128, 128, 64, True),   # block 128 streaming pool, ragged, one partial chunk
     (2, 4, 2, 2500, 64, 128, 48, False),   # block 128, D=64, non-causal, 20 blocks (two chunks)
     (1, 4, 2, 1000, 128, 32, 64, True),    # block 32 streaming pool, 32 blocks (two chunks)
@@ -156,9 +158,13 @@ def test_config2_gate_full_size_sampled_heads():
 
 
 @pytest.mark.parametrize(("B", "Hq", "Hkv", "S", "D", "hidden"), [
+    # One launch (more than 256 chunks of 16 blocks):
     (4, 32, 8, 8192, 128, 128),  # config 2
-    (1, 2, 1, 9000, 128, 32),    # two 128-key groups per row
-    (2, 4, 2, 700, 64, 64),      # D = 64, partial last query chunk
+    (1, 28, 4, 9000, 128, 32),   # two 128-key groups per row
+    (8, 32, 8, 1100, 64, 64),    # D = 64, partial last query chunk
+    # A pooling launch and the pairwise tiles:
+    (1, 2, 1, 9000, 128, 32),
+    (2, 4, 2, 700, 64, 64),
 ])
 def test_causal_rows_skip_matches_full_evaluation(B, Hq, Hkv, S, D, hidden):
     """Without logits, the causal gate evaluates only the key blocks a query chunk needs
@@ -223,14 +229,19 @@ def _gate_c_abi(gate, q, k, taus, workspace, flags=3):
     return soft, mask, count
 
 
-def test_one_launch_gate_reuses_its_workspace():
-    """The one-launch gate (block 64) on one workspace, first filled with 0xFF bytes (its
-    completion counters included), twice in a row with different inputs: each call's outputs
-    equal a fresh-workspace call's bit for bit, and the count (bit 63 clear) is the mask's sum."""
+@pytest.mark.parametrize(("B", "Hq", "Hkv", "S"), [
+    (8, 28, 4, 1100),  # 512 chunks of 16 blocks: one launch
+    (2, 8, 2, 2048),   # 40: a pooling launch and the pairwise tiles
+])
+def test_one_launch_gate_reuses_its_workspace(B, Hq, Hkv, S):
+    """The gate at block 64 (the one-launch form and the small one) on one workspace, first
+    filled with 0xFF bytes (the completion counters included), twice in a row with different
+    inputs: each call's outputs equal a fresh-workspace call's bit for bit, and the count (bit 63
+    clear) is the mask's sum."""
     from tasft_amd import _native
 
     dev = require_gpu()
-    B, Hq, Hkv, S, D, hidden = 2, 8, 2, 2048, 128, 64
+    D, hidden = 128, 64
     gate = _gate(Hq, D, 64, hidden, True, seed=91).to(dev).requires_grad_(False)
     taus = torch.linspace(0.4, 0.6, Hq, device=dev)
     lib = _native.load_library()
@@ -250,7 +261,11 @@ def test_one_launch_gate_reuses_its_workspace():
         assert torch.equal(mod.hard_mask.to(torch.uint8), mask)
 
 
-def test_one_launch_gate_wait_error_path():
+@pytest.mark.parametrize(("B", "Hq", "Hkv", "S"), [
+    (1, 4, 2, 1024),
+    (8, 28, 4, 1100),  # 512 chunks of 16 blocks: one launch without the switch, too
+])
+def test_one_launch_gate_wait_error_path(B, Hq, Hkv, S):
     """With the diagnostic switch on, the key workgroups publish nothing: every query
     workgroup's bounded wait gives up (every workgroup still exits), its rows get NaN scores
     and no mask bit, bit 63 of the count is set and GateOutput.sparsity_ratio raises
@@ -259,9 +274,9 @@ def test_one_launch_gate_wait_error_path():
     from tasft_amd.exceptions import KernelError
 
     dev = require_gpu()
-    gate = _gate(4, 128, 64, 64, True, seed=17).to(dev).requires_grad_(False)
-    q = wl.randn_bf16((1, 4, 1024, 128), 71, scale=1.0).to(dev)
-    k = wl.randn_bf16((1, 2, 1024, 128), 72, scale=1.0).to(dev)
+    gate = _gate(Hq, 128, 64, 64, True, seed=17).to(dev).requires_grad_(False)
+    q = wl.randn_bf16((B, Hq, S, 128), 71, scale=1.0).to(dev)
+    k = wl.randn_bf16((B, Hkv, S, 128), 72, scale=1.0).to(dev)
     with torch.no_grad():
         good = gate(q, k, threshold=0.5)
     good_sparsity = good.sparsity_ratio

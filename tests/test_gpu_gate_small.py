@@ -56,3 +56,18 @@ def test_both_forms(B, Hq, Hkv, S, D, hidden, causal, dtype):
     on = (out.soft_scores >= 0.5) | torch.eye(ref.shape[-1], dtype=torch.bool, device=dev)
     assert torch.equal(out.hard_mask, on)
     assert out.sparsity_ratio == pytest.approx(1 - on.double().mean().item(), abs=1e-9)
+
+
+def test_forms_agree_on_the_same_heads():
+    """A batch above the limit (one kernel) against its entries alone (two launches)."""
+    dev = require_gpu()
+    B, Hq, Hkv, S, D, hidden = 8, 28, 4, 1100, 128, 64  # 512 chunks; 64 each
+    gate = _gate(Hq, D, hidden, True, dev)
+    g = torch.Generator(device=dev).manual_seed(S)
+    q = torch.randn(B, Hq, S, D, generator=g, device=dev).bfloat16()
+    k = torch.randn(B, Hkv, S, D, generator=g, device=dev).bfloat16()
+    both = gate(q, k, threshold=0.5)
+    for b in range(B):
+        one = gate(q[b:b + 1], k[b:b + 1], threshold=0.5)
+        # Two orders of the fp32 sums, each within 2e-6 of the exact score (test_both_forms).
+        torch.testing.assert_close(one.soft_scores, both.soft_scores[b:b + 1], rtol=0, atol=4e-6)

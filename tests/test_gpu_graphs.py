@@ -1,10 +1,10 @@
-"""HIP-graph capture of the hot path: the gate (one kernel after its counter reset), the
-prefill (two-wave kernel; the persistent four-wave kernel with its ticket reset; block 128 on
-the block-64 kernel) and the split-K decode are captured once and replayed with new inputs.
+"""HIP-graph capture of the hot path: the gate (one kernel after its counter reset; the small
+form's two), the prefill (both head dims; block 128 on the block-64 kernel) and the split-K
+decode are captured once and replayed with new inputs.
 
 Each replay is preceded by eager work on the same tensors (the same call run eagerly on the
 replay's inputs, then a synchronisation), and every replay must equal that eager result bit
-for bit: counters, tickets and workspaces that a replay finds must have been reset by kernels
+for bit: counters and workspaces that a replay finds must have been reset by kernels
 inside the graph, since no host code runs between replays.
 """
 from __future__ import annotations
@@ -38,9 +38,13 @@ def _capture(fn):
     return g, out
 
 
-def test_gate_one_kernel_replays():
+@pytest.mark.parametrize(("B", "Hq", "Hkv", "S"), [
+    (8, 28, 4, 1100),  # 512 chunks of 16 blocks: one kernel after its counter reset
+    (2, 8, 2, 2048),   # 40: a pooling launch and the pairwise tiles
+])
+def test_gate_one_kernel_replays(B, Hq, Hkv, S):
     dev = require_gpu()
-    B, Hq, Hkv, S, D, hidden = 2, 8, 2, 2048, 128, 64
+    D, hidden = 128, 64
     torch.manual_seed(3)
     gate = AttnGate(num_heads=Hq, head_dim=D, block_size=64, gate_hidden_dim=hidden).to(dev)
     gate.requires_grad_(False)
