@@ -7,7 +7,7 @@ import pytest
 import torch
 
 import attn_inputs as ai
-from helpers import assert_close_bf16, bar, require_gpu, to_np
+from helpers import MAX_ABS_TOL, assert_close_bf16, bar, require_gpu, to_np
 from oracle import tasft_oracle as orc
 from tasft_amd.kernels import BlockSparseFlashAttention
 
@@ -27,6 +27,24 @@ pytestmark = pytest.mark.gpu
     (4200, 3, 3, 64, 128, False),
 ])
 def test_few_rows(S, Hq, Hkv, D, bs, causal, kind):
+    _check(S, Hq, Hkv, D, bs, causal, kind)
+
+
+@pytest.mark.parametrize("kind", ["unit", "peaky"])
+@pytest.mark.parametrize(("S", "Hq", "Hkv", "D", "bs", "causal"), [
+    (4200, 8, 2, 128, 64, False),    # 528 rows
+    (4200, 8, 2, 128, 128, True),    # 528 rows of 64 tokens
+    (4200, 16, 4, 64, 64, False),    # 1056 rows
+    (4200, 16, 4, 64, 128, True),
+])
+def test_one_pair_long_rows(S, Hq, Hkv, D, bs, causal, kind):
+    """One pair, more than 64 key blocks per row and a ragged end. A row that attends to one key
+    returns its V row, and among millions of values some exceed 4, where half a unit of the
+    bf16 output is 2^-6 alone; P's rounding adds at most 2^-9 max|v|."""
+    _check(S, Hq, Hkv, D, bs, causal, kind, rounding_bound=True)
+
+
+def _check(S, Hq, Hkv, D, bs, causal, kind, rounding_bound=False):
     dev = require_gpu()
     nb = -(-S // bs)
     print(f"prefill pairs S={S} Hq={Hq} D={D} block {bs} causal={causal} {kind}", flush=True)
@@ -39,7 +57,31 @@ def test_few_rows(S, Hq, Hkv, D, bs, causal, kind):
         q.to(dev), k.to(dev), v.to(dev), mask.to(dev), causal=causal)
     torch.cuda.synchronize()
     ref = orc.attention_block_gather(to_np(q), to_np(k), to_np(v), mask.numpy(), bs, causal)
-    assert_close_bf16(out, ref, f"prefill pairs S={S} D={D} block {bs} {kind}")
+    bound = MAX_ABS_TOL
+    if rounding_bound:
+        bound = max(bound, 2.0 ** (np.floor(np.log2(np.abs(ref).max())) - 8) + 2.0 ** -9 * float(v.abs().max()))
+    assert_close_bf16(out, ref, f"prefill pairs S={S} D={D} block {bs} {kind}", max_abs=bound)
+
+
+@pytest.mark.parametrize("D", [64, 128])
+@pytest.mark.parametrize("causal", [True, False])
+def test_packed_one_pair(causal, D):
+    """A packed call above the row limits (the longest sequence's rows count for each), its
+    first sequence of more than 64 key blocks."""
+    dev = require_gpu()
+    lens, Hq, Hkv = [4200, 700, 65], 8, 2
+    cu = np.cumsum([0] + lens).tolist()
+    print(f"prefill one pair packed D={D} causal={causal}", flush=True)
+    nb = -(-max(lens) // 64)
+    q, k, v = (t[0].transpose(0, 1).contiguous() for t in ai.qkv("unit", (1, Hq, cu[-1], D), (1, Hkv, cu[-1], D),
+                                                                 7 + D, 64))
+    mask = torch.rand(len(lens), Hq, nb, nb, generator=torch.Generator().manual_seed(D)) < 0.2
+    mask |= torch.eye(nb, dtype=torch.bool)
+    out = BlockSparseFlashAttention(block_size=64, min_sparsity_for_speedup=0.0).forward_varlen(
+        q.to(dev), k.to(dev), v.to(dev), mask.to(dev), torch.tensor(cu, dtype=torch.int32), causal=causal)
+    torch.cuda.synchronize()
+    ref = orc.attention_varlen(to_np(q), to_np(k), to_np(v), cu, mask.numpy(), 64, causal)
+    assert_close_bf16(out, ref, f"prefill one pair packed D={D} causal={causal}")
 
 
 @pytest.mark.parametrize("dtype", [torch.bfloat16, torch.float16])
