@@ -85,14 +85,13 @@ def random_mask(shape, density: float, seed: int) -> torch.Tensor:
 
 # ----------------------------------------------------------------------------- cases
 # Prefill: (B, Hq, Hkv, S, D, bs, causal, density, variant). ``variant`` names the kernel
-# the shape selects: "2w" the two-wave block-64 D=128 kernel; "4w" the four-wave block-64
-# D=64 kernel (run both with and without its persistent work queue); "gen" the generic
-# kernel (block 32 or 128).
+# the shape selects: "2w" the two-wave block-64 kernel at D=128; "2w64" the same at D=64 (run
+# with and without a workspace); "gen" the block-32 kernel or block 128 on the block-64 one.
 PREFILL_CASES = [
     (1, 8, 2, 1000, 128, 64, True, 0.45, "2w"),
     (2, 4, 4, 384, 128, 64, False, 0.5, "2w"),
-    (1, 4, 2, 700, 64, 64, True, 0.5, "4w"),
-    (1, 4, 1, 448, 64, 64, False, 0.5, "4w"),
+    (1, 4, 2, 700, 64, 64, True, 0.5, "2w64"),
+    (1, 4, 1, 448, 64, 64, False, 0.5, "2w64"),
     (1, 4, 2, 600, 128, 32, True, 0.4, "gen"),
     (1, 2, 2, 520, 64, 128, True, 0.6, "gen"),
     (1, 4, 4, 300, 64, 32, False, 0.5, "gen"),

@@ -25,7 +25,7 @@ from tasft_amd.kernels import BlockSparseFlashAttention
 pytestmark = pytest.mark.gpu
 
 PREFILL = [
-    # B, Hq, Hkv, S, D, bs (kernel: two-wave, four-wave, block 32, block 128 on block 64)
+    # B, Hq, Hkv, S, D, bs (two waves at D=128 and D=64, block 32, block 128 on block 64)
     (1, 4, 2, 700, 128, 64),
     (1, 4, 2, 700, 64, 64),
     (1, 4, 2, 300, 128, 32),

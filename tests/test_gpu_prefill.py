@@ -207,7 +207,7 @@ def test_config4_full_size_sampled_heads():
 
 
 def _prefill_capi(q, k, v, mask, bs, causal, workspace=None):
-    """tasft_bsfa_prefill_fwd called directly (``workspace`` None: one workgroup per row)."""
+    """tasft_bsfa_prefill_fwd called directly, with or without a workspace."""
     import ctypes
 
     from tasft_amd import _native
@@ -232,7 +232,7 @@ def _prefill_capi(q, k, v, mask, bs, causal, workspace=None):
 def test_prefill_discriminating_inputs(case, kind):
     """Scores far from uniform (unit scale; peaky keys that move the running maximum):
     pins QK^T, the exp2 scale, max tracking and the lazy rescale of every prefill kernel.
-    The four-wave kernel runs with its persistent queue (the Python path) and without."""
+    At head dim 64 the C call runs too, with a workspace (the Python path passes none)."""
     dev = require_gpu()
     B, Hq, Hkv, S, D, bs, causal, _dens, variant = case
     print(f"prefill discriminating {case} {kind}", flush=True)
@@ -241,9 +241,10 @@ def test_prefill_discriminating_inputs(case, kind):
     qd, kd, vd, md = q.to(dev), k.to(dev), v.to(dev), mask.to(dev)
     out = _run(qd, kd, vd, md, bs, causal)
     assert_close_bf16(out, ref, f"prefill {variant} {kind}")
-    if variant == "4w":
-        direct = _prefill_capi(qd, kd, vd, md, bs, causal)
-        assert_close_bf16(direct, ref, f"prefill {variant} {kind} (no work queue)")
+    if variant == "2w64":
+        ws = torch.full((256,), 0xFF, dtype=torch.uint8, device=dev)
+        direct = _prefill_capi(qd, kd, vd, md, bs, causal, ws)
+        assert_close_bf16(direct, ref, f"prefill {variant} {kind} (workspace)")
         assert torch.equal(direct, out)
 
 
@@ -263,15 +264,14 @@ def test_prefill_varlen_discriminating_inputs(case, kind):
 
 
 @pytest.mark.parametrize(("B", "Hq", "Hkv", "S", "D", "bs"), [
-    (2, 16, 4, 2048, 64, 64),    # 8 KV groups: per-XCD partitions of the work queue
-    (2, 6, 3, 1500, 64, 64),     # 6 KV groups: one partition, ragged
-    (2, 16, 4, 2048, 128, 64),   # two-wave kernel: the workspace is left unused
-    (1, 8, 2, 1024, 128, 128),   # block 128 on the two-wave kernel
-    (2, 16, 4, 1500, 64, 128),   # block 128 on the four-wave kernel's work queue, ragged
+    (2, 16, 4, 2048, 64, 64),    # 8 KV groups: dealt to the XCDs
+    (2, 6, 3, 1500, 64, 64),     # 6 KV groups: in turn, ragged
+    (2, 16, 4, 2048, 128, 64),
+    (1, 8, 2, 1024, 128, 128),   # block 128 on the block-64 kernel
+    (2, 16, 4, 1500, 64, 128),   # the same at head dim 64, ragged
 ])
-def test_persistent_queue_is_bit_identical(B, Hq, Hkv, S, D, bs):
-    """The persistent work queue (workspace given; head dim 64 at block 64 or 128) must not
-    change any output bit against one workgroup per row."""
+def test_workspace_is_accepted_and_unused(B, Hq, Hkv, S, D, bs):
+    """A workspace must not change any output bit, and is left as it was."""
     dev = require_gpu()
     q, k, v = ai.qkv("unit", (B, Hq, S, D), (B, Hkv, S, D), 4242 + S + D, bs)
     shape = wl.Shape(B, Hq, Hkv, S, D, bs)
@@ -279,12 +279,14 @@ def test_persistent_queue_is_bit_identical(B, Hq, Hkv, S, D, bs):
     mask[0, 1, -3:, :] = True   # whole rows lit, as a gate can produce
     mask[B - 1, Hq - 1, 5, :] = True
     q, k, v, mask = q.to(dev), k.to(dev), v.to(dev), mask.to(dev)
-    out_ws = _run(q, k, v, mask, bs, True)  # the Python path passes a workspace
-    out = _prefill_capi(q, k, v, mask, bs, True)
-    assert torch.equal(out, out_ws)
+    ws = torch.full((256,), 0xFF, dtype=torch.uint8, device=dev)
+    out_ws = _prefill_capi(q, k, v, mask, bs, True, ws)
+    assert bool((ws == 0xFF).all())
+    assert torch.equal(_prefill_capi(q, k, v, mask, bs, True), out_ws)
+    assert torch.equal(_run(q, k, v, mask, bs, True), out_ws)
     ref = orc.attention_block_gather(to_np(q.cpu()), to_np(k.cpu()), to_np(v.cpu()),
                                      mask.cpu().numpy(), bs, True)
-    assert_close_bf16(out_ws, ref, "persistent prefill")
+    assert_close_bf16(out_ws, ref, "prefill with a workspace")
 
 
 # ----------------------------------------------------------------------------- varlen
@@ -304,11 +306,11 @@ def _packed(lens, Hq, Hkv, D, seed, pad=5):
 VARLEN_CASES = [
     # lengths, Hq, Hkv, D, bs, causal, density
     ([100, 0, 257, 64, 1], 8, 2, 128, 64, True, 0.5),   # two-wave kernel; empty and 1-token
-    ([300, 45, 128], 4, 4, 64, 64, True, 0.5),          # four-wave kernel (D=64)
+    ([300, 45, 128], 4, 4, 64, 64, True, 0.5),          # head dim 64
     ([130, 77], 4, 2, 64, 32, False, 0.6),              # generic kernel, non-causal
     ([513, 200], 7, 1, 128, 128, True, 0.4),            # bs=128, G=7
     ([64, 1, 95, 700], 16, 2, 128, 32, True, 0.3),      # G=8, bs=32, block-aligned and 1-token
-    ([333, 334], 8, 1, 64, 64, False, 0.7),             # non-causal four-wave kernel
+    ([333, 334], 8, 1, 64, 64, False, 0.7),             # non-causal, head dim 64
 ]
 
 
@@ -365,7 +367,7 @@ def _expand128(mask128: torch.Tensor, nb64: int) -> torch.Tensor:
 
 @pytest.mark.parametrize(("B", "Hq", "Hkv", "S", "D", "causal"), [
     (1, 8, 2, 1000, 128, True),    # two-wave kernel, ragged: the last 128-block is partial
-    (2, 4, 2, 1500, 64, True),     # four-wave kernel through its persistent work queue
+    (2, 4, 2, 1500, 64, True),     # head dim 64
     (1, 4, 4, 777, 128, False),    # non-causal, ragged
 ])
 def test_block128_is_bit_identical_to_expanded_block64(B, Hq, Hkv, S, D, causal):
