@@ -1245,20 +1245,6 @@ gate_pairwise_bwd_kernel(const GateBwdParams p) {
 
 using namespace tasft;
 
-// Compute units of the current device (cached per device).
-static int gate_device_cus() {
-  static int cached[64] = {0};
-  int dev = 0;
-  if (hipGetDevice(&dev) != hipSuccess || dev < 0 || dev >= 64) return 256;
-  if (cached[dev] == 0) {
-    int n = 0;
-    if (hipDeviceGetAttribute(&n, hipDeviceAttributeMultiprocessorCount, dev) != hipSuccess || n <= 0)
-      n = 256;
-    cached[dev] = n;
-  }
-  return cached[dev];
-}
-
 // The pooling and projection launch: a chunk of kFusePB blocks per workgroup; with SMALL (block
 // 64) one load group.
 template <int D, int DT, bool SMALL>

@@ -446,21 +446,6 @@ def _launch_gate(gate: AttnGate, q: torch.Tensor, k: torch.Tensor, taus: torch.T
             "q_means": qm, "k_means": km, "workspace": workspace, "w_in": w_in, "w_out": w_out}
 
 
-def _weight_grad(d: torch.Tensor, m: torch.Tensor, chunk: int = 256) -> torch.Tensor:
-    """``d^T @ m`` for tall fp32 operands ([K, hidden] and [K, D], K = B * H * NB).
-
-    The output is one small tile while K runs to tens of thousands, so a single GEMM runs
-    on a handful of workgroups that each walk all of K. Split K into chunks of ``chunk``
-    rows as a batched product and sum the partial products instead (K not a multiple of
-    ``chunk``, or a single chunk: one plain GEMM).
-    """
-    K = d.shape[0]
-    if K % chunk or K < 2 * chunk:
-        return d.t() @ m
-    c = K // chunk
-    return torch.bmm(d.view(c, chunk, -1).transpose(1, 2), m.view(c, chunk, -1)).sum(0)
-
-
 class _HipGateFunction(torch.autograd.Function):
     """AttnGate forward/backward on the HIP kernels (gate training).
 

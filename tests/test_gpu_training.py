@@ -1,11 +1,11 @@
 """Gate training on the HIP kernels: the fused KL gate loss and the AttnGate backward.
 
-* ``tasft_gate_kl_fwd`` against the oracle's KL loss and gradient (pinned to F.kl_div with
-  "batchmean" and to torch autograd).
+* ``tasft_gate_kl_loss`` (through ``_GateKL``) against the oracle's KL loss and gradient (pinned
+  to F.kl_div with "batchmean" and to torch autograd).
 * ``gate_loss_from_qk`` against the reference composition
   ``compute_gate_loss(gate, compute_gate_target(scores))`` on explicitly built fp32 scores
   (with and without an attention mask), value and gradient.
-* ``AttnGate`` training through ``tasft_gate_bwd`` against torch autograd of the reference
+* ``AttnGate`` training through ``tasft_gate_grads`` against torch autograd of the reference
   formula (the torch path of the same module) for every parameter and for Q and K.
 """
 from __future__ import annotations
