@@ -35,9 +35,9 @@ from typing import Any
 import torch
 import torch.nn.functional as F
 from torch import nn
-from torch.autograd.function import once_differentiable
 
 from tasft_amd import _native
+from tasft_amd._autograd import first_order_only
 from tasft_amd.exceptions import KernelError, ValidationError
 
 
@@ -464,17 +464,15 @@ class _HipGateFunction(torch.autograd.Function):
         ctx.gate_cfg = (gate.block_size, gate.gate_hidden_dim, gate.is_causal)
         ctx.shapes = (tuple(q.shape), tuple(k.shape))
         ctx.dtypes = (q.dtype, k.dtype, w_in.dtype, b_in.dtype, w_out.dtype)
-        # The weights detached: they may be the parameters themselves, and a graph through them
-        # alone would be a part of the second derivative.
-        ctx.save_for_backward(r["soft"], r["workspace"], r["q_means"], r["k_means"],
-                              r["w_in"].detach(), r["w_out"].detach())
+        ctx.save_for_backward(r["soft"], r["workspace"], r["q_means"], r["k_means"], r["w_in"],
+                              r["w_out"])
         ctx.mark_non_differentiable(r["mask"], r["active"])
         # No zero gradients for the mask and the count (two fills of their size per backward).
         ctx.set_materialize_grads(False)
         return r["soft"], r["mask"], r["active"]
 
     @staticmethod
-    @once_differentiable
+    @first_order_only
     def backward(ctx, grad_soft, _grad_mask, _grad_active):
         if grad_soft is None:
             return (None,) * 8

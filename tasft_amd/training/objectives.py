@@ -20,9 +20,9 @@ import math
 
 import torch
 import torch.nn.functional as F
-from torch.autograd.function import once_differentiable
 
 from tasft_amd import _native
+from tasft_amd._autograd import first_order_only
 from tasft_amd.exceptions import KernelError, NaNDetectedError
 
 _NORMALIZE = {"flat": 0, "row": 1, "none": 2}
@@ -252,7 +252,7 @@ class _GateKL(torch.autograd.Function):
         return loss
 
     @staticmethod
-    @once_differentiable
+    @first_order_only
     def backward(ctx, grad_out: torch.Tensor):
         (grad,) = ctx.saved_tensors
         if grad is None:
