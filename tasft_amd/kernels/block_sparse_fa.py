@@ -100,14 +100,17 @@ def _kernel_ready(t: torch.Tensor) -> torch.Tensor:
     return t if _native.kernel_layout(t) else t.contiguous()
 
 
-def _prefill_ready(t: torch.Tensor, token_dim: int, block_size: int) -> torch.Tensor:
-    """``_kernel_ready`` for the prefill kernels. At head dim 128 those of blocks 64 and 128 read
-    tiles whose rows do not overlap: a token stride below the head dim (0 in an expanded
-    tensor) is copied."""
-    t = _kernel_ready(t)
-    if t.shape[-1] == 128 and block_size != 32 and t.stride(token_dim) < 128:
-        return t.clone(memory_format=torch.contiguous_format)
-    return t
+def _prefill_ready(q: torch.Tensor, k: torch.Tensor, v: torch.Tensor, token_dim: int, block_size: int):
+    """q, k and v as the prefill kernels read them (``_kernel_ready``), and their strides. At head
+    dim 128 the kernels of blocks 64 and 128 read tiles whose rows do not overlap: a tensor
+    with a token stride below the head dim (0 in an expanded one) is copied."""
+    q, k, v = _kernel_ready(q), _kernel_ready(k), _kernel_ready(v)
+    sq, sk, sv = q.stride(), k.stride(), v.stride()
+    if q.shape[-1] == 128 and block_size != 32 and min(sq[token_dim], sk[token_dim], sv[token_dim]) < 128:
+        q, k, v = (t if t.stride(token_dim) >= 128 else t.clone(memory_format=torch.contiguous_format)
+                   for t in (q, k, v))
+        sq, sk, sv = q.stride(), k.stride(), v.stride()
+    return q, k, v, sq, sk, sv
 
 
 def _mask_bytes(mask: torch.Tensor) -> torch.Tensor:
@@ -256,16 +259,14 @@ class BlockSparseFlashAttention:
             if t.device != q.device:
                 raise KernelError("Q, K, V must be on the same device", context={"device": str(t.device)})
         lib = _native.load_library()
-        q = _prefill_ready(q, 2, self.block_size)
-        k = _prefill_ready(k, 2, self.block_size)
-        v = _prefill_ready(v, 2, self.block_size)
+        q, k, v, sq, sk, sv = _prefill_ready(q, k, v, 2, self.block_size)
         mask = _mask_bytes(block_mask if block_mask.device == q.device else block_mask.to(q.device))
         out = torch.empty((B, H, S, D), dtype=q.dtype, device=q.device)
         scale = 1.0 / math.sqrt(D)
         status = lib.tasft_bsfa_prefill_fwd(
             q.data_ptr(), k.data_ptr(), v.data_ptr(), out.data_ptr(), mask.data_ptr(),
             None, 0, B, H, k.shape[1], S, D, self.block_size,
-            _native.strides(q), _native.strides(k), _native.strides(v), _native.strides(out),
+            _native.strides_array(sq), _native.strides_array(sk), _native.strides_array(sv), _native.strides(out),
             _native.strides(mask), scale, 1 if causal else 0, dtype, _native.stream_handle(q.device),
         )
         _native.check(status, "tasft_bsfa_prefill_fwd", {"shape": [B, H, S, D]})
@@ -375,16 +376,14 @@ class BlockSparseFlashAttention:
                 raise KernelError("Q, K, V must be on the same GPU device",
                                   context={"tensor": name, "device": str(t.device)})
         lib = _native.load_library()
-        q = _prefill_ready(q, 0, self.block_size)
-        k = _prefill_ready(k, 0, self.block_size)
-        v = _prefill_ready(v, 0, self.block_size)
+        q, k, v, sq, sk, sv = _prefill_ready(q, k, v, 0, self.block_size)
         mask = _mask_bytes(block_mask if block_mask.device == q.device else block_mask.to(q.device))
         cu_dev = _int32_on(cu_seqlens, q.device)
         out = torch.empty_like(q)
         status = lib.tasft_bsfa_prefill_varlen_fwd(
             q.data_ptr(), k.data_ptr(), v.data_ptr(), out.data_ptr(), mask.data_ptr(),
             cu_dev.data_ptr(), n_seq, H, k.shape[1], max_seqlen, D, self.block_size,
-            _native.strides(q), _native.strides(k), _native.strides(v), _native.strides(out),
+            _native.strides_array(sq), _native.strides_array(sk), _native.strides_array(sv), _native.strides(out),
             _native.strides(mask), 1.0 / math.sqrt(D), 1 if causal else 0, dtype,
             _native.stream_handle(q.device),
         )

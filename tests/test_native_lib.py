@@ -219,15 +219,20 @@ def test_prefill_refuses_overlapping_rows_at_head_dim_128(which, block):
 
 def test_prefill_copies_overlapping_rows_at_head_dim_128():
     from tasft_amd.kernels.block_sparse_fa import _prefill_ready
-    t = torch.randn(2, 1, 1, 128).bfloat16().expand(2, 3, 70, 128)
-    c = _prefill_ready(t, 2, 64)
-    assert c.stride(2) == 128 and torch.equal(c, t)
-    assert _prefill_ready(t, 2, 32) is t  # the block-32 kernel reads them in place
-    assert _prefill_ready(t[..., :64], 2, 64).stride(2) == 0  # and so does head dim 64
+    rows = torch.randn(2, 70, 3, 128).bfloat16().transpose(1, 2)
+    same = torch.randn(2, 1, 1, 128).bfloat16().expand(2, 3, 70, 128)
+    for i in range(3):
+        t = [rows, rows, rows]
+        t[i] = same
+        out = _prefill_ready(*t, 2, 64)
+        assert out[i].stride(2) == 128 and torch.equal(out[i], same)
+        assert all(out[j] is rows for j in range(3) if j != i)
+        assert [tuple(s) for s in out[3:]] == [x.stride() for x in out[:3]]
+    assert _prefill_ready(same, same, same, 2, 32)[1] is same  # block 32 reads them in place
+    half = same[..., :64]
+    assert _prefill_ready(half, half, half, 2, 64)[1] is half  # and so does head dim 64
     one = torch.randn(4, 128).bfloat16().as_strided((1, 4, 1, 128), (512, 128, 0, 1))
-    assert _prefill_ready(one, 2, 64).stride(2) == 128
-    rows = torch.randn(70, 3, 128).bfloat16().transpose(0, 1)[None]
-    assert _prefill_ready(rows, 2, 64) is rows
+    assert _prefill_ready(one, one, one, 2, 64)[0].stride(2) == 128
 
 
 def test_check_raises_kernel_error_with_message():
