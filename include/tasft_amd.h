@@ -195,7 +195,8 @@ int tasft_bsfa_decode_fwd_noalloc(const void* q, const void* k_cache, const void
  * kv_len_max bounds every kv_lens[b]; block_mask [B, Hq, 1, ceil(kv_len_max/bs)].
  * block_size 32, 64 or 128 (vLLM's per-layer block size, tasft/inference/vllm_patch.py:522-525;
  * a 128-key block is read as its two 64-key halves, and num_splits then counts 64-key
- * blocks: ceil(kv_len_max/64) / num_splits <= 1024); page_size a power of two >= 8.
+ * blocks: ceil(kv_len_max/64) / num_splits <= 1024); page_size a power of two >= 8;
+ * token strides of the pools at least head_dim (K's only with pages of 16 tokens or more).
  * Other arguments as in tasft_bsfa_decode_fwd (same workspace size).
  */
 int tasft_bsfa_decode_paged_fwd(const void* q, const void* k_pages, const void* v_pages,

@@ -594,6 +594,11 @@ class BlockSparseFlashAttention:
         q = q.contiguous()
         k_pages = _kernel_ready(k_pages)
         v_pages = _kernel_ready(v_pages)
+        sk, sv = k_pages.stride(), v_pages.stride()
+        if sk[1] < D or sv[1] < D:  # tokens that overlap (an expanded pool) are copied
+            k_pages, v_pages = (t if t.stride(1) >= D else t.clone(memory_format=torch.contiguous_format)
+                                for t in (k_pages, v_pages))
+            sk, sv = k_pages.stride(), v_pages.stride()
         mask = _mask_bytes(block_mask if block_mask.device == q.device else block_mask.to(q.device))
         # The kernel reads the table with a unit column stride.
         table = _int32_on(block_table, q.device)
@@ -605,7 +610,7 @@ class BlockSparseFlashAttention:
             q.data_ptr(), k_pages.data_ptr(), v_pages.data_ptr(), out.data_ptr(), mask.data_ptr(),
             table.data_ptr(), lens.data_ptr(), workspace.data_ptr(), ws_bytes, B, H, Hkv, S_kv, D,
             self.block_size, page_size, k_pages.shape[0], num_splits,
-            _native.strides(q), _native.strides(k_pages), _native.strides(v_pages),
+            _native.strides(q), _native.strides_array(sk), _native.strides_array(sv),
             _native.strides(out), _native.strides(mask), table.stride(0), 1.0 / math.sqrt(D), dtype,
             _native.stream_handle(q.device),
         )

@@ -217,6 +217,21 @@ def test_prefill_refuses_overlapping_rows_at_head_dim_128(which, block):
         assert rc == -1 and b"at least head_dim" in lib.tasft_last_error()
 
 
+def test_paged_decode_refuses_overlapping_tokens():
+    """A tile's buffer would cut such rows off; pages below 16 tokens read K without one."""
+    lib = _native.load_library()
+    ok, low, mask = _i64([2048, 128, 128, 1]), _i64([2048, 120, 128, 1]), _i64([0, 0, 0, 1])
+    fake = ctypes.c_void_p(16)
+
+    def call(page, k, v):
+        return lib.tasft_bsfa_decode_paged_fwd(
+            fake, fake, fake, fake, fake, fake, fake, fake, 1 << 24, 1, 32, 8, 1024, 128, 64, page, 100, 4,
+            ok, k, v, ok, mask, 64, 1.0, 0, None)
+
+    for page, k, v in ((16, low, ok), (16, ok, low), (64, low, low), (8, ok, low)):
+        assert call(page, k, v) == -1 and b"at least head_dim" in lib.tasft_last_error()
+
+
 def test_prefill_copies_overlapping_rows_at_head_dim_128():
     from tasft_amd.kernels.block_sparse_fa import _prefill_ready
     rows = torch.randn(2, 70, 3, 128).bfloat16().transpose(1, 2)
