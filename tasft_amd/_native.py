@@ -176,20 +176,21 @@ def is_available() -> bool:
 
 
 @functools.lru_cache(maxsize=4096)
-def _kept_array(values: tuple[int, ...]) -> ctypes.Array:
+def kept_strides(values: tuple[int, ...]) -> ctypes.Array:
+    """A tuple of element strides as a C int64 array. Arrays are kept by their values (not to be
+    written to; the library only reads them): building the five of a call took as long as the
+    call."""
     return (ctypes.c_int64 * len(values))(*values)
 
 
 def strides_array(values: Sequence[int]) -> ctypes.Array:
-    """A sequence of element strides as a C int64 array. Arrays are kept by their values (not to
-    be written to; the library only reads them): building the five of a call took as long as
-    the call."""
-    return _kept_array(tuple(values))
+    """Any sequence of element strides as a C int64 array (``kept_strides``)."""
+    return kept_strides(tuple(values))
 
 
 def strides(t: torch.Tensor) -> ctypes.Array:
-    """Element strides of a tensor as a C int64 array (``strides_array``)."""
-    return _kept_array(t.stride())
+    """Element strides of a tensor as a C int64 array (``kept_strides``)."""
+    return kept_strides(t.stride())
 
 
 # Element types of the 16-bit tensors (TASFT_DTYPE_BF16 / TASFT_DTYPE_F16).
@@ -244,5 +245,5 @@ def check(status: int, what: str, context: dict[str, object] | None = None) -> N
 
 
 __all__ = ["DTYPE_BF16", "DTYPE_F16", "EXPORTED_SYMBOLS", "KERNEL_DTYPES", "LIB_PATH", "check",
-           "dtype_code", "is_available", "kernel_layout", "load_library", "ptr", "stream_handle", "strides",
-           "strides_array"]
+           "dtype_code", "is_available", "kept_strides", "kernel_layout", "load_library", "ptr",
+           "stream_handle", "strides", "strides_array"]

@@ -135,8 +135,8 @@ class SparseAttentionDecoder:
             # One launch per (b, KV head): block sums, both projections, the kept key unit of
             # block i and the rows (tasft_gate_decode_rows_fwd).
             status = lib.tasft_gate_decode_rows_fwd(
-                q_new.data_ptr(), k.data_ptr() + 2 * at * k_st[2], _native.strides_array(q_st),
-                _native.strides_array(k_st), self._qsum.data_ptr(), self._ksum.data_ptr(),
+                q_new.data_ptr(), k.data_ptr() + 2 * at * k_st[2], _native.kept_strides(q_st),
+                _native.kept_strides(k_st), self._qsum.data_ptr(), self._ksum.data_ptr(),
                 self._vk.data_ptr(), self._vk.shape[2] * hid, self._wq_t.data_ptr(),
                 self._wk_t.data_ptr(), self._b_in.data_ptr(), self._w_out.data_ptr(),
                 self._taus.data_ptr(),

@@ -266,7 +266,7 @@ class BlockSparseFlashAttention:
         status = lib.tasft_bsfa_prefill_fwd(
             q.data_ptr(), k.data_ptr(), v.data_ptr(), out.data_ptr(), mask.data_ptr(),
             None, 0, B, H, k.shape[1], S, D, self.block_size,
-            _native.strides_array(sq), _native.strides_array(sk), _native.strides_array(sv), _native.strides(out),
+            _native.kept_strides(sq), _native.kept_strides(sk), _native.kept_strides(sv), _native.strides(out),
             _native.strides(mask), scale, 1 if causal else 0, dtype, _native.stream_handle(q.device),
         )
         _native.check(status, "tasft_bsfa_prefill_fwd", {"shape": [B, H, S, D]})
@@ -383,7 +383,7 @@ class BlockSparseFlashAttention:
         status = lib.tasft_bsfa_prefill_varlen_fwd(
             q.data_ptr(), k.data_ptr(), v.data_ptr(), out.data_ptr(), mask.data_ptr(),
             cu_dev.data_ptr(), n_seq, H, k.shape[1], max_seqlen, D, self.block_size,
-            _native.strides_array(sq), _native.strides_array(sk), _native.strides_array(sv), _native.strides(out),
+            _native.kept_strides(sq), _native.kept_strides(sk), _native.kept_strides(sv), _native.strides(out),
             _native.strides(mask), 1.0 / math.sqrt(D), 1 if causal else 0, dtype,
             _native.stream_handle(q.device),
         )
@@ -610,7 +610,7 @@ class BlockSparseFlashAttention:
             q.data_ptr(), k_pages.data_ptr(), v_pages.data_ptr(), out.data_ptr(), mask.data_ptr(),
             table.data_ptr(), lens.data_ptr(), workspace.data_ptr(), ws_bytes, B, H, Hkv, S_kv, D,
             self.block_size, page_size, k_pages.shape[0], num_splits,
-            _native.strides(q), _native.strides_array(sk), _native.strides_array(sv),
+            _native.strides(q), _native.kept_strides(sk), _native.kept_strides(sv),
             _native.strides(out), _native.strides(mask), table.stride(0), 1.0 / math.sqrt(D), dtype,
             _native.stream_handle(q.device),
         )
@@ -700,7 +700,7 @@ def default_decode_splits(batch: int, num_kv_heads: int, num_blocks: int,
                           q_per_kv: int = 1) -> int:
     """Split-K factor giving about one decode workgroup per CU (256 on MI355X), for every
     head count up to 16 query heads per KV head. Two workgroups fit per CU, but one per CU
-    is the fastest count or within 7% of it, merge included, over 1 to 32 splits: at B=8,
+    is the fastest count or within 8% of it, merge included, over 1 to 32 splits: at B=8,
     S=8192 with 28/4 heads 8 splits take 23.2 us (4: 27.6, 16: 23.5), with 32/8 heads 4 take
     27.1 us (2: 32.7, 8: 25.3); at B=16, S=4096, 32/8 heads 2 take 28.6 us (1: 29.2, 4: 26.7,
     8: 29.3); at B=2, S=2048 16 take 11.2 us (8: 12.4, 32: 12.1); at B=64 with 28/4 heads one

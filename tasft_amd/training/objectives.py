@@ -223,7 +223,7 @@ def _padded_attention_mask(mask: torch.Tensor, B: int, H: int, S: int, padded: i
     _native.check(code, "tasft_gate_mask_pad", {"attention_mask": list(mask.shape)})
     st = buf.stride()
     strides = (st[0] if mb > 1 else 0, st[1] if mh > 1 else 0, st[2] if rows > 1 else 0)
-    return buf, _native.strides_array(strides)
+    return buf, _native.kept_strides(strides)
 
 
 class _GateKL(torch.autograd.Function):
