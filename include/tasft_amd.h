@@ -236,7 +236,8 @@ size_t tasft_gate_workspace_bytes(int64_t batch, int64_t num_q_heads, int64_t nu
  * TASFT_GATE_FORCE_DIAGONAL (set the diagonal blocks in hard_mask regardless of tau).
  * head_dim a multiple of 8, at most 256; any block_size >= 1.
  * Block size 64 with head_dim 64 or 128 and hidden a multiple of 32 up to 128 runs, unless
- * small (at most 256 chunks of 16 blocks over all heads), as one kernel (after a one-workgroup reset of its counters in the workspace): workgroups that
+ * small (at most 256 chunks of 16 blocks over all heads) or with a token stride below head_dim,
+ * as one kernel (after a one-workgroup reset of its counters in the workspace): workgroups that
  * pool the query blocks wait, bounded by 1 ms of wall clock, for the workgroups that pool
  * the key blocks. Should that wait ever give up, bit 63 of active_count is set and the
  * affected rows hold NaN scores and no mask bit; callers that read active_count check it.

@@ -929,8 +929,13 @@ extern "C" int tasft_gate_target_fwd(const void* q, const void* k, const float* 
   p.pool = pool;
   p.NBO = (int)nb;
   p.fine = fine;
-  // One-wave kernel. Groups in turn when an XCD's share of K fits half its 4 MB L2 (B=4,
-  // 32/8 heads, S=1500, key-padding row: 73 us against 89 group by group).
+  // One-wave kernel. Groups in turn when an XCD's share of K fits half its 4 MB L2: every CU
+  // then starts on long rows, and K stays in L2 all the same. 32/8 heads at B=4, in turn against
+  // group by group: S=1500 (1.5 MB) 51 us against 58, with a key-padding row 59 against 67;
+  // S=2000 (2 MB) 70 against 87; 12/4 heads, B=8, S=1000, D=64 (0.5 MB) 24 against 32 with the
+  // row; one group per XCD the same (B=1, S=4096 69 us). Larger shares gain as well when taken in
+  // turn, less with their size (2.9 MB 126 against 172 us, 4 MB 217 against 229, 8 MB 836 against
+  // 847); they keep the group order.
   const int64_t group_rows = (num_q_heads / num_kv_heads * nb_run + kW1Waves - 1) / kW1Waves;
   p.interleave = (batch * num_kv_heads + 7) / 8 * seq_len * head_dim * 2 <= (2 << 20) ? 1 : 0;
   // Rows are cut into runs when there are too few of them to even out over the 512 workgroups

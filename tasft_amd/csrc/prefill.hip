@@ -172,7 +172,8 @@ __device__ __forceinline__ void dma16_lds(__amdgpu_buffer_rsrc_t r, uint8_t* dst
 // Head dim 64 takes 16 KB of LDS and three waves per SIMD (129 registers; four, with 122,
 // measured 4% faster at B=4, S=8192 and 4% slower on dense masks). Against four waves per query
 // block with two LDS stages and a merge of key halves, 32/8 heads, a fifth of the blocks: B=2,
-// S=4096 53 us (66.5); B=4, S=8192 310 us (332); S=1000 14.5 us (17); blocks of 128 58 us (69).
+// S=4096 55.7 us (68.6), with blocks of 128 55.3 us (68.4), nine tenths of the blocks 160 us
+// (167); B=4, S=8192 298 us (330).
 // ---------------------------------------------------------------------------------------
 // Workgroup barrier without a memory fence. The caller waits (s_waitcnt) for what the
 // barrier publishes; the memory clobber keeps the compiler from moving memory accesses
